@@ -16,6 +16,7 @@
 namespace kmst {
 
 using u8 = std::uint8_t;
+using u16 = std::uint16_t;
 using u32 = std::uint32_t;
 using u64 = std::uint64_t;
 using i64 = std::int64_t;
@@ -127,6 +128,23 @@ __device__ __forceinline__ int wave_id() { return threadIdx.x / WAVE; }
 __device__ __forceinline__ u32 mbcnt(u64 mask) {
   return __builtin_amdgcn_mbcnt_hi(static_cast<u32>(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo(static_cast<u32>(mask), 0u));
+}
+
+// popcount(mask & lanes-below-me) + acc
+__device__ __forceinline__ u32 mbcnt_acc(u64 mask, u32 acc) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<u32>(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<u32>(mask), acc));
+}
+
+// Hash of an undirected edge for the symmetry sums.  It costs two 32 x 32 -> 64 multiply-adds (the passes that take it
+// are bound by instruction issue): the first mixes the pair non-linearly, its
+// addend (b, a) keeping distinct pairs apart where a factor is zero; the
+// second folds the weight in, so that for a fixed pair the hash is injective
+// in w (a reverse record of another weight always changes the sums).
+__device__ __forceinline__ u64 sym_hash(u32 a, u32 b, u32 w) {
+  const u64 p = u64(a ^ 0x9E3779B9u) * u64(b ^ 0x85EBCA77u) + ((u64(b) << 32) | a);
+  const u32 c = static_cast<u32>(p) ^ static_cast<u32>(p >> 32) ^ w;
+  return u64(c) * 0xC2B2AE3Du + p;
 }
 
 template <typename T>

@@ -196,17 +196,6 @@ void scan_exclusive_u64(hipStream_t st, const u64* in, u64* out, u64 n, u64* scr
 // and hash sums of (min, max, w) over min<max and over max<min records:
 // the input is symmetric as a multiset iff both counts agree and the hash
 // sums agree, up to a collision of the sums.
-// The hash costs two 32 x 32 -> 64 multiply-adds (the passes that take it
-// are bound by instruction issue): the first mixes the pair non-linearly, its
-// addend (b, a) keeping distinct pairs apart where a factor is zero; the
-// second folds the weight in, so that for a fixed pair the hash is injective
-// in w (a reverse record of another weight always changes the sums).
-__device__ __forceinline__ u64 sym_hash(u32 a, u32 b, u32 w) {
-  const u64 p = u64(a ^ 0x9E3779B9u) * u64(b ^ 0x85EBCA77u) + ((u64(b) << 32) | a);
-  const u32 c = static_cast<u32>(p) ^ static_cast<u32>(p >> 32) ^ w;
-  return u64(c) * 0xC2B2AE3Du + p;
-}
-
 __global__ __launch_bounds__(BLOCK) void fingerprint_kernel(const u32* __restrict__ s,
                                                           const u32* __restrict__ d,
                                                           const u32* __restrict__ w, u64 count,
@@ -3051,12 +3040,6 @@ struct ScatterChunk {
   static constexpr int UNITS = WAVES * WAVE_UNITS;
   static constexpr int RECORDS = UNITS * int(UNIT_RECORDS);
 };
-
-// popcount(mask & lanes-below-me) + acc
-__device__ __forceinline__ u32 mbcnt_acc(u64 mask, u32 acc) {
-  return __builtin_amdgcn_mbcnt_hi(static_cast<u32>(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo(static_cast<u32>(mask), acc));
-}
 
 template <bool VEC, bool CHECK, bool LAZY>
 __global__ __launch_bounds__(BLOCK) void class_scatter_kernel(

@@ -387,6 +387,71 @@ struct PersistArgs {
 // cooperative launches are not supported.
 u32 persistent_blocks_max(int device);
 u32 persistent_threads();
+u32 compute_units(int device);
 void persistent_rounds(hipStream_t st, const PersistArgs& a, u32 blocks);
+
+// The direct solve (kmst_union.hip): a whole solve in one launch of resident
+// workgroups, on undirected edge lists over a union-find parent array.
+constexpr int UNION_THREADS = 1024;
+constexpr u32 UNION_BLOCKS_MAX = 256;  // one per CU
+constexpr u64 UNION_UNIT = 256;        // records a wave takes per step
+constexpr u64 UNION_VERTICES_MAX = u64{1} << 20;
+constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
+constexpr u32 UNION_ROUNDS_MAX = 200;
+constexpr u32 UNION_LOG = 61;          // u64 words: list lengths of the rounds, ...
+constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 3 phases
+constexpr u32 UNION_BAR_WORDS = 12 * 16;  // u64 words of the grid barrier
+enum : u32 {     // words of UnionArgs::ctl
+  UC_PIVOT = 0,  // two pivots: weights up to them are in the light pass's lists
+  UC_DONE = 2,   // the output is written
+  UC_GIANT = 3,  // 1 + a root that lived on after the last hook (0: none noted)
+  UC_WORDS = 4
+};
+struct UnionArgs {
+  const u32 *src = nullptr, *dst = nullptr, *wt = nullptr;  // the input: m records, ids < n
+  u64 m = 0;
+  u32 n = 0;
+  u32 chunk = 1;            // union_chunk(m, blocks)
+  u32 samples = 0;          // union_samples(m)
+  u32 rank[2] = {0, 0};     // the pivots' ranks among the samples
+  bool has_mid = false;     // the second class is not empty (rank[0] < rank[1])
+  bool has_heavy = false;   // nor is what lies above it
+  // list buffers of m edges, rounded up to whole chunks
+  u32* s[2] = {nullptr, nullptr};
+  u32* d[2] = {nullptr, nullptr};
+  u64* v[2] = {nullptr, nullptr};
+  u64* best[2] = {nullptr, nullptr};  // n + 1 words each
+  u32* parent = nullptr;
+  u64* bits = nullptr;   // one bit per vertex: the giant component
+  u32* marks = nullptr;  // one bit per input position: MST edges
+  u64* found = nullptr;  // 4 words per workgroup
+  u64* bar = nullptr;    // UNION_BAR_WORDS, zero
+  u32* joined = nullptr; // zero
+  u32* ctl = nullptr;    // UC_WORDS, zero
+  u32* ctr = nullptr;    // the 64 counter words that hold ctl and the like
+  u32* fwd_count = nullptr;
+  u64* hsum = nullptr;
+  u64* log = nullptr;    // UNION_LOG_TOTAL, zero
+  u32* err = nullptr;
+  u32* count = nullptr;  // MST edges
+  u32 *out_s = nullptr, *out_d = nullptr, *out_w = nullptr;
+  u64 out_cap = 0;
+};
+u64 union_mark_words(u64 m);
+u32 union_samples(u64 m);
+u32 union_blocks(u64 m, u32 cus);
+u32 union_chunk(u64 m, u32 blocks);
+// The solve, then the total weight into *total (written when the output is)
+// and the number of smaller endpoints with more than MST_GROUP_SMALL edges
+// into *groups (zero before).  Where the workgroups were not all resident
+// (*joined keeps another value than `blocks`), nothing is done: the caller
+// solves another way.
+// With p.host the 64 counter words at a.ctr and the log are published.
+struct Publication {
+  u32* host = nullptr;
+  u32 extra_at = 0, seq_at = 0, seq = 0;
+};
+void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
+                 u32* ended, const Publication& p);
 
 }  // namespace kmst

@@ -404,6 +404,12 @@ u32 persistent_blocks_max(int device) {
   return cached;
 }
 
+u32 compute_units(int device) {
+  int cus = 0;
+  KMST_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  return static_cast<u32>(cus);
+}
+
 u32 persistent_threads() { return PB; }
 
 double persistent_ticks_per_us(int device) {

@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -59,6 +60,8 @@ void KernelTimer::end(hipStream_t st) noexcept {
   ++used;
 }
 void KernelTimer::collect() {
+  // published counters arrive before the end of the kernel that wrote them
+  if (used) KMST_HIP(hipEventSynchronize(pool[used - 1].second));
   for (size_t i = 0; i < used; ++i) {
     float ms = 0.f;
     KMST_HIP(hipEventElapsedTime(&ms, pool[i].first, pool[i].second));
@@ -167,7 +170,7 @@ std::vector<DevBuf*> kmst_context::all_bufs() {
           &scan_scratch, &hist,  &counters,  &lookback, &in_s, &in_d,
           &in_w,     &out_s,      &out_d,   &out_w,     &samples, &gen_a, &gen_b,
           &gen_c,    &gen_d,      &tune,    &codec_bytes, &codec_off, &codec_first,
-          &persist_log, &part_giant};
+          &persist_log, &part_giant, &marks};
 }
 
 namespace kmst {
@@ -180,6 +183,11 @@ enum Ctr : int {
   C_ROOTS = 11,                   // parent-array roots with records (after a flatten)
   C_TOTAL64 = 16, C_HSUM64 = 18, C_ROUND64 = 22,
   C_CLASS64 = 24,   // MAX_CLASSES u64 class counts (words 24..41)
+  C_UNION = 42,     // UC_WORDS control words of the direct solve
+  C_UJOINED = 46,   // its workgroups that were resident together
+  C_UENDED = 47,    // workgroups of its last launch that have ended
+  C_UCOUNT = 48,    // its MST edges
+  C_UGROUPS = 49,   // smaller endpoints with more than MST_GROUP_SMALL of them
   C_OUTSIDE = 60    // outside_list: count (60), u64 total range length (62..63)
 };
 
@@ -193,6 +201,10 @@ struct RecView {
   const u32* w = nullptr;
   RecView at(u64 off, u64 cnt) const { return RecView{s + off, d + off, v + off, cnt, nullptr}; }
 };
+
+// inputs of at least this many records may cut the direct solve's lists in
+// chunks of more than one unit
+constexpr u64 DIRECT_CHUNK_MIN = u64{1} << 22;
 
 class Solver {
  public:
@@ -239,6 +251,11 @@ class Solver {
   u32* scan_scratch = nullptr;
   ArgPiece* pieces = nullptr;
   u32* samples = nullptr;
+  u32* marks = nullptr;  // direct solve: one bit per input record
+
+  // the whole solve on undirected edge lists (kmst_union.hip)
+  bool use_direct() const;
+  bool direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n, u64* total);
 
   WeightPivots pivots{};  // weight classes of the input (filter-Boruvka)
 
@@ -248,7 +265,9 @@ class Solver {
   void setup(bool filter, bool plan_classes);
   // packed keys when bits(max weight) + 2 bits(n) <= 64 (from the counters)
   void set_key_format();
-  // errors and the symmetry test of a finished input check
+  // errors and the symmetry test of a finished input check (from the counters,
+  // or reading them back first)
+  void check_input_words();
   void check_input();
   // set by setup when the class scatter validates the input
   bool check_in_scatter = false;
@@ -258,8 +277,11 @@ class Solver {
   void plan_pivots();
   void filter_classes();
   void check_errors(const char* where);
+  void check_error_word(const char* where);
   void read_counters();
   void fetch(const u32* extra, u32 words);
+  // waits until the device has published `seq`
+  void await_published(u32 seq);
   u64 counter64(int word) const {
     u64 x;
     std::memcpy(&x, C.host_counters + word, 8);
@@ -323,7 +345,8 @@ class Solver {
 };
 
 void Solver::allocate() {
-  const u64 m = m0 ? m0 : 1;
+  // the direct solve's lists are cut in whole chunks, long ones on large inputs
+  const u64 m = m0 + (m0 >= DIRECT_CHUNK_MIN ? UNION_CHUNK_MAX : 1) * UNION_UNIT;
   const u64 n = u64(n0) + 1;
   X = RecView{static_cast<u32*>(C.xs.get(m * 4)), static_cast<u32*>(C.xd.get(m * 4)),
               static_cast<u64*>(C.xv.get(m * 8)), m};
@@ -352,10 +375,12 @@ void Solver::allocate() {
   const u64 scan_max = std::max<u64>({n, (m + CMP_TILE - 1) / CMP_TILE + 1, record_units(m)});
   // u64 scans reuse the same scratch, so size it in u64 units
   scan_scratch = static_cast<u32*>(C.scan_scratch.get(scan_scratch_elems(scan_max) * 8 + 64));
-  ctr = static_cast<u32*>(C.counters.get(256));
+  ctr = static_cast<u32*>(
+      C.counters.get(256 + (UNION_LOG_TOTAL + UNION_BAR_WORDS + 4 * UNION_BLOCKS_MAX) * 8));
   samples = static_cast<u32*>(C.samples.get(4096 * 4));
   persist_log = static_cast<u64*>(
       C.persist_log.get(PERSIST_CTL_WORDS * 4 + PERSIST_LOG_TOTAL * 8 + PERSIST_GROUP_WORDS * 4));
+  marks = static_cast<u32*>(C.marks.get(union_mark_words(m) * 4));
   part_giant = part_count ? static_cast<u32*>(C.part_giant.get(u64(part_count) * 4 + 4)) : nullptr;
 }
 
@@ -384,6 +409,10 @@ void Solver::fetch(const u32* extra, u32 words) {
   }
   const u32 seq = ++C.publish_seq;
   publish_words(st, ctr, 64, extra, words, C.host_counters, HOST_SAMPLE_WORD, HOST_SEQ_WORD, seq);
+  await_published(seq);
+}
+
+void Solver::await_published(u32 seq) {
   u32* flag = C.host_counters + HOST_SEQ_WORD;
   for (u32 spins = 1;; ++spins) {
     if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) return;
@@ -404,6 +433,10 @@ void Solver::fetch(const u32* extra, u32 words) {
 
 void Solver::check_errors(const char* where) {
   read_counters();
+  check_error_word(where);
+}
+
+void Solver::check_error_word(const char* where) {
   const u32 e = C.host_counters[C_ERR];
   if (e & ERR_SPIN) throw Error(KMST_EDEVICE, std::string(where) + ": bounded wait expired");
   if (e & ERR_BOUNDS) throw Error(KMST_EDEVICE, std::string(where) + ": output position out of range");
@@ -468,7 +501,12 @@ void Solver::set_key_format() {
 }
 
 void Solver::check_input() {
-  check_errors("input");
+  read_counters();
+  check_input_words();
+}
+
+void Solver::check_input_words() {
+  check_error_word("input");
   if (u64(C.host_counters[C_FWD]) * 2 != m0 || counter64(C_HSUM64) != counter64(C_HSUM64 + 2))
     throw Error(KMST_EASYMMETRIC, "input: records are not symmetric (src,dst,w) <-> (dst,src,w)");
 }
@@ -946,6 +984,116 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
   filter_heavy(Q.at(L, H), P.at(L, H), Q.at(L, H), depth);
 }
 
+// The direct solve takes every size from the device, so its cost on a small
+// graph is one launch and one read-back, where the round loop needs 60 to 190
+// launches and 7 to 27 read-backs.  Its random accesses are atomic minima and
+// root walks over 12 bytes per vertex: up to UNION_VERTICES_MAX the parent
+// array (4 bytes) fits an XCD's L2 and the bitmap of the giant component
+// (n / 8 bytes) the LDS.  Measured, direct / round loop: 110 / 179 us at 256
+// vertices, 235 / 528 at 2^14, 338 / 1400 at 2^17, 627 / 1746 and 843 / 2673 at
+// 10^6 (16 and 32 records per vertex).  Sparse inputs (fewer than two records per
+// vertex: forests) stay with the round loop, and so does a context whose
+// persistent-round limit was set by hand.
+constexpr double DIRECT_FIRST_DEGREE = 2.2;
+constexpr u64 DIRECT_MID_VERTICES = u64{1} << 16;
+bool Solver::use_direct() const {
+  return n0 <= UNION_VERTICES_MAX && m0 >= 2 * u64(n0) &&
+         C.tuning.persistent_max == PERSIST_MAX_DEFAULT;
+}
+
+// False when the workgroups were not resident together (the GPU was shared
+// with other work): nothing was done, the round loop solves.
+bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n, u64* total) {
+  const double degree = double(m0) / double(n0);
+  // light records per vertex: the filter threshold, or more on dense inputs,
+  // whose crossing heavy edges fall off exponentially with it
+  const double target = std::max(double(std::max<u64>(filter_threshold, 2)), 2.0 + std::log(degree));
+  const bool heavy = target < 0.85 * degree;
+  const double light = heavy ? target / degree : 1.0;
+  // of those, first the DIRECT_FIRST_DEGREE lightest, where the rounds' work
+  // outweighs the barriers of another phase
+  const bool mid = n0 >= DIRECT_MID_VERTICES && DIRECT_FIRST_DEGREE < 0.7 * std::min(target, degree);
+  const double first = mid ? DIRECT_FIRST_DEGREE / degree : light;
+  UnionArgs a;
+  a.src = in_s;
+  a.dst = in_d;
+  a.wt = in_w;
+  a.m = m0;
+  a.n = n0;
+  const u32 blocks = union_blocks(m0, compute_units(C.device));
+  a.chunk = m0 >= DIRECT_CHUNK_MIN ? union_chunk(m0, blocks) : 1;
+  a.samples = union_samples(m0);
+  auto rank = [&](double share) {
+    return share >= 1.0 ? a.samples : static_cast<u32>(share * a.samples);
+  };
+  a.rank[0] = rank(first);
+  a.rank[1] = rank(light);
+  a.has_mid = a.rank[0] < a.rank[1];
+  a.has_heavy = a.rank[1] < a.samples;
+  a.s[0] = X.s;
+  a.d[0] = X.d;
+  a.v[0] = X.v;
+  a.s[1] = Y.s;
+  a.d[1] = Y.d;
+  a.v[1] = Y.v;
+  a.best[0] = best_val;
+  a.best[1] = state;
+  a.parent = parent;
+  a.bits = reinterpret_cast<u64*>(label);
+  a.marks = marks;
+  // log, barrier and the workgroups' words follow the counters
+  a.ctr = ctr;
+  a.log = reinterpret_cast<u64*>(ctr + 64);
+  a.bar = a.log + UNION_LOG_TOTAL;
+  a.found = a.bar + UNION_BAR_WORDS;
+  a.ctl = ctr + C_UNION;
+  a.joined = ctr + C_UJOINED;
+  a.count = ctr + C_UCOUNT;
+  a.fwd_count = ctr + C_FWD;
+  a.hsum = reinterpret_cast<u64*>(ctr + C_HSUM64);
+  a.err = ctr + C_ERR;
+  a.out_s = out_s;
+  a.out_d = out_d;
+  a.out_w = out_w;
+  a.out_cap = out_cap;
+  fill_u32(st, ctr, 64 + 2 * (UNION_LOG_TOTAL + UNION_BAR_WORDS), 0);
+  Publication p;
+  if (C.host_mapped) p = Publication{C.host_counters, HOST_SAMPLE_WORD, HOST_SEQ_WORD, ++C.publish_seq};
+  union_solve(st, a, blocks, reinterpret_cast<u64*>(ctr + C_TOTAL64), ctr + C_UGROUPS,
+              ctr + C_UENDED, p);
+  if (p.host) await_published(p.seq);
+  else fetch(reinterpret_cast<const u32*>(a.log), 2 * UNION_LOG_TOTAL);
+  if (blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
+  check_input_words();
+  if (!C.host_counters[C_UNION + UC_DONE]) throw Error(KMST_EDEVICE, "direct solve: not finished");
+  const u64 cnt = C.host_counters[C_UCOUNT];
+  if (cnt > out_cap) throw Error(KMST_EINVAL, "output capacity too small");
+  C.stats.packed_keys = false;
+  C.stats.mst_long_groups = C.host_counters[C_UGROUPS];
+  u64 lg[UNION_LOG_TOTAL];
+  std::memcpy(lg, C.host_counters + HOST_SAMPLE_WORD, sizeof(lg));
+  for (u32 i = 0; i < UNION_LOG && lg[i]; ++i) {
+    RoundStat rs;
+    rs.n = n0;
+    rs.m = lg[i];
+    rs.n_next = n0;
+    rs.m_next = i + 1 < UNION_LOG ? lg[i + 1] : 0;
+    rs.direct = true;
+    C.stats.rounds.push_back(rs);
+  }
+  for (u32 p = 0; p < 3; ++p) {
+    if ((p == 1 && !a.has_mid) || (p == 2 && !a.has_heavy)) continue;
+    FilterStat f{0, m0, 2 * lg[0], C.host_counters[C_UNION + UC_PIVOT + (p == 2)], p == 0, 0};
+    if (p > 0) f.heavy_kept = 2 * lg[std::min<u64>(lg[UNION_LOG + (p == 2 && a.has_mid)], UNION_LOG - 1)];
+    C.stats.filter.push_back(f);
+  }
+  *out_n = cnt;
+  *total = counter64(C_TOTAL64);
+  C.stats.mst_edges = cnt;
+  C.stats.total_weight = *total;
+  return true;
+}
+
 void Solver::run(const kmst_config& cfg, u32* out_s, u32* out_d, u32* out_w, u64 out_cap,
                  u64* out_n, u64* total) {
   C.stats = SolveStats{};
@@ -954,6 +1102,7 @@ void Solver::run(const kmst_config& cfg, u32* out_s, u32* out_d, u32* out_w, u64
   C.stats.algorithm = cfg.algorithm;
   filter_threshold = cfg.filter_threshold;
   allocate();
+  if (use_direct() && direct(out_s, out_d, out_w, out_cap, out_n, total)) return;
   const double avg_degree = double(m0) / double(std::max<u32>(n0, 1));
   const bool filter = cfg.algorithm == KMST_ALGO_FILTER_BORUVKA;
   const bool filter_base = avg_degree <= double(filter_threshold) || m0 <= 1000;
@@ -1480,7 +1629,8 @@ size_t kmst_context_stats_json(const kmst_context* ctx, char* buf, size_t cap) {
       << ",\"m_next\":" << r.m_next << ",\"run_starts\":" << r.run_starts
       << ",\"far_starts\":" << r.far_starts
       << ",\"persistent\":" << (r.persistent ? "true" : "false")
-      << ",\"twins\":" << (r.twins ? "true" : "false");
+      << ",\"twins\":" << (r.twins ? "true" : "false")
+      << ",\"direct\":" << (r.direct ? "true" : "false");
     if (r.persistent)
       o << ",\"phase_us\":[" << r.phase_us[0] << "," << r.phase_us[1] << "," << r.phase_us[2]
         << "," << r.phase_us[3] << "]";

@@ -37,6 +37,7 @@ struct RoundStat {
   u32 far_starts = 0;       // ... whose source is 16 or more ids from the record before
   bool persistent = false;  // ran inside the persistent launch
   bool twins = false;       // relabelled the src < dst half, both directions written
+  bool direct = false;      // a round of the direct solve: m counts undirected edges
   double phase_us[4] = {0, 0, 0, 0};  // persistent: bind, hook, jump, relabel
 };
 struct FilterStat {
@@ -133,7 +134,7 @@ struct kmst_context {
       mst;
   // kernel scratch
   kmst::DevBuf pieces, scan_scratch, hist, counters, samples, lookback, persist_log,
-      part_giant;
+      part_giant, marks;
   kmst::SortWork sort_work;  // radix sort state over `hist`
   kmst::LookbackWork lb_work;  // compaction look-back state over `lookback`
   kmst_tuning tuning{0, 1, kmst::SORT_WIDE_MIN, kmst::PERSIST_MAX_DEFAULT};  // launch shapes of later solves

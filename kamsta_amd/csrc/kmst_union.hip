@@ -1,0 +1,1148 @@
+// kmst_union.hip -- the direct solve: a whole minimum spanning forest in one
+// launch of resident workgroups, on undirected edge lists over a union-find
+// parent array.
+//
+// Phases (every size is read on the device; a grid barrier between phases):
+//
+//   init     parent[v] = v, minima and edge marks cleared, weight pivots from
+//            a sample of the weights;
+//   light    one pass over the input: validation, every vertex's lightest
+//            record, and the forward (src < dst) records of the two lightest
+//            weight classes, each wave listing its own;
+//   rounds   hook and relabel (below) on the listed edges until none is left;
+//   flatten  every vertex points at its root;
+//   cross    the second class, then the rest of the input: the edges that
+//            still join different components, followed by their rounds
+//            (boruvka_recursive, hybrid_boruvka_edgefilter.hpp:227-330, with
+//            the classes as its levels);
+//   output   the marked input positions in order: the input is sorted by
+//            (src, dst), so this is the MST sorted by (min, max).
+//
+// A list holds each undirected edge once as (a, b, key) with a and b roots of
+// the parent array; best[v] is the smallest key of the edges at root v.
+//   hook     an edge that is the minimum of one of its ends hooks that end
+//            onto the other; of a mutual pair the lower end stays root (the
+//            lower-endpoint rule of determine_mst_edges,
+//            include/algorithms/gbbs_reimplementation.hpp:100-130).  The
+//            edges that hook an end are MST edges.  Keys order edges
+//            strictly, so every component of the hooks holds exactly one
+//            mutual pair, whose lower end is the only root that lives on: it
+//            clears its minimum of the next round.
+//   relabel  both ends walk to their roots (shortening the walked paths, as
+//            update_parents, gbbs_reimplementation.hpp:162-169), self-loops
+//            drop (relabel_edges / filter_out_self_loops, :184-219), and the
+//            kept edges offer their keys to the minima of the next round.
+// Against the sort-based rounds this moves each undirected edge once instead
+// of both directed records, and needs no vertex renumbering, sort, pass over
+// the vertices or read-back.
+//
+// What bounds it: a small or medium solve is a chain of dependent memory
+// round trips (about 0.7 us each) and barriers.  A barrier costs 2.1 us at 16
+// workgroups and 2.6 us at 256, because what workgroups share between phases
+// (parent, minima, marks, counters) is accessed with agent-scope relaxed
+// atomics, which are coherent by themselves; with plain accesses each barrier
+// needs an agent-scope fence per workgroup, an L2 write-back, and costs 2.4 to
+// 11.4 us.  A launch per phase costs 4 us and more.  Agent-scope gathers run
+// at the rate of plain ones (250 10^9/s from a 4 MB table, 58 10^9/s from 64
+// MB); atomic minima run at 26 10^9/s spread out and 12 10^6/s on one address.
+// Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
+// records 110 / 179 us; 2^14, 4.9 10^5 235 / 528 us; 2^17, 2.1 10^6 338 / 1400
+// us; 10^6, 3.2 10^7 843 / 2673 us (a copy of its bytes: 81 us).
+// Lists are private to a wave, so they need no coherence, counters or
+// workgroup barriers, and their compaction is in place.
+#include "kmst_kernels.hpp"
+
+namespace kmst {
+
+namespace {
+
+constexpr int UT = UNION_THREADS;  // 1024: one workgroup per CU
+constexpr int UW = UT / WAVE;
+constexpr u64 WALL_TICKS_PER_MS = 100000;              // 100 MHz wall clock
+constexpr u64 BARRIER_TICKS = 10000 * WALL_TICKS_PER_MS;  // bound of a barrier's wait
+constexpr u64 JOIN_TICKS = 5 * WALL_TICKS_PER_MS;      // bound of the first one's
+constexpr u32 WALK_LIMIT = 1u << 26;                   // a longer walk is a corrupted forest
+
+// wave index, in a scalar register: what follows from it (a wave's units, list
+// and counts) is then wave-uniform to the compiler too
+__device__ __forceinline__ u32 wave_index() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+}
+
+// ------------------------------------------------------------ shared data
+template <typename T>
+__device__ __forceinline__ T get(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void put(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void lower(u64* best, u32 v, u64 k) {
+  (void)__hip_atomic_fetch_min(best + v, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void offer(u64* best, u32 v, u64 k) {
+  if (k < get(best + v)) lower(best, v, k);
+}
+
+// ------------------------------------------------------------ barrier
+// Workgroups arrive on one of eight group words (workgroup id mod 8, one XCD
+// each) and a group's last arrival adds the group to the root word, so that no
+// address takes more than 32 arrivals.  The words also sum a payload, returned
+// to every workgroup.  Group words are cleared by their last arrival; the root
+// words rotate, and workgroup 0 clears the one after next (nobody arrives on
+// it before workgroup 0 has arrived on the next).
+// Every wave waits for its own stores and atomics (vmcnt 0) before its
+// workgroup arrives.  The first barrier is the admission check: an ordinary
+// launch does not promise that all workgroups are resident together, so if
+// they are not within JOIN_TICKS the launch is called off, by one atomic
+// decision that later arrivals see, and every workgroup leaves with nothing
+// changed but scratch.  Once it has passed, all are resident, and the other
+// barriers complete (their wait is bounded all the same).
+constexpr u32 GROUPS = 8;
+constexpr u32 LINE = 16;  // u64 words per 128-byte line
+constexpr u64 PAYLOAD_SHIFT = 16;
+constexpr u32 CALLED_OFF = 0x80000000u;
+
+struct Barrier {
+  u64* words;  // root words at lines 0..3, group words at lines 4..11
+  u32 k = 0;
+  u32* err;
+};
+
+// (thread 0's payload counts)
+__device__ __forceinline__ bool sync_grid(Barrier& bar, u64 payload, u64& sum) {
+  __shared__ u64 s_sum;
+  __shared__ u32 s_ok;
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  if (gridDim.x == 1) {
+    if (threadIdx.x == 0) s_sum = payload;
+    __syncthreads();
+    sum = s_sum;
+    return true;
+  }
+  if (threadIdx.x == 0) {
+    const u32 g = blockIdx.x % GROUPS, groups = min(GROUPS, gridDim.x);
+    const u32 members = (gridDim.x - g + GROUPS - 1) / GROUPS;
+    u64* root = bar.words + (bar.k & 3) * LINE;
+    u64* grp = bar.words + (4 + g) * LINE;
+    const u64 mine = (payload << PAYLOAD_SHIFT) | 1;
+    const u64 now = __hip_atomic_fetch_add(grp, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
+    if ((now & 0xFFFF) == members) {
+      put(grp, u64{0});
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // cleared before the group's next arrivals
+      (void)__hip_atomic_fetch_add(root, (now & ~u64{0xFFFF}) | 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const u64 t0 = wall_clock64();
+    u32 ok = 1;
+    u64 r;
+    while (((r = get(root)) & 0xFFFF) != groups) {
+      if (wall_clock64() - t0 > BARRIER_TICKS || (get(bar.err) & ERR_SPIN)) {
+        atomicOr(bar.err, ERR_SPIN);
+        ok = 0;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    if (blockIdx.x == 0) put(bar.words + ((bar.k + 2) & 3) * LINE, u64{0});
+    s_sum = r >> PAYLOAD_SHIFT;
+    s_ok = ok;
+  }
+  ++bar.k;
+  __syncthreads();
+  sum = s_sum;
+  return s_ok != 0;
+}
+
+__device__ __forceinline__ bool join_grid(u32* joined) {
+  __shared__ u32 s_join;
+  if (threadIdx.x == 0) {
+    u32 ok = 1;
+    if (gridDim.x > 1) {
+      u32 seen = __hip_atomic_fetch_add(joined, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+      const u64 t0 = wall_clock64();
+      while (seen != gridDim.x && !(seen & CALLED_OFF)) {
+        if (wall_clock64() - t0 > JOIN_TICKS)
+          (void)atomicCAS(joined, seen, seen | CALLED_OFF);  // fails if someone joined: look again
+        else
+          __builtin_amdgcn_s_sleep(1);
+        seen = get(joined);
+      }
+      ok = seen & CALLED_OFF ? 0u : 1u;
+    }
+    s_join = ok;
+  }
+  __syncthreads();
+  return s_join != 0;
+}
+
+// ------------------------------------------------------------ loads
+// Four consecutive words, with the alignment of one: global_load_dwordx4
+// needs 4-byte alignment only, so arrays at any address take the wide loads.
+// The passes over the input read each word once: non-temporal loads leave
+// the parent array and the minima in the L2s.
+typedef u32 u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load4(const u32* p, u32 (&x)[4]) {
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = v[e];
+}
+
+// One wave's 256 consecutive records, lane l those at 4l .. 4l + 3, and the
+// record before them ((0, 0), which no valid record precedes, before the
+// first).  Past the end: copies of the last record, which change no minimum.
+struct Unit {
+  u32 s[4], d[4], w[4];
+  u32 ps, pd;
+};
+template <bool PREV>
+__device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit) {
+  const u64 r0 = unit * UNION_UNIT + 4 * lane_id();
+  if ((unit + 1) * UNION_UNIT <= a.m) {
+    load4(a.src + r0, x.s);
+    load4(a.dst + r0, x.d);
+    load4(a.wt + r0, x.w);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const u64 i = min(r0 + e, a.m - 1);
+      x.s[e] = a.src[i];
+      x.d[e] = a.dst[i];
+      x.w[e] = a.wt[i];
+    }
+  }
+  if (PREV) {
+    const u64 i = unit * UNION_UNIT;
+    x.ps = i ? a.src[i - 1] : 0u;
+    x.pd = i ? a.dst[i - 1] : 0u;
+  }
+}
+
+// ------------------------------------------------------------ union-find
+// Roots of N vertices, their walks in lockstep so that a step's dependent
+// loads are in flight together; a walk that has ended loads no more (the
+// longest of a wave's walks is several times the mean).  A walk stores nothing
+// but every eighth step (a load waits for the stores before it, a round trip to
+// memory per step; the stores that remain let walks over a long chain double),
+// and the root it found where (x's hash ^ salt) & thin is 0.
+template <int N>
+__device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u32 salt, u32* err) {
+  u32 p[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) p[j] = get(parent + x[j]);
+  u32 open = 0, moved = 0;  // bit j: walk j has not ended / has left its first parent
+#pragma unroll
+  for (int j = 0; j < N; ++j) open |= p[j] != x[j] ? 1u << j : 0u;
+  for (u32 step = 1; __any(open != 0); ++step) {
+    u32 y[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      y[j] = p[j];
+      if ((open >> j) & 1) y[j] = get(parent + p[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (y[j] == p[j]) {
+        open &= ~(1u << j);
+      } else {
+        moved |= 1u << j;
+        p[j] = y[j];
+        if ((step & 7) == 0) put(parent + x[j], y[j]);
+      }
+    }
+    if (step > WALK_LIMIT) {
+      atomicOr(err, ERR_SPIN);
+      break;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if (((moved >> j) & 1) && ((((x[j] * 0x9E3779B1u) >> 16) ^ salt) & thin) == 0)
+      put(parent + x[j], p[j]);
+    x[j] = p[j];
+  }
+}
+
+// ------------------------------------------------------------ minima in LDS
+// Minima of a workgroup's offers by vertex: few roots share many edges in
+// late rounds, and atomics on one address take about 80 ns each.  First come,
+// first served: an offer whose slot belongs to another vertex goes to the
+// shared minimum at once.
+constexpr int TABLE_BITS = 12;
+struct OfferTable {
+  static constexpr u32 SIZE = 1u << TABLE_BITS;
+  u32 id[SIZE];
+  u64 key[SIZE];
+};
+__device__ __forceinline__ void table_clear(OfferTable& t) {
+  for (u32 i = threadIdx.x; i < t.SIZE; i += UT) {
+    t.id[i] = NONE32;
+    t.key[i] = VAL_NONE;
+  }
+}
+__device__ __forceinline__ void table_offer(OfferTable& t, u64* best, u32 v, u64 k) {
+  const u32 slot = (v * 0x9E3779B1u) >> (32 - TABLE_BITS);
+  u32 owner = t.id[slot];
+  if (owner == NONE32) owner = atomicCAS(&t.id[slot], NONE32, v);
+  if (owner == NONE32 || owner == v) {
+    if (k < t.key[slot])
+      atomicMin(reinterpret_cast<unsigned long long*>(&t.key[slot]),
+                static_cast<unsigned long long>(k));
+    // keeps the two atomics apart: merged, they become one flat access
+    asm volatile("; lds offer");
+  } else {
+    offer(best, v, k);
+  }
+}
+__device__ __forceinline__ void table_flush(OfferTable& t, u64* best) {
+  for (u32 i = threadIdx.x; i < t.SIZE; i += UT)
+    if (t.id[i] != NONE32) offer(best, t.id[i], t.key[i]);
+}
+
+// ------------------------------------------------------------ pivots
+// The sampled weights at ranks rank0 <= rank1 (a rank at or past `samples`:
+// all ones, everything is below), by workgroup 0: a radix select over 8-bit
+// digits, histograms of the samples still in the running from the highest
+// digit that is not zero everywhere.
+constexpr u32 PIVOT_PER_THREAD = 1;
+constexpr u32 PIVOT_SAMPLES_MAX = UT * PIVOT_PER_THREAD;
+
+__device__ void pick_pivots(const UnionArgs& a) {
+  __shared__ u32 h[256];
+  __shared__ u32 s_scan[UW];
+  __shared__ u32 s_digit, s_below, s_max;
+  const u32 t = threadIdx.x, samples = a.samples;
+  if (t == 0) s_max = 0;
+  __syncthreads();
+  u32 x[PIVOT_PER_THREAD], mx = 0;
+  if (a.rank[0] < samples) {
+#pragma unroll
+    for (u32 j = 0; j < PIVOT_PER_THREAD; ++j) {
+      const u64 q = min(j * UT + t, samples - 1);
+      x[j] = a.wt[(q * a.m) / samples];  // < m
+      mx = max(mx, x[j]);
+    }
+  }
+  atomicMax(&s_max, mx);
+  __syncthreads();
+  const int top = s_max >> 24 ? 24 : s_max >> 16 ? 16 : s_max >> 8 ? 8 : 0;
+  for (int which = 0; which < 2; ++which) {
+    u32 want = a.rank[which], pivot = NONE32;
+    if (want < samples) {
+      u32 prefix = 0;
+      for (int shift = top; shift >= 0; shift -= 8) {
+        if (t < 256) h[t] = 0;
+        __syncthreads();
+#pragma unroll
+        for (u32 j = 0; j < PIVOT_PER_THREAD; ++j)
+          if (j * UT + t < samples && (shift == top || (x[j] >> (shift + 8)) == prefix))
+            atomicAdd(&h[(x[j] >> shift) & 255], 1u);
+        __syncthreads();
+        const u32 c = t < 256 ? h[t] : 0u;
+        const u32 incl = wave_inclusive_sum(c);
+        if (lane_id() == WAVE - 1) s_scan[wave_id()] = incl;
+        __syncthreads();
+        if (t < 256) {
+          u32 below = incl - c;
+          for (int w = 0; w < wave_id(); ++w) below += s_scan[w];
+          if (want >= below && want < below + c) {
+            s_digit = t;
+            s_below = below;
+          }
+        }
+        __syncthreads();
+        prefix = (prefix << 8) | s_digit;
+        want -= s_below;
+        __syncthreads();
+      }
+      pivot = prefix;
+    }
+    if (t == 0) put(a.ctl + UC_PIVOT + which, pivot);
+  }
+}
+
+// ------------------------------------------------------------ light pass
+// Bound: 12 bytes per record from HBM, then instruction issue.
+//
+// A list edge's key is (weight << 32) | the record's position.  Positions
+// follow (min, max), so keys order the edges by (weight, min, max), parallel
+// copies of one weight (the same triple) by position.
+// The first minima are (weight << 32) | dst over a vertex's records in both
+// directions: among the edges at one vertex v, dst < v sorts by min = dst
+// before dst > v by max = dst, so (weight, dst) orders them as (weight, min,
+// max) does, and no record needs its twin's position.  The input is sorted by
+// src, so the minima are a segmented minimum over runs: a run inside a chunk of
+// a.chunk consecutive units, which one wave takes, is stored; only the runs at
+// the chunk's ends take an atomic.  (Atomics at the ends of every unit took 95
+// of 230 us at 10^6 vertices, 3.2 10^7 records: neighbouring waves share lines.)
+__device__ __forceinline__ u64 dst_key(u32 w, u32 d) { return (u64(w) << 32) | d; }
+
+// The run a chunk's next unit may continue (wave-uniform).
+struct Carry {
+  u32 s;
+  u64 v;
+  u32 inside;  // it began in this chunk, after the chunk's first record or with it
+  bool any;    // false at the chunk's first unit
+};
+
+// Minima of a unit; sources at or past n share word n.
+__device__ __forceinline__ void run_minima(const Unit& x, bool first_unit, bool last_of_chunk,
+                                           u32 n, u64* best, Carry& c) {
+  const int lane = lane_id();
+  const u32 head_s = x.s[0];
+  u32 tail_s = head_s;
+  u64 tail_v = dst_key(x.w[0], x.d[0]);
+  u64 head_v = tail_v;
+  bool multi = false;  // the lane's records hold more than one run
+#pragma unroll
+  for (int e = 1; e < 4; ++e) {
+    const u64 k = dst_key(x.w[e], x.d[e]);
+    if (x.s[e] != tail_s) {
+      if (!multi) head_v = tail_v;
+      else put(best + min(tail_s, n), tail_v);  // a run inside the lane
+      multi = true;
+      tail_s = x.s[e];
+      tail_v = k;
+    } else {
+      tail_v = k < tail_v ? k : tail_v;
+    }
+  }
+  // the run before a lane's: the previous lane's last one, or the carry
+  u32 prev_s = __shfl_up(tail_s, 1, WAVE);
+  bool joins = prev_s == head_s;
+  u32 began = 1;  // the lane's head run began inside the chunk, if it joins none
+  if (lane == 0) {
+    joins = c.any && c.s == head_s;
+    began = c.any || first_unit || x.ps != head_s ? 1u : 0u;
+    if (c.any && !joins) {
+      if (c.inside) put(best + min(c.s, n), c.v);
+      else lower(best, min(c.s, n), c.v);
+    }
+    if (joins && !multi) tail_v = c.v < tail_v ? c.v : tail_v;
+  }
+  // whether the tail run began inside the chunk; lanes that continue a run
+  // learn it, with the run's minimum, from the lanes before
+  u32 inside = multi ? 1u : joins ? (lane == 0 ? c.inside : 0u) : began;
+  bool open = lane > 0 && joins && !multi;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    if (!__any(open)) break;
+    const u64 v = __shfl_up(static_cast<unsigned long long>(tail_v), o, WAVE);
+    const u32 in = __shfl_up(inside, o, WAVE);
+    const u32 still = __shfl_up(open ? 1u : 0u, o, WAVE);
+    if (open) {
+      tail_v = v < tail_v ? v : tail_v;
+      inside = in;
+      open = still != 0;
+    }
+  }
+  u64 prev_v = __shfl_up(static_cast<unsigned long long>(tail_v), 1, WAVE);
+  u32 prev_in = __shfl_up(inside, 1, WAVE);
+  const u32 next_s = __shfl_down(head_s, 1, WAVE);
+  if (lane == 0) {
+    prev_v = c.v;
+    prev_in = c.inside;
+  }
+  if (multi) {
+    if (joins && prev_v < head_v) head_v = prev_v;
+    if (joins ? prev_in : began) put(best + min(head_s, n), head_v);
+    else lower(best, min(head_s, n), head_v);
+  }
+  if (lane < WAVE - 1 && next_s != tail_s) {
+    if (inside) put(best + min(tail_s, n), tail_v);
+    else lower(best, min(tail_s, n), tail_v);
+  }
+  if (last_of_chunk && lane == WAVE - 1) lower(best, min(tail_s, n), tail_v);
+  c.s = __builtin_amdgcn_readlane(tail_s, WAVE - 1);
+  c.v = (u64(static_cast<u32>(__builtin_amdgcn_readlane(static_cast<u32>(tail_v >> 32), WAVE - 1))) << 32) |
+        static_cast<u32>(__builtin_amdgcn_readlane(static_cast<u32>(tail_v), WAVE - 1));
+  c.inside = __builtin_amdgcn_readlane(inside, WAVE - 1);
+  c.any = !last_of_chunk;
+}
+
+// What a workgroup found in the input.
+struct Found {
+  u64 hash_fwd, hash_rev;
+  u32 fwd, bad, dup;
+};
+
+// A wave's own lists: c edges from `base` on, and c_mid edges of the second
+// class from the end of the other buffer's same range of `cap` edges down.
+// Every edge comes from one of the wave's own records, so cap (their number)
+// is never exceeded, whatever the input.
+struct WaveLists {
+  u64 base, cap;
+  u32 c, c_mid;
+};
+
+// The units of a wave: chunks of `chunk` consecutive units, the chunks dealt
+// to the waves in turn.
+struct UnitWalk {
+  u64 unit, end, left_in_chunk, skip;
+  u32 chunk;
+  __device__ __forceinline__ UnitWalk(const UnionArgs& a, u64 wave, u64 waves, u64 units)
+      : unit(wave * a.chunk), end(units), left_in_chunk(a.chunk), skip((waves - 1) * a.chunk),
+        chunk(a.chunk) {}
+  __device__ __forceinline__ bool valid() const { return unit < end; }
+  __device__ __forceinline__ bool last_of_chunk() const {
+    return left_in_chunk == 1 || unit + 1 == end;
+  }
+  __device__ __forceinline__ void next() {
+    ++unit;
+    if (--left_in_chunk == 0) {
+      unit += skip;
+      left_in_chunk = chunk;
+    }
+  }
+};
+
+// A wave's taken edges wait in LDS and leave 64 at a time, in whole lines
+// (stored as they were taken, a few per unit, they cost 70 of 178 us at 10^6
+// vertices, 3.2 10^7 records).  Class c at [c * STAGE, (c + 1) * STAGE).
+constexpr u32 STAGE = 2 * WAVE;
+struct Stage {
+  u32 s[2 * STAGE], d[2 * STAGE];
+  u64 v[2 * STAGE];
+};
+
+// The first min(n, 64) staged edges of a class to its list, the rest (fewer
+// than 64) to the front.
+template <int CLASS>
+__device__ __forceinline__ void drain(const UnionArgs& a, WaveLists& l, Stage& st, u32& n) {
+  const u32 lane = lane_id(), at = CLASS * STAGE + lane, out = min<u32>(n, WAVE);
+  if (lane < out) {
+    const u64 q = CLASS ? l.base + l.cap - 1 - (l.c_mid + lane) : l.base + l.c + lane;
+    a.s[CLASS][q] = st.s[at];
+    a.d[CLASS][q] = st.d[at];
+    a.v[CLASS][q] = st.v[at];
+  }
+  if (CLASS) l.c_mid += out;
+  else l.c += out;
+  n -= out;
+  if (lane < n) {
+    st.s[at] = st.s[at + WAVE];
+    st.d[at] = st.d[at + WAVE];
+    st.v[at] = st.v[at + WAVE];
+  }
+}
+
+__device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, UnitWalk at, Stage& st,
+                                           Found& out) {
+  __shared__ Found s_found[UW];
+  const int lane = lane_id();
+  const u32 q0 = get(a.ctl + UC_PIVOT), q1 = get(a.ctl + UC_PIVOT + 1);
+  // wave-uniform: lanes that saw an error or a parallel record, forward count
+  u64 bad_id = 0, bad_order = 0, dup = 0;
+  u32 fwd = 0;
+  u64 hf = 0, hall = 0;  // hash sums of the forward and of all records
+  Carry carry{0, 0, 0, false};
+  u32 n0 = 0, n1 = 0;  // staged edges of the two classes
+  Unit next;
+  if (at.valid()) load_unit<true>(next, a, at.unit);
+  while (at.valid()) {
+    const Unit x = next;
+    const u64 unit = at.unit;
+    const bool last = at.last_of_chunk();
+    at.next();
+    if (at.valid()) load_unit<true>(next, a, at.unit);
+    const u64 r0 = unit * UNION_UNIT + 4 * lane;
+    const bool full = (unit + 1) * UNION_UNIT <= a.m;
+    u32 ps = __shfl_up(x.s[3], 1, WAVE), pd = __shfl_up(x.d[3], 1, WAVE);
+    if (lane == 0) {
+      ps = x.ps;
+      pd = x.pd;
+    }
+    u64 b0[4], b1[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const u32 s = x.s[e], d = x.d[e], w = x.w[e];
+      const u64 in = full ? ~0ull : __ballot(r0 + e < a.m);
+      const u32 lo = min(s, d), hi = max(s, d);
+      const u64 prev = (u64(ps) << 32) | pd, here = (u64(s) << 32) | d;
+      bad_id |= __ballot(hi >= a.n) | __ballot(lo == hi);
+      bad_order |= __ballot(prev > here);  // (copies past the end equal their predecessor)
+      dup |= __ballot(prev == here) & in;
+      ps = s;
+      pd = d;
+      const u64 f = __ballot(s < d) & in;
+      const u64 l0 = __ballot(w <= q0), l1 = __ballot(w <= q1);
+      u64 h = sym_hash(lo, hi, w);
+      if (!full && r0 + e >= a.m) h = 0;
+      fwd += static_cast<u32>(__popcll(f));
+      hf += s < d ? h : 0ull;
+      hall += h;
+      b0[e] = f & l0;
+      b1[e] = f & l1 & ~l0;
+    }
+    run_minima(x, unit == 0, last, a.n, a.best[0], carry);
+    // a lane's taken records leave one per step (a lane seldom takes more
+    // than two, so this needs fewer steps than one per record)
+    u32 take = 0, mids = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      take |= ((b0[e] | b1[e]) >> lane) & 1ull ? 1u << e : 0u;
+      mids |= (b1[e] >> lane) & 1ull ? 1u << e : 0u;
+    }
+    while (__any(take != 0)) {
+      const u32 e = static_cast<u32>(__ffs(take) - 1);
+      const bool any = take != 0, mid = any && ((mids >> e) & 1u);
+      const u64 t0 = __ballot(any && !mid), t1 = __ballot(mid);
+      if (any) {
+        const u32 s = e < 2 ? (e ? x.s[1] : x.s[0]) : (e == 2 ? x.s[2] : x.s[3]);
+        const u32 d = e < 2 ? (e ? x.d[1] : x.d[0]) : (e == 2 ? x.d[2] : x.d[3]);
+        const u32 w = e < 2 ? (e ? x.w[1] : x.w[0]) : (e == 2 ? x.w[2] : x.w[3]);
+        const u32 q = mid ? STAGE + n1 + mbcnt(t1) : n0 + mbcnt(t0);
+        st.s[q] = s;
+        st.d[q] = d;
+        st.v[q] = (u64(w) << 32) | (r0 + e);
+        take &= take - 1;
+      }
+      n0 += static_cast<u32>(__popcll(t0));
+      n1 += static_cast<u32>(__popcll(t1));
+      if (n0 >= WAVE) drain<0>(a, l, st, n0);
+      if (n1 >= WAVE) drain<1>(a, l, st, n1);
+    }
+  }
+  if (n0) drain<0>(a, l, st, n0);
+  if (n1) drain<1>(a, l, st, n1);
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    hf += __shfl_xor(hf, o, WAVE);
+    hall += __shfl_xor(hall, o, WAVE);
+  }
+  if (lane == 0)
+    s_found[wave_index()] = Found{hf, hall - hf, fwd,
+                               (bad_id ? u32(ERR_INVALID) : 0u) | (bad_order ? u32(ERR_UNSORTED) : 0u),
+                               dup ? 1u : 0u};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    Found f{0, 0, 0, 0, 0};
+    for (int w = 0; w < UW; ++w) {
+      f.hash_fwd += s_found[w].hash_fwd;
+      f.hash_rev += s_found[w].hash_rev;
+      f.fwd += s_found[w].fwd;
+      f.bad |= s_found[w].bad;
+      f.dup |= s_found[w].dup;
+    }
+    out = f;
+  }
+}
+
+// ------------------------------------------------------------ crossing edges
+// Nearly every crossing edge touches one giant component, whose minimum would
+// take one atomic per edge at one address.  It gets none: a root without a
+// minimum hooks nowhere, and the components that choose an edge to it hook
+// onto it, which is all a round needs to make progress.  Any root may be the
+// passive one; it is a root that lived on after the last hook of the phase
+// before (with few of them left each hook notes one).
+// The flatten marks its component in a bitmap (n / 8 bytes, at most 128 KB),
+// which the pass over the input keeps in LDS, and most records lie inside it.
+// Neither changes in these passes: after an acquire at agent scope plain loads
+// are current, and the gathers of a source's records hit the L1.
+__device__ __forceinline__ void offer_ends(u64* best, u32 s, u32 d, u64 k, u32 giant) {
+  if (s != giant) offer(best, s, k);
+  if (d != giant) offer(best, d, k);
+}
+
+// Appends to the wave's list the edges of four per lane whose ends (roots,
+// 0 / 0 where a lane has none) differ, with their offers.
+__device__ __forceinline__ void append_crossing(const UnionArgs& a, WaveLists& l, const u32 (&s)[4],
+                                                const u32 (&d)[4], const u64 (&k)[4], u64* best,
+                                                u32 giant) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const u64 b = __ballot(s[e] != d[e]);
+    if (!b) continue;
+    if (s[e] != d[e]) {
+      const u64 q = l.base + l.c + mbcnt(b);
+      a.s[0][q] = s[e];
+      a.d[0][q] = d[e];
+      a.v[0][q] = k[e];
+      offer_ends(best, s[e], d[e], k[e], giant);
+    }
+    l.c += static_cast<u32>(__popcll(b));
+  }
+}
+
+// Second class: the wave's own list, from its low end up (what is appended
+// never reaches what is still to be read: both fit the wave's range).
+__device__ __forceinline__ void cross_mid(const UnionArgs& a, WaveLists& l, u64* best, u32 giant) {
+  const u64 lo = l.base + l.cap - l.c_mid;
+  for (u32 j0 = 0; j0 < l.c_mid; j0 += 4 * WAVE) {
+    u32 x[8], s[4], d[4];
+    u64 k[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const u64 q = lo + min<u32>(j0 + e * WAVE + lane_id(), l.c_mid - 1);
+      x[e] = a.s[1][q];
+      x[4 + e] = a.d[1][q];
+      k[e] = a.v[1][q];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = a.parent[x[e]];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = j0 + e * WAVE + lane_id() < l.c_mid;
+      s[e] = in ? x[e] : 0u;
+      d[e] = in ? x[4 + e] : 0u;
+    }
+    append_crossing(a, l, s, d, k, best, giant);
+  }
+  l.c_mid = 0;
+}
+
+// The rest of the input: the wave's own forward records above the pivot, two
+// units per step, every load of a kind in flight before the next kind's.
+// `inside` is the giant's bitmap in LDS: gathered from the L2s, at 250 10^9/s,
+// its words alone took 80 of 150 us at 10^6 vertices, 1.6 10^7 edges.
+__device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, UnitWalk at,
+                                            u64* best, u32 giant, const u32* inside) {
+  constexpr int U = 2;
+  const u32 pivot = get(a.ctl + UC_PIVOT + 1);
+  while (at.valid()) {
+    Unit x[U];
+    u64 r0[U];
+    int have = 0;  // (wave-uniform)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      r0[u] = a.m;
+      if (at.valid()) {
+        r0[u] = at.unit * UNION_UNIT + 4 * lane_id();
+        load_unit<false>(x[u], a, at.unit);
+        at.next();
+        have = u + 1;
+      }
+    }
+    u32 live = 0;  // bit 4u + e
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u >= have) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32 s = x[u].s[e], d = x[u].d[e];
+        const u32 in = (inside[s >> 5] >> (s & 31)) & (inside[d >> 5] >> (d & 31)) & 1u;
+        live |= r0[u] + e < a.m && x[u].w[e] > pivot && s < d && !in ? 1u << (4 * u + e) : 0u;
+      }
+    }
+    if (!__any(live != 0)) continue;
+    u32 s[U][4], d[U][4];
+#pragma unroll
+    for (int k = 0; k < 4 * U; ++k) {
+      s[k / 4][k % 4] = d[k / 4][k % 4] = 0;
+      if ((live >> k) & 1) {
+        s[k / 4][k % 4] = a.parent[x[k / 4].s[k % 4]];
+        d[k / 4][k % 4] = a.parent[x[k / 4].d[k % 4]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u >= have) continue;
+      u64 k[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) k[e] = (u64(x[u].w[e]) << 32) | (r0[u] + e);
+      append_crossing(a, l, s[u], d[u], k, best, giant);
+    }
+  }
+}
+
+// ------------------------------------------------------------ rounds
+constexpr int UR = 4;  // rows of one edge per lane a wave loads before use
+
+// With `first` the minima are the light pass's, (weight << 32) | the other
+// end; parallel copies of one weight then share a minimum, so with copies in
+// the input the hook claims its child and one of them is taken.  Returns the
+// wave's roots that live on.
+__device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int cur, bool first,
+                                    bool copies, u32 giant, bool note) {
+  const u64* best = a.best[cur];
+  u64* next = a.best[cur ^ 1];
+  u32 live = 0;
+  for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
+    u32 x[UR], y[UR];
+    u64 k[UR], bx[UR], by[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u64 i = l.base + min<u32>(j0 + u * WAVE + lane_id(), l.c - 1);
+      x[u] = a.s[0][i];
+      y[u] = a.d[0][i];
+      k[u] = a.v[0][i];
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      bx[u] = get(best + x[u]);
+      by[u] = get(best + y[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u32 w = static_cast<u32>(k[u] >> 32);
+      // (the passive root's word is an old minimum)
+      const bool mx = bx[u] == (first ? dst_key(w, y[u]) : k[u]) && x[u] != giant;
+      const bool my = by[u] == (first ? dst_key(w, x[u]) : k[u]) && y[u] != giant;
+      if (j0 + u * WAVE + lane_id() >= l.c || (!mx && !my)) continue;
+      u32 child = x[u], other = y[u];
+      if (mx && my) {
+        child = max(x[u], y[u]);
+        other = min(x[u], y[u]);
+      } else if (my) {
+        child = y[u];
+        other = x[u];
+      }
+      if (copies) {
+        if (atomicCAS(a.parent + child, child, other) != child) continue;
+      } else {
+        put(a.parent + child, other);
+      }
+      if (mx && my) {
+        put(next + other, VAL_NONE);  // the root that lives on
+        if (note) put(a.ctl + UC_GIANT, other + 1);
+        ++live;
+      }
+      const u32 pos = static_cast<u32>(k[u]);
+      (void)__hip_atomic_fetch_or(a.marks + (pos >> 5), 1u << (pos & 31), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) live += __shfl_xor(live, o, WAVE);
+  return live;
+}
+
+// Rounds with at most this many live roots fold their offers in LDS; with
+// more, most offers of a workgroup are to distinct roots.
+constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
+constexpr u64 NOTE_LIVE = 64;  // hooks on at most this many roots note a survivor
+
+__device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
+                                        OfferTable& t, u32 giant, u32 wave) {
+  u64* best = a.best[out];
+  const bool table = live <= TABLE_LIVE;
+  // with few roots every wave meets the same ones: some waves' stores do
+  const u32 thin = !table ? 0u : live > 1024 ? 3u : live > 128 ? 31u : 255u;
+  if (table) {
+    table_clear(t);
+    __syncthreads();
+  }
+  u32 kept = 0;
+  for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
+    u32 xy[2 * UR];
+    u64 k[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u64 i = l.base + min<u32>(j0 + u * WAVE + lane_id(), l.c - 1);
+      xy[u] = a.s[0][i];
+      xy[UR + u] = a.d[0][i];
+      k[u] = a.v[0][i];
+    }
+    find_roots<2 * UR>(a.parent, xy, thin, wave, a.err);
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u32 x = xy[u], y = xy[UR + u];
+      const bool keep = j0 + u * WAVE + lane_id() < l.c && x != y;
+      const u64 b = __ballot(keep);
+      if (keep) {
+        // in place: the rows up to here have been read
+        const u64 q = l.base + kept + mbcnt(b);
+        a.s[0][q] = x;
+        a.d[0][q] = y;
+        a.v[0][q] = k[u];
+        if (table) {
+          if (x != giant) table_offer(t, best, x, k[u]);
+          if (y != giant) table_offer(t, best, y, k[u]);
+        } else {
+          offer_ends(best, x, y, k[u], giant);
+        }
+      }
+      kept += static_cast<u32>(__popcll(b));
+    }
+  }
+  l.c = kept;
+  if (table) {
+    __syncthreads();
+    table_flush(t, best);
+  }
+}
+
+// ------------------------------------------------------------ the solve
+union Scratch {
+  Stage stage[UW];
+  OfferTable table;
+  u16 pos[UW][UNION_UNIT * 8];  // marked positions of a wave's 64 mark words
+  u64 inside[UNION_VERTICES_MAX / 64];
+};
+
+// Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
+__device__ __forceinline__ u64 block_total(u64 wave_value) {
+  __shared__ u64 s_v[UW];
+  if (lane_id() == 0) s_v[wave_index()] = wave_value;
+  __syncthreads();
+  u64 t = 0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < UW; ++w) t += s_v[w];
+  return t;
+}
+
+__global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
+  __shared__ Scratch s_x;
+  __shared__ Found s_all;
+  if (!join_grid(a.joined)) return;
+  Barrier bar{a.bar, 0, a.err};
+  const u32 n = a.n;
+  const int lane = lane_id();
+  const u64 G = gridDim.x, gthread = u64(blockIdx.x) * UT + threadIdx.x, threads = G * UT;
+  const u64 wave = u64(blockIdx.x) * UW + wave_index(), waves = G * UW;
+  u64 sum;
+
+  // init
+  for (u64 v = gthread; v < n; v += threads) {
+    put(a.parent + v, static_cast<u32>(v));
+    put(a.best[0] + v, VAL_NONE);
+  }
+  const u64 words = (a.m + 31) / 32;
+  for (u64 i = gthread; i < words; i += threads) put(a.marks + i, 0u);
+  if (blockIdx.x == 0) pick_pivots(a);
+  if (!sync_grid(bar, 0, sum)) return;
+
+  // light pass
+  const u64 units = (a.m + UNION_UNIT - 1) / UNION_UNIT;
+  // a wave's range of the list buffers: as many edges as its chunks have
+  // records (only the input's last chunk may be short)
+  const u64 chunks = (units + a.chunk - 1) / a.chunk;
+  const u64 q = chunks / waves, rem = chunks % waves;
+  WaveLists l;
+  l.base = (wave * q + min(wave, rem)) * a.chunk * UNION_UNIT;
+  l.cap = (q + (wave < rem ? 1 : 0)) * a.chunk * UNION_UNIT;
+  l.c = l.c_mid = 0;
+  Found mine{};
+  light_pass(a, l, UnitWalk(a, wave, waves, units), s_x.stage[wave_index()], mine);
+  if (threadIdx.x == 0) {
+    u64* f = a.found + blockIdx.x * 4;
+    put(f, mine.hash_fwd);
+    put(f + 1, mine.hash_rev);
+    put(f + 2, (u64(mine.bad) << 32) | mine.dup);
+  }
+  if (!sync_grid(bar, mine.fwd, sum)) return;
+  if (wave_id() == 0) {
+    u64 hf = 0, hr = 0, bd = 0;
+    for (u32 b = lane; b < G; b += WAVE) {
+      hf += get(a.found + b * 4);
+      hr += get(a.found + b * 4 + 1);
+      bd |= get(a.found + b * 4 + 2);
+    }
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) {
+      hf += __shfl_xor(hf, o, WAVE);
+      hr += __shfl_xor(hr, o, WAVE);
+      bd |= __shfl_xor(bd, o, WAVE);
+    }
+    if (lane == 0)
+      s_all = Found{hf, hr, static_cast<u32>(sum), static_cast<u32>(bd >> 32), static_cast<u32>(bd)};
+  }
+  __syncthreads();
+  const Found all = s_all;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *a.fwd_count = all.fwd;
+    a.hsum[0] = all.hash_fwd;
+    a.hsum[1] = all.hash_rev;
+    if (all.bad) atomicOr(a.err, all.bad);
+  }
+  // the minima of a malformed input may hook a cycle: leave, the host reports
+  if (all.bad || u64(all.fwd) * 2 != a.m || all.hash_fwd != all.hash_rev) return;
+
+  // rounds of each class
+  const bool copies = all.dup != 0;
+  u32 round = 0, giant = NONE32;
+  int cur = 0;
+  for (u32 phase = 0; phase < 3; ++phase) {
+    if (phase > 0) {
+      // the minima are cleared for every vertex: a root that took no part in
+      // the last round holds an old one
+      giant = get(a.ctl + UC_GIANT) - 1;  // NONE32: none noted
+      for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
+        u32 x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          x[j] = static_cast<u32>(v0 + j * threads < n ? v0 + j * threads : v0);
+        find_roots<4>(a.parent, x, 0, 0, a.err);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
+          const u64 b = __ballot(v < n && x[j] == giant);
+          if (v < n) put(a.best[cur] + v, VAL_NONE);
+          if (lane == 0 && v < n) put(a.bits + v / 64, b);
+        }
+      }
+      if (!sync_grid(bar, 0, sum)) return;
+      // one wave acquires for the CU: the L1 is its workgroup's alone
+      if (wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      __syncthreads();
+      if (phase == 1) {
+        cross_mid(a, l, a.best[cur], giant);
+      } else {
+        for (u32 i = threadIdx.x; i < (n + 63) / 64; i += UT) s_x.inside[i] = a.bits[i];
+        __syncthreads();
+        cross_input(a, l, UnitWalk(a, wave, waves, units), a.best[cur], giant,
+                    reinterpret_cast<const u32*>(s_x.inside));
+      }
+    }
+    u64 edges, live = n;
+    if (!sync_grid(bar, block_total(l.c), edges)) return;
+    while (edges) {
+      if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges;
+      const bool first = phase == 0 && round == 0;
+      const u32 lw = hook(a, l, cur, first, first && copies, giant, live <= NOTE_LIVE);
+      if (!sync_grid(bar, block_total(lw), live)) return;
+      relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
+      cur ^= 1;
+      ++round;
+      if (!sync_grid(bar, block_total(l.c), edges)) return;
+      if (round >= UNION_ROUNDS_MAX) {
+        // every round at least halves the components that have edges
+        if (gthread == 0) atomicOr(a.err, ERR_SPIN);
+        return;
+      }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.log[UNION_LOG + phase] = round;
+    if (phase == 0 && !a.has_mid) ++phase;
+    if (phase == 1 && !a.has_heavy) ++phase;
+  }
+
+  // output: workgroups own equal contiguous parts of the mark words, their
+  // waves equal parts of those
+  const u64 rows = (words + WAVE - 1) / WAVE;  // rows of 64 words
+  const u64 r0 = (wave * rows) / waves, r1 = ((wave + 1) * rows) / waves;
+  u32 cnt = 0;
+  for (u64 r = r0; r < r1; ++r) {
+    const u64 w = r * WAVE + lane;
+    cnt += w < words ? static_cast<u32>(__popc(get(a.marks + w))) : 0u;
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, WAVE);
+  __shared__ u32 s_waves[UW];
+  __shared__ u64 s_base;
+  if (lane == 0) s_waves[wave_id()] = cnt;
+  const u64 block_count = block_total(cnt);
+  if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_count);
+  u64 total;
+  if (!sync_grid(bar, block_count, total)) return;
+  if (wave_id() == 0) {
+    u64 before = 0;
+    for (u32 b = lane; b < blockIdx.x; b += WAVE) before += get(a.found + b * 4 + 3);
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
+    if (lane == 0) s_base = before;
+  }
+  __syncthreads();
+  u64 at = s_base;
+  for (int w = 0; w < wave_id(); ++w) at += s_waves[w];
+  u16* pos = s_x.pos[wave_index()];
+  u64 weight = 0;
+  for (u64 r = r0; r < r1; ++r) {
+    const u64 w = r * WAVE + lane;
+    const u32 bits = w < words ? get(a.marks + w) : 0u;
+    const u32 c = static_cast<u32>(__popc(bits));
+    const u32 incl = wave_inclusive_sum(c);
+    const u32 row = __shfl(incl, WAVE - 1, WAVE);
+    u32 p = incl - c;
+    for (u32 b = bits; b; b &= b - 1) pos[p++] = static_cast<u16>(lane * 32 + __ffs(b) - 1);
+    __builtin_amdgcn_wave_barrier();
+    for (u32 j = lane; j < row; j += WAVE) {
+      const u64 e = r * (WAVE * 32) + pos[j], o = at + j;
+      const u32 wt = a.wt[e];
+      weight += wt;
+      if (o < a.out_cap) {
+        a.out_s[o] = a.src[e];
+        a.out_d[o] = a.dst[e];
+        a.out_w[o] = wt;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    at += row;
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) weight += __shfl_xor(weight, o, WAVE);
+  const u64 block_weight = block_total(weight);
+  if (threadIdx.x == 0) {
+    a.found[blockIdx.x * 4] = block_weight;
+    if (blockIdx.x == 0) {
+      *a.count = static_cast<u32>(total);
+      a.ctl[UC_DONE] = 1;
+    }
+  }
+}
+
+// Sums the workgroups' weights and counts the smaller endpoints with more
+// than MST_GROUP_SMALL edges in the output (the edge MST_GROUP_SMALL past the
+// first of its group counts the group).  The last workgroup to end publishes
+// the counters and the log, as publish_words does.
+__global__ __launch_bounds__(UT) void union_finish_kernel(UnionArgs a, u32 blocks, u64* total,
+                                                          u32* groups, u32* ended, Publication p) {
+  __shared__ u32 s_last;
+  const u64 count = a.ctl[UC_DONE] ? min<u64>(*a.count, a.out_cap) : 0;
+  u32 c = 0;
+  for (u64 i = u64(blockIdx.x) * UT + threadIdx.x + MST_GROUP_SMALL; i < count;
+       i += u64(gridDim.x) * UT) {
+    const u32 s = a.out_s[i];
+    c += s == a.out_s[i - MST_GROUP_SMALL] &&
+                 (i == MST_GROUP_SMALL || a.out_s[i - MST_GROUP_SMALL - 1] != s)
+             ? 1u
+             : 0u;
+  }
+  if (c) atomicAdd(groups, c);
+  if (blockIdx.x == 0 && wave_id() == 0) {
+    u64 w = 0;
+    for (u32 b = lane_id(); b < blocks; b += WAVE) w += a.found[b * 4];
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) w += __shfl_xor(w, o, WAVE);
+    if (lane_id() == 0) *total = w;
+  }
+  if (!p.host) return;
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = atomicAdd(ended, 1u) + 1 == gridDim.x ? 1u : 0u;
+  __syncthreads();
+  if (!s_last) return;
+  __threadfence();
+  for (u32 i = threadIdx.x; i < 64; i += UT) p.host[i] = get(a.ctr + i);
+  const u32* lg = reinterpret_cast<const u32*>(a.log);
+  for (u32 i = threadIdx.x; i < 2 * UNION_LOG_TOTAL; i += UT) p.host[p.extra_at + i] = get(lg + i);
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(p.host + p.seq_at, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace
+
+u64 union_mark_words(u64 m) { return (m + 31) / 32; }
+u32 union_samples(u64 m) { return static_cast<u32>(std::min<u64>(PIVOT_SAMPLES_MAX, m)); }
+
+u32 union_blocks(u64 m, u32 cus) {
+  // two units per wave at least: fewer workgroups make the barriers cheaper
+  const u64 want = (m + 2 * UW * UNION_UNIT - 1) / (2 * UW * UNION_UNIT);
+  return static_cast<u32>(std::max<u64>(1, std::min<u64>({want, cus, UNION_BLOCKS_MAX})));
+}
+
+u32 union_chunk(u64 m, u32 blocks) {
+  // long chunks spare atomics at their ends, several chunks per wave even out
+  // how many edges the waves list
+  const u64 per_wave = (m + UNION_UNIT - 1) / UNION_UNIT / (u64(blocks) * UW);
+  return static_cast<u32>(std::max<u64>(1, std::min<u64>(per_wave / 4, UNION_CHUNK_MAX)));
+}
+
+void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
+                 u32* ended, const Publication& p) {
+  if (blocks == 0 || blocks > UNION_BLOCKS_MAX) throw Error(KMST_EINVAL, "direct solve: workgroups");
+  {
+    KTScope t(st, K_PERSIST, 24.0 * a.m + 24.0 * a.n);
+    union_solve_kernel<<<blocks, UT, 0, st>>>(a);
+    KMST_HIP(hipGetLastError());
+  }
+  KTScope t(st, K_OTHER, 8.0 * a.n);
+  const u32 grid = static_cast<u32>(std::max<u64>(1, std::min<u64>((a.n + 4 * UT - 1) / (4 * UT), 64)));
+  union_finish_kernel<<<grid, UT, 0, st>>>(a, blocks, total, groups, ended, p);
+  KMST_HIP(hipGetLastError());
+}
+
+}  // namespace kmst
