@@ -422,6 +422,7 @@ struct UnionArgs {
   u64* v[2] = {nullptr, nullptr};
   u64* best[2] = {nullptr, nullptr};  // n + 1 words each
   u32* parent = nullptr;
+  u64* span = nullptr;   // per vertex, n + 1 words: its row's first position, its end << 32
   u64* bits = nullptr;   // one bit per vertex: the giant component
   u32* marks = nullptr;  // one bit per input position: MST edges
   u64* found = nullptr;  // 4 words per workgroup

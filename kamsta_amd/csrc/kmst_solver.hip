@@ -988,9 +988,8 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // graph is one launch and one read-back, where the round loop needs 60 to 190
 // launches and 7 to 27 read-backs.  Its random accesses are atomic minima and
 // root walks over 12 bytes per vertex: up to UNION_VERTICES_MAX the parent
-// array (4 bytes) fits an XCD's L2 and the bitmap of the giant component
-// (n / 8 bytes) the LDS.  Measured, direct / round loop: 110 / 179 us at 256
-// vertices, 235 / 528 at 2^14, 338 / 1400 at 2^17, 627 / 1746 and 843 / 2673 at
+// array (4 bytes) fits an XCD's L2.  Measured, direct / round loop: 110 / 179 us at 256
+// vertices, 235 / 528 at 2^14, 338 / 1400 at 2^17, 624 / 1746 and 808 / 2673 at
 // 10^6 (16 and 32 records per vertex).  Sparse inputs (fewer than two records per
 // vertex: forests) stay with the round loop, and so does a context whose
 // persistent-round limit was set by hand.
@@ -1039,6 +1038,7 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   a.best[0] = best_val;
   a.best[1] = state;
   a.parent = parent;
+  a.span = pos;
   a.bits = reinterpret_cast<u64*>(label);
   a.marks = marks;
   // log, barrier and the workgroups' words follow the counters

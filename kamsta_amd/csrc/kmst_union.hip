@@ -47,7 +47,7 @@
 // MB); atomic minima run at 26 10^9/s spread out and 12 10^6/s on one address.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
 // records 110 / 179 us; 2^14, 4.9 10^5 235 / 528 us; 2^17, 2.1 10^6 338 / 1400
-// us; 10^6, 3.2 10^7 843 / 2673 us (a copy of its bytes: 81 us).
+// us; 10^6, 3.2 10^7 808 / 2673 us (a copy of its bytes: 81 us).
 // Lists are private to a wave, so they need no coherence, counters or
 // workgroup barriers, and their compaction is in place.
 #include "kmst_kernels.hpp"
@@ -533,6 +533,7 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
   __shared__ Found s_found[UW];
   const int lane = lane_id();
   const u32 q0 = get(a.ctl + UC_PIVOT), q1 = get(a.ctl + UC_PIVOT + 1);
+  u32* span = reinterpret_cast<u32*>(a.span);
   // wave-uniform: lanes that saw an error or a parallel record, forward count
   u64 bad_id = 0, bad_order = 0, dup = 0;
   u32 fwd = 0;
@@ -564,6 +565,10 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       bad_id |= __ballot(hi >= a.n) | __ballot(lo == hi);
       bad_order |= __ballot(prev > here);  // (copies past the end equal their predecessor)
       dup |= __ballot(prev == here) & in;
+      if (ps != s) {  // (the first record's predecessor is (0, 0): row 0 ends, or begins, at 0)
+        put(span + 2 * u64(min(ps, a.n)) + 1, static_cast<u32>(r0 + e));
+        put(span + 2 * u64(min(s, a.n)), static_cast<u32>(r0 + e));
+      }
       ps = s;
       pd = d;
       const u64 f = __ballot(s < d) & in;
@@ -576,6 +581,7 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       b0[e] = f & l0;
       b1[e] = f & l1 & ~l0;
     }
+    if (r0 < a.m && r0 + 4 >= a.m) put(span + 2 * u64(min(x.s[3], a.n)) + 1, static_cast<u32>(a.m));
     run_minima(x, unit == 0, last, a.n, a.best[0], carry);
     // a lane's taken records leave one per step (a lane seldom takes more
     // than two, so this needs fewer steps than one per record)
@@ -637,8 +643,8 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
 // onto it, which is all a round needs to make progress.  Any root may be the
 // passive one; it is a root that lived on after the last hook of the phase
 // before (with few of them left each hook notes one).
-// The flatten marks its component in a bitmap (n / 8 bytes, at most 128 KB),
-// which the pass over the input keeps in LDS, and most records lie inside it.
+// The flatten marks its component in a bitmap (n / 8 bytes); most records lie
+// inside it.
 // Neither changes in these passes: after an acquire at agent scope plain loads
 // are current, and the gathers of a source's records hit the L1.
 __device__ __forceinline__ void offer_ends(u64* best, u32 s, u32 d, u64 k, u32 giant) {
@@ -693,12 +699,11 @@ __device__ __forceinline__ void cross_mid(const UnionArgs& a, WaveLists& l, u64*
   l.c_mid = 0;
 }
 
-// The rest of the input: the wave's own forward records above the pivot, two
+// The rest of the input where the giant leaves many records outside, or rows
+// too long for one wave: the wave's own forward records above the pivot, two
 // units per step, every load of a kind in flight before the next kind's.
-// `inside` is the giant's bitmap in LDS: gathered from the L2s, at 250 10^9/s,
-// its words alone took 80 of 150 us at 10^6 vertices, 1.6 10^7 edges.
 __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, UnitWalk at,
-                                            u64* best, u32 giant, const u32* inside) {
+                                            u64* best, u32 giant) {
   constexpr int U = 2;
   const u32 pivot = get(a.ctl + UC_PIVOT + 1);
   while (at.valid()) {
@@ -717,14 +722,26 @@ __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, Un
     }
     u32 live = 0;  // bit 4u + e
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (u >= have) continue;
+    for (int u = 0; u < U; ++u)
+      if (u < have)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const u32 s = x[u].s[e], d = x[u].d[e];
-        const u32 in = (inside[s >> 5] >> (s & 31)) & (inside[d >> 5] >> (d & 31)) & 1u;
-        live |= r0[u] + e < a.m && x[u].w[e] > pivot && s < d && !in ? 1u << (4 * u + e) : 0u;
+        for (int e = 0; e < 4; ++e)
+          live |= r0[u] + e < a.m && x[u].w[e] > pivot && x[u].s[e] < x[u].d[e] ? 1u << (4 * u + e) : 0u;
+    if (giant != NONE32) {
+      u64 bd[4 * U], bs[4 * U];
+#pragma unroll
+      for (int k = 0; k < 4 * U; ++k) {
+        bd[k] = 0;
+        bs[k] = 0;
+        if ((live >> k) & 1) {
+          bd[k] = a.bits[x[k / 4].d[k % 4] >> 6];
+          bs[k] = a.bits[x[k / 4].s[k % 4] >> 6];
+        }
       }
+#pragma unroll
+      for (int k = 0; k < 4 * U; ++k)
+        if ((bd[k] >> (x[k / 4].d[k % 4] & 63)) & (bs[k] >> (x[k / 4].s[k % 4] & 63)) & 1)
+          live &= ~(1u << k);
     }
     if (!__any(live != 0)) continue;
     u32 s[U][4], d[U][4];
@@ -743,6 +760,118 @@ __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, Un
 #pragma unroll
       for (int e = 0; e < 4; ++e) k[e] = (u64(x[u].w[e]) << 32) | (r0[u] + e);
       append_crossing(a, l, s[u], d[u], k, best, giant);
+    }
+  }
+}
+
+// The rest of the input where the giant leaves few records outside: a crossing
+// edge has an end outside, so the rows of the vertices outside hold them all.
+// A wave takes 64 vertices at a time (the flatten's share of the wave), and its
+// lanes spread over the records of their rows together.  An edge with one end
+// inside is found from its outer end; its key is the position of its forward
+// record, which a binary search of the inner end's row finds (no parallel
+// records: the position is unique).  At 10^6 vertices, 3.2 10^7 records: 12 us,
+// a pass over the input 146 us; at 2^24, 5.4 10^8: 130 to 200 us and 3.1 ms.
+constexpr u64 ROW_LONG = 4096;   // a longer row outside: cross_input instead
+constexpr u64 ROWS_SHARE = 4;    // also with more than 1/4 of the records outside
+struct Rows {
+  u32 upto[WAVE];   // records of the group's rows up to this one's end
+  u32 shift[WAVE];  // position of the row's j-th record of the group: shift + j
+  u32 root[WAVE];
+};
+__device__ __forceinline__ void cross_rows(const UnionArgs& a, WaveLists& l, u64 wave, u64 waves,
+                                           u64* best, u32 giant, Rows& rows) {
+  const u32 pivot = get(a.ctl + UC_PIVOT + 1);
+  const u64 groups = (u64(a.n) + WAVE - 1) / WAVE;
+  const u32 lane = lane_id();
+  for (u64 g0 = wave; g0 < groups; g0 += waves * WAVE) {
+    const u64 own = g0 + lane * waves;
+    const u64 word = own < groups ? a.bits[own] : ~0ull;
+    for (u64 todo = __ballot(word != ~0ull); todo; todo &= todo - 1) {
+      const u32 i = static_cast<u32>(__ffsll(static_cast<unsigned long long>(todo)) - 1);
+      const u64 v0 = (g0 + i * waves) * WAVE;
+      const u64 in = __shfl(static_cast<unsigned long long>(word), i, WAVE);
+      u32 begin = 0, len = 0, root = 0;
+      if (!((in >> lane) & 1) && v0 + lane < a.n) {
+        const u64 sp = a.span[v0 + lane];
+        begin = static_cast<u32>(sp);
+        len = static_cast<u32>(sp >> 32) - begin;
+        root = a.parent[v0 + lane];
+      }
+      const u32 upto = wave_inclusive_sum(len);
+      const u32 total = __shfl(upto, WAVE - 1, WAVE);
+      rows.upto[lane] = upto;
+      rows.shift[lane] = begin - (upto - len);
+      rows.root[lane] = root;
+      __builtin_amdgcn_wave_barrier();
+      for (u32 j0 = 0; j0 < total; j0 += 4 * WAVE) {
+        u32 s[4], d[4], rs[4], w[4], p[4];
+        bool ok[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const u32 j = min(j0 + e * WAVE + lane, total - 1);
+          u32 r = 0;
+#pragma unroll
+          for (u32 h = WAVE / 2; h > 0; h >>= 1) r += rows.upto[r + h - 1] <= j ? h : 0u;
+          p[e] = rows.shift[r] + j;
+          rs[e] = rows.root[r];
+          s[e] = static_cast<u32>(v0) + r;
+          d[e] = a.dst[p[e]];
+          w[e] = a.wt[p[e]];
+          ok[e] = j0 + e * WAVE + lane < total;
+        }
+        u32 rd[4];
+        bool inner[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ok[e] = ok[e] && w[e] > pivot;
+          inner[e] = ok[e] && ((a.bits[d[e] >> 6] >> (d[e] & 63)) & 1);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          rd[e] = giant;
+          if (ok[e] && !inner[e] && s[e] < d[e]) rd[e] = a.parent[d[e]];
+          ok[e] = ok[e] && (inner[e] || s[e] < d[e]) && rd[e] != rs[e];
+        }
+        // positions of the forward records
+        u32 lo[4], hi[4];
+        u32 open = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          lo[e] = p[e];
+          hi[e] = p[e];
+          if (ok[e] && s[e] > d[e]) {
+            const u64 sp = a.span[d[e]];
+            lo[e] = static_cast<u32>(sp);
+            hi[e] = static_cast<u32>(sp >> 32) - 1;
+          }
+        }
+        do {
+          u32 x[4];
+          open = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[e] = 0;
+            if (lo[e] < hi[e]) x[e] = a.dst[lo[e] + (hi[e] - lo[e]) / 2];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (lo[e] >= hi[e]) continue;
+            const u32 mid = lo[e] + (hi[e] - lo[e]) / 2;
+            if (x[e] < s[e]) lo[e] = mid + 1;
+            else hi[e] = mid;
+            open |= lo[e] < hi[e] ? 1u : 0u;
+          }
+        } while (__any(open != 0));
+        u64 k[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          k[e] = (u64(w[e]) << 32) | lo[e];
+          if (!ok[e]) rs[e] = rd[e];
+        }
+        append_crossing(a, l, rs, rd, k, best, giant);
+      }
+      __builtin_amdgcn_wave_barrier();
     }
   }
 }
@@ -869,7 +998,7 @@ union Scratch {
   Stage stage[UW];
   OfferTable table;
   u16 pos[UW][UNION_UNIT * 8];  // marked positions of a wave's 64 mark words
-  u64 inside[UNION_VERTICES_MAX / 64];
+  Rows rows[UW];
 };
 
 // Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
@@ -886,6 +1015,7 @@ __device__ __forceinline__ u64 block_total(u64 wave_value) {
 __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   __shared__ Scratch s_x;
   __shared__ Found s_all;
+  __shared__ u64 s_waves[UW], s_base;  // prefix sums over the waves
   if (!join_grid(a.joined)) return;
   Barrier bar{a.bar, 0, a.err};
   const u32 n = a.n;
@@ -898,6 +1028,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   for (u64 v = gthread; v < n; v += threads) {
     put(a.parent + v, static_cast<u32>(v));
     put(a.best[0] + v, VAL_NONE);
+    put(a.span + v, u64{0});
   }
   const u64 words = (a.m + 31) / 32;
   for (u64 i = gthread; i < words; i += threads) put(a.marks + i, 0u);
@@ -959,6 +1090,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
       // the minima are cleared for every vertex: a root that took no part in
       // the last round holds an old one
       giant = get(a.ctl + UC_GIANT) - 1;  // NONE32: none noted
+      u64 outside = 0;                    // the wave's records in rows outside it
       for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
         u32 x[4];
 #pragma unroll
@@ -971,19 +1103,38 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
           const u64 b = __ballot(v < n && x[j] == giant);
           if (v < n) put(a.best[cur] + v, VAL_NONE);
           if (lane == 0 && v < n) put(a.bits + v / 64, b);
+          if (phase == 2 && v < n && x[j] != giant) {
+            const u64 sp = get(a.span + v), len = (sp >> 32) - static_cast<u32>(sp);
+            outside += len > ROW_LONG ? a.m : len;
+          }
         }
       }
-      if (!sync_grid(bar, 0, sum)) return;
+#pragma unroll
+      for (int o = WAVE / 2; o > 0; o >>= 1) outside += __shfl_xor(outside, o, WAVE);
+      if (lane == 0) s_waves[wave_index()] = outside;
+      outside = min(block_total(outside), a.m);
+      if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, outside);
+      if (!sync_grid(bar, outside, sum)) return;
       // one wave acquires for the CU: the L1 is its workgroup's alone
       if (wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       __syncthreads();
       if (phase == 1) {
         cross_mid(a, l, a.best[cur], giant);
+      } else if (copies || sum * ROWS_SHARE > a.m) {
+        cross_input(a, l, UnitWalk(a, wave, waves, units), a.best[cur], giant);
       } else {
-        for (u32 i = threadIdx.x; i < (n + 63) / 64; i += UT) s_x.inside[i] = a.bits[i];
+        // a wave's list holds as many edges as its rows have records
+        if (wave_index() == 0) {
+          u64 before = 0;
+          for (u32 b = lane; b < blockIdx.x; b += WAVE) before += get(a.found + b * 4 + 3);
+#pragma unroll
+          for (int o = WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
+          if (lane == 0) s_base = before;
+        }
         __syncthreads();
-        cross_input(a, l, UnitWalk(a, wave, waves, units), a.best[cur], giant,
-                    reinterpret_cast<const u32*>(s_x.inside));
+        l.base = s_base;
+        for (u32 w = 0; w < wave_index(); ++w) l.base += s_waves[w];
+        cross_rows(a, l, wave, waves, a.best[cur], giant, s_x.rows[wave_index()]);
       }
     }
     u64 edges, live = n;
@@ -1019,8 +1170,6 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   }
 #pragma unroll
   for (int o = WAVE / 2; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, WAVE);
-  __shared__ u32 s_waves[UW];
-  __shared__ u64 s_base;
   if (lane == 0) s_waves[wave_id()] = cnt;
   const u64 block_count = block_total(cnt);
   if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_count);

@@ -86,11 +86,21 @@ def shape(name):
         u = np.repeat(np.arange(4), n - 4)
         v = np.tile(np.arange(4, n), 4)
         return n, u, v, rng.integers(1, 255, len(u))
+    if name in ("outer hub", "outer rows"):  # a dense block, and beside it rows of 5000 / 40 records
+        u, v = rng.integers(0, 9000, 200000), rng.integers(0, 9000, 200000)
+        u, v = np.unique(np.stack([np.minimum(u, v), np.maximum(u, v)])[:, u != v], axis=1)
+        wheels = 1 if name == "outer hub" else 100
+        rim = np.arange(5000 // wheels if wheels == 1 else 40)
+        size = len(rim) + 1
+        at = 9000 + size * np.arange(wheels)[:, None]
+        u = np.concatenate([u, (at + 0 * rim).ravel(), (at + 1 + rim[:-1]).ravel()])
+        v = np.concatenate([v, (at + 1 + rim).ravel(), (at + 2 + rim[:-1]).ravel()])
+        return 9000 + wheels * size, u, v, rng.integers(1, 255, len(u))
     raise KeyError(name)
 
 
 @pytest.mark.parametrize("name", ["pair", "triangle", "ring", "ladder", "parallel", "equal", "extremes",
-                                  "islands", "hubs"])
+                                  "islands", "hubs", "outer hub", "outer rows"])
 def test_shapes(gpu, ctx, name):
     n, u, v, w = shape(name)
     check(gpu, ctx, *symmetric(u, v, w), n)
