@@ -395,17 +395,19 @@ void persistent_rounds(hipStream_t st, const PersistArgs& a, u32 blocks);
 constexpr int UNION_THREADS = 1024;
 constexpr u32 UNION_BLOCKS_MAX = 256;  // one per CU
 constexpr u64 UNION_UNIT = 256;        // records a wave takes per step
-constexpr u64 UNION_VERTICES_MAX = u64{1} << 20;
+constexpr u64 UNION_VERTICES_MAX = u64{1} << 30;
+constexpr u32 UNION_CLASSES = 3;       // light weight classes at most
 constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
 constexpr u32 UNION_ROUNDS_MAX = 200;
-constexpr u32 UNION_LOG = 61;          // u64 words: list lengths of the rounds, ...
-constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 3 phases
+constexpr u32 UNION_LOG = 60;          // u64 words: rounds (edges, roots << 32), ...
+constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 4 phases
 constexpr u32 UNION_BAR_WORDS = 12 * 16;  // u64 words of the grid barrier
 enum : u32 {     // words of UnionArgs::ctl
-  UC_PIVOT = 0,  // two pivots: weights up to them are in the light pass's lists
-  UC_DONE = 2,   // the output is written
-  UC_GIANT = 3,  // 1 + a root that lived on after the last hook (0: none noted)
-  UC_WORDS = 4
+  UC_PIVOT = 0,  // UNION_CLASSES pivots: the classes' largest weights
+  UC_DONE = 3,   // the output is written
+  UC_FAR = 4,    // sampled records whose ids are FAR_SPAN or more apart
+  UC_RUNS = 5,   // sampled records that begin a run of one source
+  UC_WORDS = 8
 };
 struct UnionArgs {
   const u32 *src = nullptr, *dst = nullptr, *wt = nullptr;  // the input: m records, ids < n
@@ -413,9 +415,9 @@ struct UnionArgs {
   u32 n = 0;
   u32 chunk = 1;            // union_chunk(m, blocks)
   u32 samples = 0;          // union_samples(m)
-  u32 rank[2] = {0, 0};     // the pivots' ranks among the samples
-  bool has_mid = false;     // the second class is not empty (rank[0] < rank[1])
-  bool has_heavy = false;   // nor is what lies above it
+  u32 rank[UNION_CLASSES] = {0, 0, 0};  // the pivots' ranks among the samples, ascending
+  u32 classes = 1;          // light classes: the pivots from the last one on are the same
+  bool has_heavy = false;   // weights above them are left
   // list buffers of m edges, rounded up to whole chunks
   u32* s[2] = {nullptr, nullptr};
   u32* d[2] = {nullptr, nullptr};

@@ -184,10 +184,10 @@ enum Ctr : int {
   C_TOTAL64 = 16, C_HSUM64 = 18, C_ROUND64 = 22,
   C_CLASS64 = 24,   // MAX_CLASSES u64 class counts (words 24..41)
   C_UNION = 42,     // UC_WORDS control words of the direct solve
-  C_UJOINED = 46,   // its workgroups that were resident together
-  C_UENDED = 47,    // workgroups of its last launch that have ended
-  C_UCOUNT = 48,    // its MST edges
-  C_UGROUPS = 49,   // smaller endpoints with more than MST_GROUP_SMALL of them
+  C_UJOINED = 50,   // its workgroups that were resident together
+  C_UENDED = 51,    // workgroups of its last launch that have ended
+  C_UCOUNT = 52,    // its MST edges
+  C_UGROUPS = 53,   // smaller endpoints with more than MST_GROUP_SMALL of them
   C_OUTSIDE = 60    // outside_list: count (60), u64 total range length (62..63)
 };
 
@@ -985,16 +985,26 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 }
 
 // The direct solve takes every size from the device, so its cost on a small
-// graph is one launch and one read-back, where the round loop needs 60 to 190
-// launches and 7 to 27 read-backs.  Its random accesses are atomic minima and
-// root walks over 12 bytes per vertex: up to UNION_VERTICES_MAX the parent
-// array (4 bytes) fits an XCD's L2.  Measured, direct / round loop: 110 / 179 us at 256
-// vertices, 235 / 528 at 2^14, 338 / 1400 at 2^17, 624 / 1746 and 808 / 2673 at
-// 10^6 (16 and 32 records per vertex).  Sparse inputs (fewer than two records per
-// vertex: forests) stay with the round loop, and so does a context whose
-// persistent-round limit was set by hand.
+// graph is one launch and one read-back, where the round loop needs 60 to 250
+// launches and 7 to 34 read-backs; on a large one it moves each edge of the
+// lightest classes once a round and the others hardly at all, where the round
+// loop scatters, sorts and renumbers both records.  Measured, direct / round
+// loop: 110 / 179 us at 256 vertices, 238 / 549 at 2^14, 361 / 1394 at 2^17, 617
+// / 1736 and 821 / 2599 at 10^6 (16 and 32 records per vertex); 7.5 ms at 2^24
+// (32, random) against 10.4 filtering and 76 not, 5.0 / 8.0 geometric.  Sparse inputs (fewer than
+// two records per vertex: forests) stay with the round loop, and so does a
+// context whose persistent-round limit was set by hand.
+//
+// Light edges beyond what joins vertices stay in the lists round after round,
+// until their components meet: on a random graph 0.25 n of 1.1 n edges at
+// degree 2.2, 0.03 n of 0.7 n at 1.4.  From 2^16 vertices the rounds' work
+// outweighs the barriers of a second light class (at 2^17, 340 us with it, 390
+// without), from DIRECT_FINE_VERTICES that of a third (at 2^24 7.5 ms with three, 9.0
+// with two; at 10^6 random 815 / 835 us, geometric 710 / 650).
 constexpr double DIRECT_FIRST_DEGREE = 2.2;
 constexpr u64 DIRECT_MID_VERTICES = u64{1} << 16;
+constexpr double DIRECT_FINE_DEGREES[2] = {1.4, 2.4};
+constexpr u64 DIRECT_FINE_VERTICES = u64{1} << 21;
 bool Solver::use_direct() const {
   return n0 <= UNION_VERTICES_MAX && m0 >= 2 * u64(n0) &&
          C.tuning.persistent_max == PERSIST_MAX_DEFAULT;
@@ -1008,11 +1018,6 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   // whose crossing heavy edges fall off exponentially with it
   const double target = std::max(double(std::max<u64>(filter_threshold, 2)), 2.0 + std::log(degree));
   const bool heavy = target < 0.85 * degree;
-  const double light = heavy ? target / degree : 1.0;
-  // of those, first the DIRECT_FIRST_DEGREE lightest, where the rounds' work
-  // outweighs the barriers of another phase
-  const bool mid = n0 >= DIRECT_MID_VERTICES && DIRECT_FIRST_DEGREE < 0.7 * std::min(target, degree);
-  const double first = mid ? DIRECT_FIRST_DEGREE / degree : light;
   UnionArgs a;
   a.src = in_s;
   a.dst = in_d;
@@ -1025,10 +1030,16 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   auto rank = [&](double share) {
     return share >= 1.0 ? a.samples : static_cast<u32>(share * a.samples);
   };
-  a.rank[0] = rank(first);
-  a.rank[1] = rank(light);
-  a.has_mid = a.rank[0] < a.rank[1];
-  a.has_heavy = a.rank[1] < a.samples;
+  a.has_heavy = heavy;
+  a.classes = 0;
+  const bool fine = n0 >= DIRECT_FINE_VERTICES;
+  if (n0 >= DIRECT_MID_VERTICES)
+    for (int c = 0; c < (fine ? 2 : 1); ++c) {
+      const double step = fine ? DIRECT_FINE_DEGREES[c] : DIRECT_FIRST_DEGREE;
+      if (step < 0.7 * std::min(target, degree)) a.rank[a.classes++] = rank(step / degree);
+    }
+  for (u32 c = a.classes++; c < UNION_CLASSES; ++c) a.rank[c] = heavy ? rank(target / degree) : a.samples;
+  const u32 phases = a.classes + (a.has_heavy ? 1 : 0);
   a.s[0] = X.s;
   a.d[0] = X.d;
   a.v[0] = X.v;
@@ -1072,20 +1083,26 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   C.stats.mst_long_groups = C.host_counters[C_UGROUPS];
   u64 lg[UNION_LOG_TOTAL];
   std::memcpy(lg, C.host_counters + HOST_SAMPLE_WORD, sizeof(lg));
-  for (u32 i = 0; i < UNION_LOG && lg[i]; ++i) {
+  const u32* ctl = C.host_counters + C_UNION;
+  const u32 logged = static_cast<u32>(std::min<u64>(lg[UNION_LOG + phases - 1], UNION_LOG));
+  for (u32 i = 0; i < logged; ++i) {
     RoundStat rs;
-    rs.n = n0;
-    rs.m = lg[i];
-    rs.n_next = n0;
-    rs.m_next = i + 1 < UNION_LOG ? lg[i + 1] : 0;
+    rs.n = lg[i] >> 32;
+    rs.m = 2 * (lg[i] & 0xFFFFFFFFull);
+    if (i + 1 < logged) {
+      rs.n_next = lg[i + 1] >> 32;
+      rs.m_next = 2 * (lg[i + 1] & 0xFFFFFFFFull);
+    }
+    if (i == 0) rs.run_starts = ctl[UC_RUNS];
+    rs.twins = i == 0 && n0 > TWINS_MIN_N && 2 * ctl[UC_FAR] > a.samples;
     rs.direct = true;
     C.stats.rounds.push_back(rs);
   }
-  for (u32 p = 0; p < 3; ++p) {
-    if ((p == 1 && !a.has_mid) || (p == 2 && !a.has_heavy)) continue;
-    FilterStat f{0, m0, 2 * lg[0], C.host_counters[C_UNION + UC_PIVOT + (p == 2)], p == 0, 0};
-    if (p > 0) f.heavy_kept = 2 * lg[std::min<u64>(lg[UNION_LOG + (p == 2 && a.has_mid)], UNION_LOG - 1)];
-    C.stats.filter.push_back(f);
+  for (u32 p = 0; p < phases; ++p) {
+    const u64 at = p ? lg[UNION_LOG + p - 1] : 0;  // the phase's first round
+    const u64 m = at < UNION_LOG && at < lg[UNION_LOG + p] ? 2 * (lg[at] & 0xFFFFFFFFull) : 0;
+    C.stats.filter.push_back(FilterStat{0, m0, p ? 0 : m, ctl[UC_PIVOT + std::min(p, UNION_CLASSES - 1)],
+                                        p == 0, p ? m : 0, false});
   }
   *out_n = cnt;
   *total = counter64(C_TOTAL64);

@@ -7,11 +7,12 @@
 //   init     parent[v] = v, minima and edge marks cleared, weight pivots from
 //            a sample of the weights;
 //   light    one pass over the input: validation, every vertex's lightest
-//            record, and the forward (src < dst) records of the two lightest
-//            weight classes, each wave listing its own;
-//   rounds   hook and relabel (below) on the listed edges until none is left;
+//            record and row, and the forward (src < dst) records of the one to
+//            three lightest weight classes, each wave listing its own;
+//   rounds   hook and relabel (below) on the first class's edges until none is
+//            left;
 //   flatten  every vertex points at its root;
-//   cross    the second class, then the rest of the input: the edges that
+//   cross    the next class, at last the rest of the input: the edges that
 //            still join different components, followed by their rounds
 //            (boruvka_recursive, hybrid_boruvka_edgefilter.hpp:227-330, with
 //            the classes as its levels);
@@ -45,11 +46,15 @@
 // 11.4 us.  A launch per phase costs 4 us and more.  Agent-scope gathers run
 // at the rate of plain ones (250 10^9/s from a 4 MB table, 58 10^9/s from 64
 // MB); atomic minima run at 26 10^9/s spread out and 12 10^6/s on one address.
+// A large one is bound by random accesses, 8 to 16 bytes of 64 to 128 MB tables
+// for every listed edge and round, and by the light pass.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
-// records 110 / 179 us; 2^14, 4.9 10^5 235 / 528 us; 2^17, 2.1 10^6 338 / 1400
-// us; 10^6, 3.2 10^7 808 / 2673 us (a copy of its bytes: 81 us).
+// records 117 / 192 us; 2^14, 4.9 10^5 238 / 549 us; 2^17, 2.1 10^6 361 / 1394
+// us; 10^6, 3.2 10^7 821 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
+// 7.5 / 10.4 ms (1.36 ms).
 // Lists are private to a wave, so they need no coherence, counters or
-// workgroup barriers, and their compaction is in place.
+// workgroup barriers, and their compaction is in place (plain accesses: a wave's
+// range changes hands once, behind a release and an acquire).
 #include "kmst_kernels.hpp"
 
 namespace kmst {
@@ -302,35 +307,64 @@ __device__ __forceinline__ void table_flush(OfferTable& t, u64* best) {
 }
 
 // ------------------------------------------------------------ pivots
-// The sampled weights at ranks rank0 <= rank1 (a rank at or past `samples`:
-// all ones, everything is below), by workgroup 0: a radix select over 8-bit
+// The sampled weights at the classes' ranks (a rank at or past `samples`: all
+// ones, everything is below), by workgroup 0: a radix select over 8-bit
 // digits, histograms of the samples still in the running from the highest
-// digit that is not zero everywhere.
-constexpr u32 PIVOT_PER_THREAD = 1;
+// digit that is not zero everywhere.  A class's size strays by the square root
+// of its rank, and the first class is a few percent of a dense input: 4096
+// samples where a solve takes long enough to pay for them.
+constexpr u32 PIVOT_PER_THREAD = 4;
 constexpr u32 PIVOT_SAMPLES_MAX = UT * PIVOT_PER_THREAD;
+// Samples are runs of 16 records: 4096 records far apart are as many pages to
+// one CU, 40 us (1024: 10 us).
+constexpr u32 SAMPLE_RUN = 16;
 
-__device__ void pick_pivots(const UnionArgs& a) {
+__device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
   __shared__ u32 h[256];
   __shared__ u32 s_scan[UW];
-  __shared__ u32 s_digit, s_below, s_max;
+  __shared__ u32 s_digit, s_below, s_max, s_far, s_runs;
   const u32 t = threadIdx.x, samples = a.samples;
-  if (t == 0) s_max = 0;
+  const u32 runs_of = (samples + SAMPLE_RUN - 1) / SAMPLE_RUN;
+  if (t == 0) s_max = s_far = s_runs = 0;
   __syncthreads();
-  u32 x[PIVOT_PER_THREAD], mx = 0;
-  if (a.rank[0] < samples) {
+  u32 x[PIVOT_PER_THREAD], mx = 0, far = 0, runs = 0;
 #pragma unroll
-    for (u32 j = 0; j < PIVOT_PER_THREAD; ++j) {
-      const u64 q = min(j * UT + t, samples - 1);
-      x[j] = a.wt[(q * a.m) / samples];  // < m
-      mx = max(mx, x[j]);
+  for (u32 j = 0; j < PIVOT_PER_THREAD; ++j) {
+    const u32 q = j * UT + t;
+    x[j] = 0;
+    if (j * UT >= samples) continue;
+    const u32 r = min(q, samples - 1);
+    const u64 i = min((u64(r / SAMPLE_RUN) * a.m) / runs_of + r % SAMPLE_RUN, a.m - 1);
+    x[j] = a.wt[i];
+    mx = max(mx, x[j]);
+    if (q < samples) {
+      const u32 s = a.src[i], d = a.dst[i];
+      far += max(s, d) - min(s, d) >= FAR_SPAN ? 1u : 0u;
+      runs += i == 0 || a.src[i - 1] != s ? 1u : 0u;
     }
   }
-  atomicMax(&s_max, mx);
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    mx = max(mx, __shfl_xor(mx, o, WAVE));
+    far += __shfl_xor(far, o, WAVE);
+    runs += __shfl_xor(runs, o, WAVE);
+  }
+  if (lane_id() == 0) {
+    atomicMax(&s_max, mx);
+    atomicAdd(&s_far, far);
+    atomicAdd(&s_runs, runs);
+  }
   __syncthreads();
+  if (t == 0) {
+    put(a.ctl + UC_FAR, s_far);
+    put(a.ctl + UC_RUNS, s_runs);
+  }
   const int top = s_max >> 24 ? 24 : s_max >> 16 ? 16 : s_max >> 8 ? 8 : 0;
-  for (int which = 0; which < 2; ++which) {
-    u32 want = a.rank[which], pivot = NONE32;
-    if (want < samples) {
+  u32 pivot = NONE32;
+  for (u32 which = 0; which < UNION_CLASSES; ++which) {
+    u32 want = a.rank[which];
+    if (want >= samples) pivot = NONE32;
+    else if (which == 0 || want != a.rank[which - 1]) {
       u32 prefix = 0;
       for (int shift = top; shift >= 0; shift -= 8) {
         if (t < 256) h[t] = 0;
@@ -468,13 +502,14 @@ struct Found {
   u32 fwd, bad, dup;
 };
 
-// A wave's own lists: c edges from `base` on, and c_mid edges of the second
-// class from the end of the other buffer's same range of `cap` edges down.
-// Every edge comes from one of the wave's own records, so cap (their number)
-// is never exceeded, whatever the input.
+// A wave's own lists, in its range of `cap` edges of both buffers: c edges
+// from `base` of the first one on; the later light classes' rest1 and rest2 edges from
+// the range's end down, the second class in the second buffer and the third in
+// the first.  Every edge comes from one of the wave's own records, so cap
+// (their number) is never exceeded, whatever the input.
 struct WaveLists {
   u64 base, cap;
-  u32 c, c_mid;
+  u32 c, rest1, rest2;
 };
 
 // The units of a wave: chunks of `chunk` consecutive units, the chunks dealt
@@ -503,8 +538,8 @@ struct UnitWalk {
 // vertices, 3.2 10^7 records).  Class c at [c * STAGE, (c + 1) * STAGE).
 constexpr u32 STAGE = 2 * WAVE;
 struct Stage {
-  u32 s[2 * STAGE], d[2 * STAGE];
-  u64 v[2 * STAGE];
+  u32 s[UNION_CLASSES * STAGE], d[UNION_CLASSES * STAGE];
+  u64 v[UNION_CLASSES * STAGE];
 };
 
 // The first min(n, 64) staged edges of a class to its list, the rest (fewer
@@ -513,13 +548,13 @@ template <int CLASS>
 __device__ __forceinline__ void drain(const UnionArgs& a, WaveLists& l, Stage& st, u32& n) {
   const u32 lane = lane_id(), at = CLASS * STAGE + lane, out = min<u32>(n, WAVE);
   if (lane < out) {
-    const u64 q = CLASS ? l.base + l.cap - 1 - (l.c_mid + lane) : l.base + l.c + lane;
-    a.s[CLASS][q] = st.s[at];
-    a.d[CLASS][q] = st.d[at];
-    a.v[CLASS][q] = st.v[at];
+    const u64 q = CLASS ? l.base + l.cap - 1 - ((CLASS == 1 ? l.rest1 : l.rest2) + lane)
+                        : l.base + l.c + lane;
+    a.s[CLASS & 1][q] = st.s[at];
+    a.d[CLASS & 1][q] = st.d[at];
+    a.v[CLASS & 1][q] = st.v[at];
   }
-  if (CLASS) l.c_mid += out;
-  else l.c += out;
+  (CLASS == 0 ? l.c : CLASS == 1 ? l.rest1 : l.rest2) += out;
   n -= out;
   if (lane < n) {
     st.s[at] = st.s[at + WAVE];
@@ -532,14 +567,15 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
                                            Found& out) {
   __shared__ Found s_found[UW];
   const int lane = lane_id();
-  const u32 q0 = get(a.ctl + UC_PIVOT), q1 = get(a.ctl + UC_PIVOT + 1);
+  const u32 q0 = get(a.ctl + UC_PIVOT), q1 = get(a.ctl + UC_PIVOT + 1),
+            q2 = get(a.ctl + UC_PIVOT + 2);
   u32* span = reinterpret_cast<u32*>(a.span);
   // wave-uniform: lanes that saw an error or a parallel record, forward count
   u64 bad_id = 0, bad_order = 0, dup = 0;
   u32 fwd = 0;
   u64 hf = 0, hall = 0;  // hash sums of the forward and of all records
   Carry carry{0, 0, 0, false};
-  u32 n0 = 0, n1 = 0;  // staged edges of the two classes
+  u32 n0 = 0, n1 = 0, n2 = 0;  // staged edges of the classes
   Unit next;
   if (at.valid()) load_unit<true>(next, a, at.unit);
   while (at.valid()) {
@@ -555,7 +591,7 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       ps = x.ps;
       pd = x.pd;
     }
-    u64 b0[4], b1[4];
+    u64 listed[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const u32 s = x.s[e], d = x.d[e], w = x.w[e];
@@ -572,47 +608,39 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       ps = s;
       pd = d;
       const u64 f = __ballot(s < d) & in;
-      const u64 l0 = __ballot(w <= q0), l1 = __ballot(w <= q1);
       u64 h = sym_hash(lo, hi, w);
       if (!full && r0 + e >= a.m) h = 0;
       fwd += static_cast<u32>(__popcll(f));
       hf += s < d ? h : 0ull;
       hall += h;
-      b0[e] = f & l0;
-      b1[e] = f & l1 & ~l0;
+      listed[e] = f & __ballot(w <= q2);
     }
     if (r0 < a.m && r0 + 4 >= a.m) put(span + 2 * u64(min(x.s[3], a.n)) + 1, static_cast<u32>(a.m));
     run_minima(x, unit == 0, last, a.n, a.best[0], carry);
-    // a lane's taken records leave one per step (a lane seldom takes more
-    // than two, so this needs fewer steps than one per record)
-    u32 take = 0, mids = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      take |= ((b0[e] | b1[e]) >> lane) & 1ull ? 1u << e : 0u;
-      mids |= (b1[e] >> lane) & 1ull ? 1u << e : 0u;
-    }
-    while (__any(take != 0)) {
-      const u32 e = static_cast<u32>(__ffs(take) - 1);
-      const bool any = take != 0, mid = any && ((mids >> e) & 1u);
-      const u64 t0 = __ballot(any && !mid), t1 = __ballot(mid);
-      if (any) {
-        const u32 s = e < 2 ? (e ? x.s[1] : x.s[0]) : (e == 2 ? x.s[2] : x.s[3]);
-        const u32 d = e < 2 ? (e ? x.d[1] : x.d[0]) : (e == 2 ? x.d[2] : x.d[3]);
-        const u32 w = e < 2 ? (e ? x.w[1] : x.w[0]) : (e == 2 ? x.w[2] : x.w[3]);
-        const u32 q = mid ? STAGE + n1 + mbcnt(t1) : n0 + mbcnt(t0);
-        st.s[q] = s;
-        st.d[q] = d;
+      if (!listed[e]) continue;
+      const u32 w = x.w[e];
+      const u64 b0 = listed[e] & __ballot(w <= q0), b1 = listed[e] & __ballot(w <= q1) & ~b0,
+                b2 = listed[e] & ~(b0 | b1);
+      if ((listed[e] >> lane) & 1) {
+        u32 q = n0 + mbcnt(b0);
+        if (w > q0) q = w > q1 ? 2 * STAGE + n2 + mbcnt(b2) : STAGE + n1 + mbcnt(b1);
+        st.s[q] = x.s[e];
+        st.d[q] = x.d[e];
         st.v[q] = (u64(w) << 32) | (r0 + e);
-        take &= take - 1;
       }
-      n0 += static_cast<u32>(__popcll(t0));
-      n1 += static_cast<u32>(__popcll(t1));
+      n0 += static_cast<u32>(__popcll(b0));
+      n1 += static_cast<u32>(__popcll(b1));
+      n2 += static_cast<u32>(__popcll(b2));
       if (n0 >= WAVE) drain<0>(a, l, st, n0);
       if (n1 >= WAVE) drain<1>(a, l, st, n1);
+      if (n2 >= WAVE) drain<2>(a, l, st, n2);
     }
   }
   if (n0) drain<0>(a, l, st, n0);
   if (n1) drain<1>(a, l, st, n1);
+  if (n2) drain<2>(a, l, st, n2);
 #pragma unroll
   for (int o = WAVE / 2; o > 0; o >>= 1) {
     hf += __shfl_xor(hf, o, WAVE);
@@ -641,12 +669,23 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
 // take one atomic per edge at one address.  It gets none: a root without a
 // minimum hooks nowhere, and the components that choose an edge to it hook
 // onto it, which is all a round needs to make progress.  Any root may be the
-// passive one; it is a root that lived on after the last hook of the phase
-// before (with few of them left each hook notes one).
+// passive one: the most frequent root of 64 sampled vertices.
 // The flatten marks its component in a bitmap (n / 8 bytes); most records lie
 // inside it.
 // Neither changes in these passes: after an acquire at agent scope plain loads
 // are current, and the gathers of a source's records hit the L1.
+__device__ __forceinline__ u32 pick_giant(const UnionArgs& a) {
+  // (the roots do not change meanwhile: every workgroup picks the same)
+  u32 x[1] = {static_cast<u32>((u64(lane_id()) * a.n) / WAVE)};
+  find_roots<1>(a.parent, x, NONE32, 0, a.err);
+  u32 votes = 0;
+  for (int i = 0; i < WAVE; ++i) votes += __shfl(x[0], i, WAVE) == x[0] ? 1u : 0u;
+  u32 most = votes;
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, WAVE));
+  return __shfl(x[0], __ffsll(static_cast<unsigned long long>(__ballot(votes == most))) - 1, WAVE);
+}
+
 __device__ __forceinline__ void offer_ends(u64* best, u32 s, u32 d, u64 k, u32 giant) {
   if (s != giant) offer(best, s, k);
   if (d != giant) offer(best, d, k);
@@ -672,31 +711,34 @@ __device__ __forceinline__ void append_crossing(const UnionArgs& a, WaveLists& l
   }
 }
 
-// Second class: the wave's own list, from its low end up (what is appended
-// never reaches what is still to be read: both fit the wave's range).
-__device__ __forceinline__ void cross_mid(const UnionArgs& a, WaveLists& l, u64* best, u32 giant) {
-  const u64 lo = l.base + l.cap - l.c_mid;
-  for (u32 j0 = 0; j0 < l.c_mid; j0 += 4 * WAVE) {
+// A later light class: the wave's own list, from its low end up (the third
+// class's crossing edges go to the same range's front: what is appended never
+// reaches what is still to be read).
+__device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32 cls, u64* best,
+                                           u32 giant) {
+  const u32 *ls = a.s[cls & 1], *ld = a.d[cls & 1], listed = cls == 1 ? l.rest1 : l.rest2;
+  const u64* lv = a.v[cls & 1];
+  const u64 lo = l.base + l.cap - listed;
+  for (u32 j0 = 0; j0 < listed; j0 += 4 * WAVE) {
     u32 x[8], s[4], d[4];
     u64 k[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const u64 q = lo + min<u32>(j0 + e * WAVE + lane_id(), l.c_mid - 1);
-      x[e] = a.s[1][q];
-      x[4 + e] = a.d[1][q];
-      k[e] = a.v[1][q];
+      const u64 q = lo + min<u32>(j0 + e * WAVE + lane_id(), listed - 1);
+      x[e] = ls[q];
+      x[4 + e] = ld[q];
+      k[e] = lv[q];
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = a.parent[x[e]];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const bool in = j0 + e * WAVE + lane_id() < l.c_mid;
+      const bool in = j0 + e * WAVE + lane_id() < listed;
       s[e] = in ? x[e] : 0u;
       d[e] = in ? x[4 + e] : 0u;
     }
     append_crossing(a, l, s, d, k, best, giant);
   }
-  l.c_mid = 0;
 }
 
 // The rest of the input where the giant leaves many records outside, or rows
@@ -705,7 +747,7 @@ __device__ __forceinline__ void cross_mid(const UnionArgs& a, WaveLists& l, u64*
 __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, UnitWalk at,
                                             u64* best, u32 giant) {
   constexpr int U = 2;
-  const u32 pivot = get(a.ctl + UC_PIVOT + 1);
+  const u32 pivot = get(a.ctl + UC_PIVOT + UNION_CLASSES - 1);
   while (at.valid()) {
     Unit x[U];
     u64 r0[U];
@@ -727,7 +769,7 @@ __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, Un
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           live |= r0[u] + e < a.m && x[u].w[e] > pivot && x[u].s[e] < x[u].d[e] ? 1u << (4 * u + e) : 0u;
-    if (giant != NONE32) {
+    {
       u64 bd[4 * U], bs[4 * U];
 #pragma unroll
       for (int k = 0; k < 4 * U; ++k) {
@@ -781,7 +823,7 @@ struct Rows {
 };
 __device__ __forceinline__ void cross_rows(const UnionArgs& a, WaveLists& l, u64 wave, u64 waves,
                                            u64* best, u32 giant, Rows& rows) {
-  const u32 pivot = get(a.ctl + UC_PIVOT + 1);
+  const u32 pivot = get(a.ctl + UC_PIVOT + UNION_CLASSES - 1);
   const u64 groups = (u64(a.n) + WAVE - 1) / WAVE;
   const u32 lane = lane_id();
   for (u64 g0 = wave; g0 < groups; g0 += waves * WAVE) {
@@ -884,7 +926,7 @@ constexpr int UR = 4;  // rows of one edge per lane a wave loads before use
 // the input the hook claims its child and one of them is taken.  Returns the
 // wave's roots that live on.
 __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int cur, bool first,
-                                    bool copies, u32 giant, bool note) {
+                                    bool copies, u32 giant) {
   const u64* best = a.best[cur];
   u64* next = a.best[cur ^ 1];
   u32 live = 0;
@@ -925,7 +967,6 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
       }
       if (mx && my) {
         put(next + other, VAL_NONE);  // the root that lives on
-        if (note) put(a.ctl + UC_GIANT, other + 1);
         ++live;
       }
       const u32 pos = static_cast<u32>(k[u]);
@@ -941,7 +982,6 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
 // Rounds with at most this many live roots fold their offers in LDS; with
 // more, most offers of a workgroup are to distinct roots.
 constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
-constexpr u64 NOTE_LIVE = 64;  // hooks on at most this many roots note a survivor
 
 __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
                                         OfferTable& t, u32 giant, u32 wave) {
@@ -1004,6 +1044,7 @@ union Scratch {
 // Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
 __device__ __forceinline__ u64 block_total(u64 wave_value) {
   __shared__ u64 s_v[UW];
+  __syncthreads();  // thread 0 may still be adding the call before
   if (lane_id() == 0) s_v[wave_index()] = wave_value;
   __syncthreads();
   u64 t = 0;
@@ -1016,6 +1057,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   __shared__ Scratch s_x;
   __shared__ Found s_all;
   __shared__ u64 s_waves[UW], s_base;  // prefix sums over the waves
+  __shared__ u32 s_giant;
   if (!join_grid(a.joined)) return;
   Barrier bar{a.bar, 0, a.err};
   const u32 n = a.n;
@@ -1044,7 +1086,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   WaveLists l;
   l.base = (wave * q + min(wave, rem)) * a.chunk * UNION_UNIT;
   l.cap = (q + (wave < rem ? 1 : 0)) * a.chunk * UNION_UNIT;
-  l.c = l.c_mid = 0;
+  l.c = l.rest1 = l.rest2 = 0;
   Found mine{};
   light_pass(a, l, UnitWalk(a, wave, waves, units), s_x.stage[wave_index()], mine);
   if (threadIdx.x == 0) {
@@ -1085,12 +1127,20 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   const bool copies = all.dup != 0;
   u32 round = 0, giant = NONE32;
   int cur = 0;
-  for (u32 phase = 0; phase < 3; ++phase) {
+  u64 live = n;  // roots, where this is known
+  for (u32 phase = 0; phase < a.classes + (a.has_heavy ? 1 : 0); ++phase) {
+    const bool last = phase == a.classes;
     if (phase > 0) {
-      // the minima are cleared for every vertex: a root that took no part in
-      // the last round holds an old one
-      giant = get(a.ctl + UC_GIANT) - 1;  // NONE32: none noted
+      // the minima are cleared for every root: one that took no part in the last
+      // round holds an old one
+      // cross_rows moves the lists' ranges to other waves: a line that one XCD's
+      // L2 still holds dirty would be written back over what another wrote since
+      if (last && wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      if (wave_index() == 0) s_giant = pick_giant(a);
+      __syncthreads();
+      giant = s_giant;
       u64 outside = 0;                    // the wave's records in rows outside it
+      u32 roots = 0;
       for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
         u32 x[4];
 #pragma unroll
@@ -1101,9 +1151,11 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
         for (int j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
           const u64 b = __ballot(v < n && x[j] == giant);
-          if (v < n) put(a.best[cur] + v, VAL_NONE);
+          const bool root = v < n && x[j] == v;
+          if (root) put(a.best[cur] + v, VAL_NONE);
+          roots += static_cast<u32>(__popcll(__ballot(root)));
           if (lane == 0 && v < n) put(a.bits + v / 64, b);
-          if (phase == 2 && v < n && x[j] != giant) {
+          if (last && v < n && x[j] != giant) {
             const u64 sp = get(a.span + v), len = (sp >> 32) - static_cast<u32>(sp);
             outside += len > ROW_LONG ? a.m : len;
           }
@@ -1113,13 +1165,23 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
       for (int o = WAVE / 2; o > 0; o >>= 1) outside += __shfl_xor(outside, o, WAVE);
       if (lane == 0) s_waves[wave_index()] = outside;
       outside = min(block_total(outside), a.m);
-      if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, outside);
+      const u64 block_roots = block_total(roots);
+      if (threadIdx.x == 0) {
+        put(a.found + blockIdx.x * 4 + 2, block_roots);
+        put(a.found + blockIdx.x * 4 + 3, outside);
+      }
       if (!sync_grid(bar, outside, sum)) return;
       // one wave acquires for the CU: the L1 is its workgroup's alone
       if (wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       __syncthreads();
-      if (phase == 1) {
-        cross_mid(a, l, a.best[cur], giant);
+      if (wave == 0) {  // (for the log)
+        live = 0;
+        for (u32 b = lane; b < G; b += WAVE) live += get(a.found + b * 4 + 2);
+#pragma unroll
+        for (int o = WAVE / 2; o > 0; o >>= 1) live += __shfl_xor(live, o, WAVE);
+      }
+      if (!last) {
+        cross_list(a, l, phase, a.best[cur], giant);
       } else if (copies || sum * ROWS_SHARE > a.m) {
         cross_input(a, l, UnitWalk(a, wave, waves, units), a.best[cur], giant);
       } else {
@@ -1137,12 +1199,12 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
         cross_rows(a, l, wave, waves, a.best[cur], giant, s_x.rows[wave_index()]);
       }
     }
-    u64 edges, live = n;
+    u64 edges;
     if (!sync_grid(bar, block_total(l.c), edges)) return;
     while (edges) {
-      if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges;
+      if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges | (live << 32);
       const bool first = phase == 0 && round == 0;
-      const u32 lw = hook(a, l, cur, first, first && copies, giant, live <= NOTE_LIVE);
+      const u32 lw = hook(a, l, cur, first, first && copies, giant);
       if (!sync_grid(bar, block_total(lw), live)) return;
       relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
       cur ^= 1;
@@ -1155,8 +1217,6 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
       }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) a.log[UNION_LOG + phase] = round;
-    if (phase == 0 && !a.has_mid) ++phase;
-    if (phase == 1 && !a.has_heavy) ++phase;
   }
 
   // output: workgroups own equal contiguous parts of the mark words, their
@@ -1265,7 +1325,9 @@ __global__ __launch_bounds__(UT) void union_finish_kernel(UnionArgs a, u32 block
 }  // namespace
 
 u64 union_mark_words(u64 m) { return (m + 31) / 32; }
-u32 union_samples(u64 m) { return static_cast<u32>(std::min<u64>(PIVOT_SAMPLES_MAX, m)); }
+u32 union_samples(u64 m) {
+  return static_cast<u32>(std::min<u64>(m >= (u64{1} << 22) ? PIVOT_SAMPLES_MAX : UT, m));
+}
 
 u32 union_blocks(u64 m, u32 cus) {
   // two units per wave at least: fewer workgroups make the barriers cheaper
