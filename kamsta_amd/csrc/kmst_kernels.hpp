@@ -395,7 +395,7 @@ void persistent_rounds(hipStream_t st, const PersistArgs& a, u32 blocks);
 constexpr int UNION_THREADS = 1024;
 constexpr u32 UNION_BLOCKS_MAX = 256;  // one per CU
 constexpr u64 UNION_UNIT = 256;        // records a wave takes per step
-constexpr u64 UNION_VERTICES_MAX = u64{1} << 30;
+constexpr u64 UNION_VERTICES_MAX = u64{1} << 28;
 constexpr u32 UNION_CLASSES = 3;       // light weight classes at most
 constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
 constexpr u32 UNION_ROUNDS_MAX = 200;
@@ -425,7 +425,13 @@ struct UnionArgs {
   u64* best[2] = {nullptr, nullptr};  // n + 1 words each
   u32* parent = nullptr;
   u64* span = nullptr;   // per vertex, n + 1 words: its row's first position, its end << 32
-  u64* bits = nullptr;   // one bit per vertex: the giant component
+  u64* bits = nullptr;   // one bit per vertex: it is in the giant component (of its part)
+  // a graph of `parts` unconnected parts (0: not known to be one): part p holds
+  // the vertices part_off[p] .. part_off[p + 1] - 1
+  const u32* part_off = nullptr;
+  u32 parts = 0;
+  u32* part_giant = nullptr;  // per part
+  u8* giants = nullptr;       // one byte per vertex: it is its part's giant's root
   u32* marks = nullptr;  // one bit per input position: MST edges
   u64* found = nullptr;  // 4 words per workgroup
   u64* bar = nullptr;    // UNION_BAR_WORDS, zero

@@ -1051,6 +1051,12 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   a.parent = parent;
   a.span = pos;
   a.bits = reinterpret_cast<u64*>(label);
+  if (part_count > 1) {
+    a.part_off = part;
+    a.parts = part_count;
+    a.part_giant = part_giant;
+    a.giants = reinterpret_cast<u8*>(rep);
+  }
   a.marks = marks;
   // log, barrier and the workgroups' words follow the counters
   a.ctr = ctr;

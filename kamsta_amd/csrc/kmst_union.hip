@@ -83,11 +83,37 @@ template <typename T>
 __device__ __forceinline__ void put(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// Element i of a per-vertex array: with at most UNION_VERTICES_MAX vertices the
+// byte offset fits 32 bits, so the access takes a scalar base and one register.
+template <typename T>
+__device__ __forceinline__ T* at(T* base, u32 i) {
+  return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + u32(i * u32(sizeof(T))));
+}
+template <typename T>
+__device__ __forceinline__ const T* at(const T* base, u32 i) {
+  return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + u32(i * u32(sizeof(T))));
+}
+__device__ __forceinline__ u64* minima(const UnionArgs& a, int which) {
+  return which ? a.best[1] : a.best[0];
+}
+
 __device__ __forceinline__ void lower(u64* best, u32 v, u64 k) {
-  (void)__hip_atomic_fetch_min(best + v, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  (void)__hip_atomic_fetch_min(at(best, v), k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void offer(u64* best, u32 v, u64 k) {
-  if (k < get(best + v)) lower(best, v, k);
+  if (k < get(at(best, v))) lower(best, v, k);
+}
+
+// Lane shifts by DPP: one instruction, where a shuffle is a round trip through
+// the LDS.  Lanes without a source keep `old`.
+constexpr int DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;  // from the lane after, before
+constexpr int DPP_ROW_SHR = 0x110;                           // + o: from o lanes before, of 16
+constexpr int DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ u32 dpp(u32 old, u32 x) {
+  return static_cast<u32>(__builtin_amdgcn_update_dpp(static_cast<int>(old), static_cast<int>(x),
+                                                      CTRL, ROWS, 0xF, false));
 }
 
 // ------------------------------------------------------------ barrier
@@ -195,15 +221,15 @@ __device__ __forceinline__ void load4(const u32* p, u32 (&x)[4]) {
   for (int e = 0; e < 4; ++e) x[e] = v[e];
 }
 
-// One wave's 256 consecutive records, lane l those at 4l .. 4l + 3, and the
-// record before them ((0, 0), which no valid record precedes, before the
-// first).  Past the end: copies of the last record, which change no minimum.
+// One wave's 256 consecutive records, lane l those at 4l .. 4l + 3; past the
+// end copies of the last record, which change no minimum.  With `before`, lane
+// 0 also gets the record before them ((0, 0), which no valid record precedes,
+// before the first); by vector loads: LDS accesses would wait for scalar ones.
 struct Unit {
   u32 s[4], d[4], w[4];
   u32 ps, pd;
 };
-template <bool PREV>
-__device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit) {
+__device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit, bool before) {
   const u64 r0 = unit * UNION_UNIT + 4 * lane_id();
   if ((unit + 1) * UNION_UNIT <= a.m) {
     load4(a.src + r0, x.s);
@@ -218,10 +244,12 @@ __device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit)
       x.w[e] = a.wt[i];
     }
   }
-  if (PREV) {
-    const u64 i = unit * UNION_UNIT;
-    x.ps = i ? a.src[i - 1] : 0u;
-    x.pd = i ? a.dst[i - 1] : 0u;
+  if (before) {
+    x.ps = x.pd = 0;
+    if (r0 != 0) {
+      x.ps = a.src[min(r0, a.m) - 1];
+      x.pd = a.dst[min(r0, a.m) - 1];
+    }
   }
 }
 
@@ -236,7 +264,7 @@ template <int N>
 __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u32 salt, u32* err) {
   u32 p[N];
 #pragma unroll
-  for (int j = 0; j < N; ++j) p[j] = get(parent + x[j]);
+  for (int j = 0; j < N; ++j) p[j] = get(at(parent, x[j]));
   u32 open = 0, moved = 0;  // bit j: walk j has not ended / has left its first parent
 #pragma unroll
   for (int j = 0; j < N; ++j) open |= p[j] != x[j] ? 1u << j : 0u;
@@ -245,7 +273,7 @@ __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       y[j] = p[j];
-      if ((open >> j) & 1) y[j] = get(parent + p[j]);
+      if ((open >> j) & 1) y[j] = get(at(parent, p[j]));
     }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -254,7 +282,7 @@ __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u
       } else {
         moved |= 1u << j;
         p[j] = y[j];
-        if ((step & 7) == 0) put(parent + x[j], y[j]);
+        if ((step & 7) == 0) put(at(parent, x[j]), y[j]);
       }
     }
     if (step > WALK_LIMIT) {
@@ -265,7 +293,7 @@ __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     if (((moved >> j) & 1) && ((((x[j] * 0x9E3779B1u) >> 16) ^ salt) & thin) == 0)
-      put(parent + x[j], p[j]);
+      put(at(parent, x[j]), p[j]);
     x[j] = p[j];
   }
 }
@@ -361,6 +389,7 @@ __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
   }
   const int top = s_max >> 24 ? 24 : s_max >> 16 ? 16 : s_max >> 8 ? 8 : 0;
   u32 pivot = NONE32;
+#pragma unroll
   for (u32 which = 0; which < UNION_CLASSES; ++which) {
     u32 want = a.rank[which];
     if (want >= samples) pivot = NONE32;
@@ -398,7 +427,13 @@ __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
 }
 
 // ------------------------------------------------------------ light pass
-// Bound: 12 bytes per record from HBM, then instruction issue.
+// Bound: 12 bytes per record from HBM, which it reads at 3.3 of the 4.9 TB/s of
+// a copy at 10^6 vertices (3.2 10^7 records, 122 us) and at 2^24 (5.4 10^8, 1.87
+// ms; 16 records per vertex 68 us and 1.0 ms).  The loads alone take 68 us at
+// 10^6; listing the light edges adds 20 us, rows 13 us, minima 20 us (vector
+// instructions fill 60 % of the issue slots; 143 us with shuffles through the
+// LDS, wave-wide error masks, scalar loads that LDS accesses waited for, and
+// atomics at the chunks' ends one by one).  Two units per step were slower (140).
 //
 // A list edge's key is (weight << 32) | the record's position.  Positions
 // follow (min, max), so keys order the edges by (weight, min, max), parallel
@@ -409,90 +444,122 @@ __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
 // max) does, and no record needs its twin's position.  The input is sorted by
 // src, so the minima are a segmented minimum over runs: a run inside a chunk of
 // a.chunk consecutive units, which one wave takes, is stored; only the runs at
-// the chunk's ends take an atomic.  (Atomics at the ends of every unit took 95
-// of 230 us at 10^6 vertices, 3.2 10^7 records: neighbouring waves share lines.)
+// the chunk's ends take an atomic.  Those wait in LDS and leave together: the
+// next loads' wait includes an atomic's, some 5 us among streaming loads (at
+// 2^24 vertices, 5.4 10^8 records, 32 chunks per wave: 0.3 of 1.95 ms).
 __device__ __forceinline__ u64 dst_key(u32 w, u32 d) { return (u64(w) << 32) | d; }
+
+// A run's lightest record so far; equal weights: the first one, as dst ascends.
+// With `inside` the run began in this chunk, after its first record or with it.
+struct Run {
+  u32 s, w, d, inside;
+};
 
 // The run a chunk's next unit may continue (wave-uniform).
 struct Carry {
-  u32 s;
-  u64 v;
-  u32 inside;  // it began in this chunk, after the chunk's first record or with it
-  bool any;    // false at the chunk's first unit
+  Run run;
+  bool any;  // false at the chunk's first unit
 };
 
-// Minima of a unit; sources at or past n share word n.
+// A wave's offers of its chunks' first and last runs.
+struct Ends {
+  u32 s[WAVE];
+  u64 k[WAVE];
+};
+constexpr u32 ENDS_PER_UNIT = 4;  // at most: the carry, a lane's head, a lane's tail, the last tail
+
+// The lanes' runs that end (sources at or past n share word n; every lane calls).
+__device__ __forceinline__ void end_run(u64* best, u32 n, bool ends, const Run& r, Ends& pending,
+                                        u32& count) {
+  const u64 b = __ballot(ends && !r.inside);
+  if (ends) {
+    const u32 s = min(r.s, n);
+    const u64 k = dst_key(r.w, r.d);
+    if (r.inside) {
+      put(at(best, s), k);
+    } else {
+      pending.s[count + mbcnt(b)] = s;
+      pending.k[count + mbcnt(b)] = k;
+    }
+  }
+  count += static_cast<u32>(__popcll(b));
+}
+__device__ __forceinline__ void offer_ends_of_chunks(u64* best, const Ends& pending, u32& count) {
+  if (lane_id() < static_cast<int>(count)) lower(best, pending.s[lane_id()], pending.k[lane_id()]);
+  count = 0;
+}
+
+// Segmented minimum over the lanes, a step: an open lane (its run began before
+// it) takes over what the lane at the step's distance knows of the run.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ void scan_step(Run& r, u32& open) {
+  const u32 w = dpp<CTRL, ROWS>(r.w, r.w), d = dpp<CTRL, ROWS>(r.d, r.d);
+  const u32 in = dpp<CTRL, ROWS>(r.inside, r.inside), still = dpp<CTRL, ROWS>(open, open);
+  if (open) {
+    const bool first = w <= r.w;
+    r.w = first ? w : r.w;
+    r.d = first ? d : r.d;
+    r.inside = in;
+    open = still;
+  }
+}
+
+// Minima of a unit.
 __device__ __forceinline__ void run_minima(const Unit& x, bool first_unit, bool last_of_chunk,
-                                           u32 n, u64* best, Carry& c) {
-  const int lane = lane_id();
-  const u32 head_s = x.s[0];
-  u32 tail_s = head_s;
-  u64 tail_v = dst_key(x.w[0], x.d[0]);
-  u64 head_v = tail_v;
+                                           u32 n, u64* best, Carry& c, Ends& pending, u32& count) {
+  const u32 lane = lane_id();
+  Run tail{x.s[0], x.w[0], x.d[0], 1}, head = tail;
   bool multi = false;  // the lane's records hold more than one run
 #pragma unroll
   for (int e = 1; e < 4; ++e) {
-    const u64 k = dst_key(x.w[e], x.d[e]);
-    if (x.s[e] != tail_s) {
-      if (!multi) head_v = tail_v;
-      else put(best + min(tail_s, n), tail_v);  // a run inside the lane
+    if (x.s[e] != tail.s) {
+      if (!multi) head = tail;
+      else put(at(best, min(tail.s, n)), dst_key(tail.w, tail.d));  // a run inside the lane
       multi = true;
-      tail_s = x.s[e];
-      tail_v = k;
-    } else {
-      tail_v = k < tail_v ? k : tail_v;
+      tail = Run{x.s[e], x.w[e], x.d[e], 1};
+    } else if (x.w[e] < tail.w) {
+      tail.w = x.w[e];
+      tail.d = x.d[e];
     }
   }
   // the run before a lane's: the previous lane's last one, or the carry
-  u32 prev_s = __shfl_up(tail_s, 1, WAVE);
-  bool joins = prev_s == head_s;
-  u32 began = 1;  // the lane's head run began inside the chunk, if it joins none
+  bool joins = dpp<DPP_WAVE_SHR1>(0, tail.s) == x.s[0];
+  u32 began = 1;  // the lane's first run began inside the chunk, if it joins none
   if (lane == 0) {
-    joins = c.any && c.s == head_s;
-    began = c.any || first_unit || x.ps != head_s ? 1u : 0u;
-    if (c.any && !joins) {
-      if (c.inside) put(best + min(c.s, n), c.v);
-      else lower(best, min(c.s, n), c.v);
+    joins = c.any && c.run.s == x.s[0];
+    began = c.any || first_unit || x.ps != x.s[0] ? 1u : 0u;
+    if (joins && !multi && c.run.w <= tail.w) {
+      tail.w = c.run.w;
+      tail.d = c.run.d;
     }
-    if (joins && !multi) tail_v = c.v < tail_v ? c.v : tail_v;
+    if (!multi) tail.inside = joins ? c.run.inside : began;
   }
-  // whether the tail run began inside the chunk; lanes that continue a run
-  // learn it, with the run's minimum, from the lanes before
-  u32 inside = multi ? 1u : joins ? (lane == 0 ? c.inside : 0u) : began;
-  bool open = lane > 0 && joins && !multi;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    if (!__any(open)) break;
-    const u64 v = __shfl_up(static_cast<unsigned long long>(tail_v), o, WAVE);
-    const u32 in = __shfl_up(inside, o, WAVE);
-    const u32 still = __shfl_up(open ? 1u : 0u, o, WAVE);
-    if (open) {
-      tail_v = v < tail_v ? v : tail_v;
-      inside = in;
-      open = still != 0;
-    }
-  }
-  u64 prev_v = __shfl_up(static_cast<unsigned long long>(tail_v), 1, WAVE);
-  u32 prev_in = __shfl_up(inside, 1, WAVE);
-  const u32 next_s = __shfl_down(head_s, 1, WAVE);
-  if (lane == 0) {
-    prev_v = c.v;
-    prev_in = c.inside;
-  }
+  end_run(best, n, lane == 0 && c.any && !joins, c.run, pending, count);
+  u32 open = lane > 0 && joins && !multi ? 1u : 0u;
+  scan_step<DPP_ROW_SHR + 1>(tail, open);
+  scan_step<DPP_ROW_SHR + 2>(tail, open);
+  scan_step<DPP_ROW_SHR + 4>(tail, open);
+  scan_step<DPP_ROW_SHR + 8>(tail, open);
+  scan_step<DPP_ROW_BCAST15, 0xA>(tail, open);
+  scan_step<DPP_ROW_BCAST31, 0xC>(tail, open);
+  const u32 pw = dpp<DPP_WAVE_SHR1>(c.run.w, tail.w), pd = dpp<DPP_WAVE_SHR1>(c.run.d, tail.d);
+  const u32 pin = dpp<DPP_WAVE_SHR1>(c.run.inside, tail.inside);
+  const u32 next_s = dpp<DPP_WAVE_SHL1>(tail.s, x.s[0]);
   if (multi) {
-    if (joins && prev_v < head_v) head_v = prev_v;
-    if (joins ? prev_in : began) put(best + min(head_s, n), head_v);
-    else lower(best, min(head_s, n), head_v);
+    if (joins && pw <= head.w) {
+      head.w = pw;
+      head.d = pd;
+    }
+    head.inside = joins ? pin : began;
   }
-  if (lane < WAVE - 1 && next_s != tail_s) {
-    if (inside) put(best + min(tail_s, n), tail_v);
-    else lower(best, min(tail_s, n), tail_v);
-  }
-  if (last_of_chunk && lane == WAVE - 1) lower(best, min(tail_s, n), tail_v);
-  c.s = __builtin_amdgcn_readlane(tail_s, WAVE - 1);
-  c.v = (u64(static_cast<u32>(__builtin_amdgcn_readlane(static_cast<u32>(tail_v >> 32), WAVE - 1))) << 32) |
-        static_cast<u32>(__builtin_amdgcn_readlane(static_cast<u32>(tail_v), WAVE - 1));
-  c.inside = __builtin_amdgcn_readlane(inside, WAVE - 1);
+  end_run(best, n, multi, head, pending, count);
+  const u32 inside = tail.inside;
+  if (lane == WAVE - 1) tail.inside = 0;  // the next chunk may continue it
+  end_run(best, n, lane < WAVE - 1 ? next_s != tail.s : last_of_chunk, tail, pending, count);
+  c.run.s = __builtin_amdgcn_readlane(tail.s, WAVE - 1);
+  c.run.w = __builtin_amdgcn_readlane(tail.w, WAVE - 1);
+  c.run.d = __builtin_amdgcn_readlane(tail.d, WAVE - 1);
+  c.run.inside = __builtin_amdgcn_readlane(inside, WAVE - 1);
   c.any = !last_of_chunk;
 }
 
@@ -521,6 +588,7 @@ struct UnitWalk {
       : unit(wave * a.chunk), end(units), left_in_chunk(a.chunk), skip((waves - 1) * a.chunk),
         chunk(a.chunk) {}
   __device__ __forceinline__ bool valid() const { return unit < end; }
+  __device__ __forceinline__ bool first_of_chunk() const { return left_in_chunk == chunk; }
   __device__ __forceinline__ bool last_of_chunk() const {
     return left_in_chunk == 1 || unit + 1 == end;
   }
@@ -540,6 +608,7 @@ constexpr u32 STAGE = 2 * WAVE;
 struct Stage {
   u32 s[UNION_CLASSES * STAGE], d[UNION_CLASSES * STAGE];
   u64 v[UNION_CLASSES * STAGE];
+  Ends ends;
 };
 
 // The first min(n, 64) staged edges of a class to its list, the rest (fewer
@@ -563,47 +632,50 @@ __device__ __forceinline__ void drain(const UnionArgs& a, WaveLists& l, Stage& s
   }
 }
 
-__device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, UnitWalk at, Stage& st,
+__device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, UnitWalk walk, Stage& st,
                                            Found& out) {
   __shared__ Found s_found[UW];
   const int lane = lane_id();
   const u32 q0 = get(a.ctl + UC_PIVOT), q1 = get(a.ctl + UC_PIVOT + 1),
             q2 = get(a.ctl + UC_PIVOT + 2);
-  u32* span = reinterpret_cast<u32*>(a.span);
-  // wave-uniform: lanes that saw an error or a parallel record, forward count
-  u64 bad_id = 0, bad_order = 0, dup = 0;
-  u32 fwd = 0;
+  u32* const span = reinterpret_cast<u32*>(a.span);
+  u32 top = 0, loop = NONE32;  // the largest id, the smallest src ^ dst of the lane's records
+  u32 unordered = 0, dup = 0, fwd = 0;  // wave-uniform
   u64 hf = 0, hall = 0;  // hash sums of the forward and of all records
-  Carry carry{0, 0, 0, false};
+  Carry carry{{0, 0, 0, 0}, false};
+  Ends& ends = st.ends;
   u32 n0 = 0, n1 = 0, n2 = 0;  // staged edges of the classes
+  u32 n_ends = 0;
   Unit next;
-  if (at.valid()) load_unit<true>(next, a, at.unit);
-  while (at.valid()) {
-    const Unit x = next;
-    const u64 unit = at.unit;
-    const bool last = at.last_of_chunk();
-    at.next();
-    if (at.valid()) load_unit<true>(next, a, at.unit);
+  u32 last_s = 0, last_d = 0;  // of the unit before, in the same chunk
+  if (walk.valid()) load_unit(next, a, walk.unit, true);
+  while (walk.valid()) {
+    Unit x = next;
+    if (!walk.first_of_chunk()) {
+      x.ps = last_s;
+      x.pd = last_d;
+    }
+    last_s = __builtin_amdgcn_readlane(x.s[3], WAVE - 1);
+    last_d = __builtin_amdgcn_readlane(x.d[3], WAVE - 1);
+    const u64 unit = walk.unit;
+    const bool last = walk.last_of_chunk();
+    walk.next();
+    if (walk.valid()) load_unit(next, a, walk.unit, walk.first_of_chunk());
     const u64 r0 = unit * UNION_UNIT + 4 * lane;
     const bool full = (unit + 1) * UNION_UNIT <= a.m;
-    u32 ps = __shfl_up(x.s[3], 1, WAVE), pd = __shfl_up(x.d[3], 1, WAVE);
-    if (lane == 0) {
-      ps = x.ps;
-      pd = x.pd;
-    }
-    u64 listed[4];
+    u32 ps = dpp<DPP_WAVE_SHR1>(x.ps, x.s[3]), pd = dpp<DPP_WAVE_SHR1>(x.pd, x.d[3]);
+    u64 listed[4], descents = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const u32 s = x.s[e], d = x.d[e], w = x.w[e];
       const u64 in = full ? ~0ull : __ballot(r0 + e < a.m);
       const u32 lo = min(s, d), hi = max(s, d);
-      const u64 prev = (u64(ps) << 32) | pd, here = (u64(s) << 32) | d;
-      bad_id |= __ballot(hi >= a.n) | __ballot(lo == hi);
-      bad_order |= __ballot(prev > here);  // (copies past the end equal their predecessor)
-      dup |= __ballot(prev == here) & in;
+      top = max(top, hi);
+      loop = min(loop, s ^ d);
+      descents |= __ballot(((u64(ps) << 32) | pd) >= ((u64(s) << 32) | d)) & in;
       if (ps != s) {  // (the first record's predecessor is (0, 0): row 0 ends, or begins, at 0)
-        put(span + 2 * u64(min(ps, a.n)) + 1, static_cast<u32>(r0 + e));
-        put(span + 2 * u64(min(s, a.n)), static_cast<u32>(r0 + e));
+        put(at(span, 2 * min(ps, a.n) + 1), static_cast<u32>(r0 + e));
+        put(at(span, 2 * min(s, a.n)), static_cast<u32>(r0 + e));
       }
       ps = s;
       pd = d;
@@ -615,8 +687,21 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       hall += h;
       listed[e] = f & __ballot(w <= q2);
     }
-    if (r0 < a.m && r0 + 4 >= a.m) put(span + 2 * u64(min(x.s[3], a.n)) + 1, static_cast<u32>(a.m));
-    run_minima(x, unit == 0, last, a.n, a.best[0], carry);
+    if (r0 < a.m && r0 + 4 >= a.m) put(at(span, 2 * min(x.s[3], a.n) + 1), static_cast<u32>(a.m));
+    if (descents) {  // parallel records or disorder (or record 0 is (0, 0): a self-loop)
+      ps = dpp<DPP_WAVE_SHR1>(x.ps, x.s[3]);
+      pd = dpp<DPP_WAVE_SHR1>(x.pd, x.d[3]);
+      for (int e = 0; e < 4; ++e) {
+        const bool here = r0 + e < a.m;
+        const u64 prev = (u64(ps) << 32) | pd, now = (u64(x.s[e]) << 32) | x.d[e];
+        unordered |= __any(here && prev > now) ? 1u : 0u;
+        dup |= __any(here && prev == now) ? 1u : 0u;
+        ps = x.s[e];
+        pd = x.d[e];
+      }
+    }
+    if (n_ends > WAVE - ENDS_PER_UNIT) offer_ends_of_chunks(a.best[0], ends, n_ends);
+    run_minima(x, unit == 0, last, a.n, a.best[0], carry, ends, n_ends);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (!listed[e]) continue;
@@ -638,6 +723,7 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
       if (n2 >= WAVE) drain<2>(a, l, st, n2);
     }
   }
+  offer_ends_of_chunks(a.best[0], ends, n_ends);
   if (n0) drain<0>(a, l, st, n0);
   if (n1) drain<1>(a, l, st, n1);
   if (n2) drain<2>(a, l, st, n2);
@@ -645,11 +731,14 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
   for (int o = WAVE / 2; o > 0; o >>= 1) {
     hf += __shfl_xor(hf, o, WAVE);
     hall += __shfl_xor(hall, o, WAVE);
+    top = max(top, __shfl_xor(top, o, WAVE));
+    loop = min(loop, __shfl_xor(loop, o, WAVE));
   }
   if (lane == 0)
     s_found[wave_index()] = Found{hf, hall - hf, fwd,
-                               (bad_id ? u32(ERR_INVALID) : 0u) | (bad_order ? u32(ERR_UNSORTED) : 0u),
-                               dup ? 1u : 0u};
+                                  (top >= a.n || loop == 0 ? u32(ERR_INVALID) : 0u) |
+                                      (unordered ? u32(ERR_UNSORTED) : 0u),
+                                  dup};
   __syncthreads();
   if (threadIdx.x == 0) {
     Found f{0, 0, 0, 0, 0};
@@ -674,16 +763,42 @@ __device__ __forceinline__ void light_pass(const UnionArgs& a, WaveLists& l, Uni
 // inside it.
 // Neither changes in these passes: after an acquire at agent scope plain loads
 // are current, and the gathers of a source's records hit the L1.
+__device__ __forceinline__ u32 most_frequent(u32 x) {
+  u32 votes = 0;
+  for (int i = 0; i < WAVE; ++i) votes += __shfl(x, i, WAVE) == x ? 1u : 0u;
+  u32 most = votes;
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, WAVE));
+  return __shfl(x, __ffsll(static_cast<unsigned long long>(__ballot(votes == most))) - 1, WAVE);
+}
 __device__ __forceinline__ u32 pick_giant(const UnionArgs& a) {
   // (the roots do not change meanwhile: every workgroup picks the same)
   u32 x[1] = {static_cast<u32>((u64(lane_id()) * a.n) / WAVE)};
   find_roots<1>(a.parent, x, NONE32, 0, a.err);
-  u32 votes = 0;
-  for (int i = 0; i < WAVE; ++i) votes += __shfl(x[0], i, WAVE) == x[0] ? 1u : 0u;
-  u32 most = votes;
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, WAVE));
-  return __shfl(x[0], __ffsll(static_cast<unsigned long long>(__ballot(votes == most))) - 1, WAVE);
+  return most_frequent(x[0]);
+}
+// A graph of unconnected parts has a giant each, one wave per part picks it.
+// They are marked by a byte each, and their minima in both arrays are 0, which no
+// offer lowers and no edge's key equals but that of the lightest edge of all, a
+// true minimum of its ends.
+__device__ __forceinline__ void pick_giants(const UnionArgs& a, u64 wave, u64 waves, bool again) {
+  for (u64 p = wave; p < a.parts; p += waves) {
+    const u32 v0 = a.part_off[p], len = a.part_off[p + 1] - v0;
+    const bool lead = lane_id() == 0;
+    if (again && lead) {
+      const u32 old = get(a.part_giant + p);
+      if (old != NONE32) put(a.giants + old, u8{0});
+    }
+    u32 g = NONE32;
+    if (len) {
+      u32 x[1] = {v0 + static_cast<u32>((u64(lane_id()) * len) / WAVE)};
+      find_roots<1>(a.parent, x, NONE32, 0, a.err);
+      g = most_frequent(x[0]);
+    }
+    if (!lead) continue;
+    put(a.part_giant + p, g);
+    if (g != NONE32) put(a.giants + g, u8{1});
+  }
 }
 
 __device__ __forceinline__ void offer_ends(u64* best, u32 s, u32 d, u64 k, u32 giant) {
@@ -716,8 +831,10 @@ __device__ __forceinline__ void append_crossing(const UnionArgs& a, WaveLists& l
 // reaches what is still to be read).
 __device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32 cls, u64* best,
                                            u32 giant) {
-  const u32 *ls = a.s[cls & 1], *ld = a.d[cls & 1], listed = cls == 1 ? l.rest1 : l.rest2;
-  const u64* lv = a.v[cls & 1];
+  const bool second = cls == 1;
+  const u32 *ls = second ? a.s[1] : a.s[0], *ld = second ? a.d[1] : a.d[0];
+  const u64* lv = second ? a.v[1] : a.v[0];
+  const u32 listed = second ? l.rest1 : l.rest2;
   const u64 lo = l.base + l.cap - listed;
   for (u32 j0 = 0; j0 < listed; j0 += 4 * WAVE) {
     u32 x[8], s[4], d[4];
@@ -730,7 +847,7 @@ __device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32
       k[e] = lv[q];
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = a.parent[x[e]];
+    for (int e = 0; e < 8; ++e) x[e] = *at(a.parent, x[e]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const bool in = j0 + e * WAVE + lane_id() < listed;
@@ -744,21 +861,21 @@ __device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32
 // The rest of the input where the giant leaves many records outside, or rows
 // too long for one wave: the wave's own forward records above the pivot, two
 // units per step, every load of a kind in flight before the next kind's.
-__device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, UnitWalk at,
+__device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, UnitWalk walk,
                                             u64* best, u32 giant) {
   constexpr int U = 2;
   const u32 pivot = get(a.ctl + UC_PIVOT + UNION_CLASSES - 1);
-  while (at.valid()) {
+  while (walk.valid()) {
     Unit x[U];
     u64 r0[U];
     int have = 0;  // (wave-uniform)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       r0[u] = a.m;
-      if (at.valid()) {
-        r0[u] = at.unit * UNION_UNIT + 4 * lane_id();
-        load_unit<false>(x[u], a, at.unit);
-        at.next();
+      if (walk.valid()) {
+        r0[u] = walk.unit * UNION_UNIT + 4 * lane_id();
+        load_unit(x[u], a, walk.unit, false);
+        walk.next();
         have = u + 1;
       }
     }
@@ -791,8 +908,8 @@ __device__ __forceinline__ void cross_input(const UnionArgs& a, WaveLists& l, Un
     for (int k = 0; k < 4 * U; ++k) {
       s[k / 4][k % 4] = d[k / 4][k % 4] = 0;
       if ((live >> k) & 1) {
-        s[k / 4][k % 4] = a.parent[x[k / 4].s[k % 4]];
-        d[k / 4][k % 4] = a.parent[x[k / 4].d[k % 4]];
+        s[k / 4][k % 4] = *at(a.parent, x[k / 4].s[k % 4]);
+        d[k / 4][k % 4] = *at(a.parent, x[k / 4].d[k % 4]);
       }
     }
 #pragma unroll
@@ -838,7 +955,7 @@ __device__ __forceinline__ void cross_rows(const UnionArgs& a, WaveLists& l, u64
         const u64 sp = a.span[v0 + lane];
         begin = static_cast<u32>(sp);
         len = static_cast<u32>(sp >> 32) - begin;
-        root = a.parent[v0 + lane];
+        root = *at(a.parent, static_cast<u32>(v0) + lane);
       }
       const u32 upto = wave_inclusive_sum(len);
       const u32 total = __shfl(upto, WAVE - 1, WAVE);
@@ -871,9 +988,9 @@ __device__ __forceinline__ void cross_rows(const UnionArgs& a, WaveLists& l, u64
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          rd[e] = giant;
-          if (ok[e] && !inner[e] && s[e] < d[e]) rd[e] = a.parent[d[e]];
-          ok[e] = ok[e] && (inner[e] || s[e] < d[e]) && rd[e] != rs[e];
+          rd[e] = rs[e];
+          if (ok[e] && (inner[e] || s[e] < d[e])) rd[e] = *at(a.parent, d[e]);
+          ok[e] = rd[e] != rs[e];
         }
         // positions of the forward records
         u32 lo[4], hi[4];
@@ -927,8 +1044,8 @@ constexpr int UR = 4;  // rows of one edge per lane a wave loads before use
 // wave's roots that live on.
 __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int cur, bool first,
                                     bool copies, u32 giant) {
-  const u64* best = a.best[cur];
-  u64* next = a.best[cur ^ 1];
+  const u64* best = minima(a, cur);
+  u64* next = minima(a, cur ^ 1);
   u32 live = 0;
   for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
     u32 x[UR], y[UR];
@@ -942,8 +1059,8 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
     }
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
-      bx[u] = get(best + x[u]);
-      by[u] = get(best + y[u]);
+      bx[u] = get(at(best, x[u]));
+      by[u] = get(at(best, y[u]));
     }
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
@@ -961,12 +1078,12 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
         other = x[u];
       }
       if (copies) {
-        if (atomicCAS(a.parent + child, child, other) != child) continue;
+        if (atomicCAS(at(a.parent, child), child, other) != child) continue;
       } else {
-        put(a.parent + child, other);
+        put(at(a.parent, child), other);
       }
       if (mx && my) {
-        put(next + other, VAL_NONE);  // the root that lives on
+        put(at(next, other), VAL_NONE);  // the root that lives on
         ++live;
       }
       const u32 pos = static_cast<u32>(k[u]);
@@ -985,7 +1102,7 @@ constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
 
 __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
                                         OfferTable& t, u32 giant, u32 wave) {
-  u64* best = a.best[out];
+  u64* best = minima(a, out);
   const bool table = live <= TABLE_LIVE;
   // with few roots every wave meets the same ones: some waves' stores do
   const u32 thin = !table ? 0u : live > 1024 ? 3u : live > 128 ? 31u : 255u;
@@ -1041,6 +1158,15 @@ union Scratch {
   Rows rows[UW];
 };
 
+// The kernel's arguments, loaded anew: held over all phases they fill the
+// scalar registers, and what spills costs vector instructions in every loop.
+__device__ __forceinline__ UnionArgs arguments() {
+  typedef const UnionArgs __attribute__((address_space(4))) * Pointer;
+  Pointer p = (Pointer)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const UnionArgs*)p;
+}
+
 // Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
 __device__ __forceinline__ u64 block_total(u64 wave_value) {
   __shared__ u64 s_v[UW];
@@ -1053,11 +1179,12 @@ __device__ __forceinline__ u64 block_total(u64 wave_value) {
   return t;
 }
 
-__global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
+__global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   __shared__ Scratch s_x;
   __shared__ Found s_all;
   __shared__ u64 s_waves[UW], s_base;  // prefix sums over the waves
   __shared__ u32 s_giant;
+  UnionArgs a = arguments();
   if (!join_grid(a.joined)) return;
   Barrier bar{a.bar, 0, a.err};
   const u32 n = a.n;
@@ -1071,6 +1198,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
     put(a.parent + v, static_cast<u32>(v));
     put(a.best[0] + v, VAL_NONE);
     put(a.span + v, u64{0});
+    if (a.parts) put(a.giants + v, u8{0});
   }
   const u64 words = (a.m + 31) / 32;
   for (u64 i = gthread; i < words; i += threads) put(a.marks + i, 0u);
@@ -1078,6 +1206,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   if (!sync_grid(bar, 0, sum)) return;
 
   // light pass
+  a = arguments();
   const u64 units = (a.m + UNION_UNIT - 1) / UNION_UNIT;
   // a wave's range of the list buffers: as many edges as its chunks have
   // records (only the input's last chunk may be short)
@@ -1124,11 +1253,13 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
   if (all.bad || u64(all.fwd) * 2 != a.m || all.hash_fwd != all.hash_rev) return;
 
   // rounds of each class
+  a = arguments();
   const bool copies = all.dup != 0;
   u32 round = 0, giant = NONE32;
   int cur = 0;
   u64 live = n;  // roots, where this is known
   for (u32 phase = 0; phase < a.classes + (a.has_heavy ? 1 : 0); ++phase) {
+    a = arguments();
     const bool last = phase == a.classes;
     if (phase > 0) {
       // the minima are cleared for every root: one that took no part in the last
@@ -1136,9 +1267,14 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
       // cross_rows moves the lists' ranges to other waves: a line that one XCD's
       // L2 still holds dirty would be written back over what another wrote since
       if (last && wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      if (wave_index() == 0) s_giant = pick_giant(a);
-      __syncthreads();
-      giant = s_giant;
+      if (a.parts) {
+        pick_giants(a, wave, waves, phase > 1);
+        if (!sync_grid(bar, 0, sum)) return;
+      } else {
+        if (wave_index() == 0) s_giant = pick_giant(a);
+        __syncthreads();
+        giant = s_giant;
+      }
       u64 outside = 0;                    // the wave's records in rows outside it
       u32 roots = 0;
       for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
@@ -1150,12 +1286,18 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
-          const u64 b = __ballot(v < n && x[j] == giant);
+          const bool in = v < n && (a.parts ? get(at(a.giants, x[j])) != 0 : x[j] == giant);
+          const u64 b = __ballot(in);
           const bool root = v < n && x[j] == v;
-          if (root) put(a.best[cur] + v, VAL_NONE);
+          if (root && a.parts && in) {
+            put(minima(a, cur) + v, u64{0});
+            put(minima(a, cur ^ 1) + v, u64{0});
+          } else if (root) {
+            put(minima(a, cur) + v, VAL_NONE);
+          }
           roots += static_cast<u32>(__popcll(__ballot(root)));
           if (lane == 0 && v < n) put(a.bits + v / 64, b);
-          if (last && v < n && x[j] != giant) {
+          if (last && v < n && !in) {
             const u64 sp = get(a.span + v), len = (sp >> 32) - static_cast<u32>(sp);
             outside += len > ROW_LONG ? a.m : len;
           }
@@ -1180,10 +1322,11 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
 #pragma unroll
         for (int o = WAVE / 2; o > 0; o >>= 1) live += __shfl_xor(live, o, WAVE);
       }
+      a = arguments();
       if (!last) {
-        cross_list(a, l, phase, a.best[cur], giant);
+        cross_list(a, l, phase, minima(a, cur), giant);
       } else if (copies || sum * ROWS_SHARE > a.m) {
-        cross_input(a, l, UnitWalk(a, wave, waves, units), a.best[cur], giant);
+        cross_input(a, l, UnitWalk(a, wave, waves, units), minima(a, cur), giant);
       } else {
         // a wave's list holds as many edges as its rows have records
         if (wave_index() == 0) {
@@ -1196,9 +1339,10 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
         __syncthreads();
         l.base = s_base;
         for (u32 w = 0; w < wave_index(); ++w) l.base += s_waves[w];
-        cross_rows(a, l, wave, waves, a.best[cur], giant, s_x.rows[wave_index()]);
+        cross_rows(a, l, wave, waves, minima(a, cur), giant, s_x.rows[wave_index()]);
       }
     }
+    a = arguments();
     u64 edges;
     if (!sync_grid(bar, block_total(l.c), edges)) return;
     while (edges) {
@@ -1206,6 +1350,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
       const bool first = phase == 0 && round == 0;
       const u32 lw = hook(a, l, cur, first, first && copies, giant);
       if (!sync_grid(bar, block_total(lw), live)) return;
+      a = arguments();
       relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
       cur ^= 1;
       ++round;
@@ -1219,6 +1364,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) a.log[UNION_LOG + phase] = round;
   }
 
+  a = arguments();
   // output: workgroups own equal contiguous parts of the mark words, their
   // waves equal parts of those
   const u64 rows = (words + WAVE - 1) / WAVE;  // rows of 64 words
@@ -1337,9 +1483,10 @@ u32 union_blocks(u64 m, u32 cus) {
 
 u32 union_chunk(u64 m, u32 blocks) {
   // long chunks spare atomics at their ends, several chunks per wave even out
-  // how many edges the waves list
-  const u64 per_wave = (m + UNION_UNIT - 1) / UNION_UNIT / (u64(blocks) * UW);
-  return static_cast<u32>(std::max<u64>(1, std::min<u64>(per_wave / 4, UNION_CHUNK_MAX)));
+  // how many edges the waves list: at most four chunks up to 64 units per wave
+  const u64 waves = u64(blocks) * UW, units = (m + UNION_UNIT - 1) / UNION_UNIT;
+  return static_cast<u32>(
+      std::max<u64>(1, std::min<u64>((units + 4 * waves - 1) / (4 * waves), UNION_CHUNK_MAX)));
 }
 
 void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
