@@ -424,6 +424,8 @@ struct UnionArgs {
   u64* v[2] = {nullptr, nullptr};
   u64* best[2] = {nullptr, nullptr};  // n + 1 words each
   u32* parent = nullptr;
+  // the few-roots rounds: vertex -> dense id, dense id -> vertex and parent id
+  u32 *dense_id = nullptr, *dense_vertex = nullptr, *dense_parent = nullptr;
   u64* span = nullptr;   // per vertex, n + 1 words: its row's first position, its end << 32
   u64* bits = nullptr;   // one bit per vertex: it is in the giant component (of its part)
   // a graph of `parts` unconnected parts (0: not known to be one): part p holds

@@ -1049,6 +1049,9 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   a.best[0] = best_val;
   a.best[1] = state;
   a.parent = parent;
+  a.dense_id = seg_start;
+  a.dense_vertex = seg_end;
+  a.dense_parent = rep_next;
   a.span = pos;
   a.bits = reinterpret_cast<u64*>(label);
   if (part_count > 1) {

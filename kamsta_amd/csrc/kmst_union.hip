@@ -49,9 +49,9 @@
 // A large one is bound by random accesses, 8 to 16 bytes of 64 to 128 MB tables
 // for every listed edge and round, and by the light pass.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
-// records 117 / 192 us; 2^14, 4.9 10^5 238 / 549 us; 2^17, 2.1 10^6 361 / 1394
-// us; 10^6, 3.2 10^7 821 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
-// 7.5 / 10.4 ms (1.36 ms).
+// records 85 / 185 us; 2^14, 4.9 10^5 205 / 525 us; 2^17, 2.1 10^6 330 / 1394
+// us; 10^6, 3.2 10^7 740 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
+// 7.2 / 10.4 ms (1.36 ms).
 // Lists are private to a wave, so they need no coherence, counters or
 // workgroup barriers, and their compaction is in place (plain accesses: a wave's
 // range changes hands once, behind a release and an acquire).
@@ -1041,9 +1041,10 @@ constexpr int UR = 4;  // rows of one edge per lane a wave loads before use
 // With `first` the minima are the light pass's, (weight << 32) | the other
 // end; parallel copies of one weight then share a minimum, so with copies in
 // the input the hook claims its child and one of them is taken.  Returns the
-// wave's roots that live on.
+// wave's roots that live on, with `note` listed from the start of the wave's range
+// of the second buffer (the later class lies at its end: both fit).
 __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int cur, bool first,
-                                    bool copies, u32 giant) {
+                                    bool copies, u32 giant, u32* parent, bool note) {
   const u64* best = minima(a, cur);
   u64* next = minima(a, cur ^ 1);
   u32 live = 0;
@@ -1068,31 +1069,32 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
       // (the passive root's word is an old minimum)
       const bool mx = bx[u] == (first ? dst_key(w, y[u]) : k[u]) && x[u] != giant;
       const bool my = by[u] == (first ? dst_key(w, x[u]) : k[u]) && y[u] != giant;
-      if (j0 + u * WAVE + lane_id() >= l.c || (!mx && !my)) continue;
       u32 child = x[u], other = y[u];
-      if (mx && my) {
-        child = max(x[u], y[u]);
-        other = min(x[u], y[u]);
-      } else if (my) {
-        child = y[u];
-        other = x[u];
+      bool lives = false;
+      if (j0 + u * WAVE + lane_id() < l.c && (mx || my)) {
+        if (mx && my) {
+          child = max(x[u], y[u]);
+          other = min(x[u], y[u]);
+        } else if (my) {
+          child = y[u];
+          other = x[u];
+        }
+        bool hooked = true;
+        if (copies) hooked = atomicCAS(at(parent, child), child, other) == child;
+        else put(at(parent, child), other);
+        if (hooked) {
+          lives = mx && my;
+          if (lives) put(at(next, other), VAL_NONE);  // the root that lives on
+          const u32 pos = static_cast<u32>(k[u]);
+          (void)__hip_atomic_fetch_or(a.marks + (pos >> 5), 1u << (pos & 31), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
-      if (copies) {
-        if (atomicCAS(at(a.parent, child), child, other) != child) continue;
-      } else {
-        put(at(a.parent, child), other);
-      }
-      if (mx && my) {
-        put(at(next, other), VAL_NONE);  // the root that lives on
-        ++live;
-      }
-      const u32 pos = static_cast<u32>(k[u]);
-      (void)__hip_atomic_fetch_or(a.marks + (pos >> 5), 1u << (pos & 31), __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
+      const u64 b = __ballot(lives);
+      if (note && lives) a.s[1][l.base + live + mbcnt(b)] = other;
+      live += static_cast<u32>(__popcll(b));
     }
   }
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) live += __shfl_xor(live, o, WAVE);
   return live;
 }
 
@@ -1150,10 +1152,111 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
   }
 }
 
+// Few roots: with at most DENSE_MAX of them left in the first class's rounds,
+// the lists hold dense ids.  A round's hooks then lie over few words, which every
+// workgroup reads into its LDS and resolves there, where a step of a walk takes a
+// tenth of the time (the trees of a round are some ten hooks deep); and its
+// offers meet in LDS before they go to the shared minima.  A graph of at most
+// DENSE_MAX vertices begins this way, its ids being the vertices.
+// At 10^6 vertices, 2 10^5 edges left, rounds of 1500 roots and less relabel in 9
+// to 7 us, 40 to 9 as walks with a hashed table of minima; at 2^14, 3 10^4 edges, in 8
+// to 5 us, 18 to 7.  Entering takes two barriers more: not worth it with few
+// edges (geometric graphs, 13 us of 570 at 10^6 vertices), nor with more ids for every workgroup to
+// read (with 8192 a solve of 2^17 vertices takes 345 us, with 4096 330).
+constexpr u32 DENSE_MAX = 4096;
+constexpr u64 DENSE_EDGES = 16, DENSE_EDGES_MIN = 4096;  // edges per root, and in all, at least
+struct DenseRound {
+  u32 root[DENSE_MAX];
+  u64 best[DENSE_MAX];
+};
+// With `enter` the lists still hold vertices.
+__device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, int out, u32 ids,
+                                              bool enter, const u32* parent, DenseRound& t,
+                                              u32 wave) {
+  u64* best = minima(a, out);
+  for (u32 i = threadIdx.x; i < ids; i += UT) t.best[i] = VAL_NONE;
+  if (!enter) {
+    u32 p[DENSE_MAX / UT];  // all in flight together
+#pragma unroll
+    for (u32 j = 0; j < DENSE_MAX / UT; ++j)
+      if (j * UT < ids) p[j] = get(at(parent, min(j * UT + threadIdx.x, ids - 1)));
+#pragma unroll
+    for (u32 j = 0; j < DENSE_MAX / UT; ++j)
+      if (j * UT + threadIdx.x < ids) t.root[j * UT + threadIdx.x] = p[j];
+  }
+  __syncthreads();
+  if (!enter) {
+    for (u32 i = threadIdx.x; i < ids; i += UT) {
+      // (others shorten the walked paths meanwhile)
+      u32 r = t.root[i], steps = 0;
+      for (u32 p; (p = t.root[r]) != r && steps < DENSE_MAX; ++steps) r = p;
+      t.root[i] = r;
+    }
+    __syncthreads();
+  }
+  u32 kept = 0;
+  for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
+    u32 xy[2 * UR];
+    u64 k[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u64 i = l.base + min<u32>(j0 + u * WAVE + lane_id(), l.c - 1);
+      xy[u] = a.s[0][i];
+      xy[UR + u] = a.d[0][i];
+      k[u] = a.v[0][i];
+    }
+    if (enter) {
+      find_roots<2 * UR>(a.parent, xy, 31, wave, a.err);
+      u32 id[2 * UR];
+#pragma unroll
+      for (int u = 0; u < 2 * UR; ++u) id[u] = get(at(a.dense_id, xy[u]));
+#pragma unroll
+      for (int u = 0; u < 2 * UR; ++u) xy[u] = id[u];
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2 * UR; ++u) xy[u] = t.root[xy[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const u32 x = xy[u], y = xy[UR + u];
+      const bool keep = j0 + u * WAVE + lane_id() < l.c && x != y;
+      const u64 b = __ballot(keep);
+      if (keep) {
+        // in place: the rows up to here have been read
+        const u64 q = l.base + kept + mbcnt(b);
+        a.s[0][q] = x;
+        a.d[0][q] = y;
+        a.v[0][q] = k[u];
+        if (k[u] < t.best[x])
+          atomicMin(reinterpret_cast<unsigned long long*>(&t.best[x]),
+                    static_cast<unsigned long long>(k[u]));
+        if (k[u] < t.best[y])
+          atomicMin(reinterpret_cast<unsigned long long*>(&t.best[y]),
+                    static_cast<unsigned long long>(k[u]));
+      }
+      kept += static_cast<u32>(__popcll(b));
+    }
+  }
+  l.c = kept;
+  __syncthreads();
+  u64 k[DENSE_MAX / UT], b[DENSE_MAX / UT];
+#pragma unroll
+  for (u32 j = 0; j < DENSE_MAX / UT; ++j) {
+    const u32 i = j * UT + threadIdx.x;
+    k[j] = i < ids ? t.best[i] : VAL_NONE;
+    b[j] = 0;
+    if (k[j] != VAL_NONE) b[j] = get(at(best, i));
+  }
+#pragma unroll
+  for (u32 j = 0; j < DENSE_MAX / UT; ++j)
+    if (k[j] < b[j]) lower(best, j * UT + threadIdx.x, k[j]);
+}
+
 // ------------------------------------------------------------ the solve
 union Scratch {
   Stage stage[UW];
   OfferTable table;
+  DenseRound dense;
   u16 pos[UW][UNION_UNIT * 8];  // marked positions of a wave's 64 mark words
   Rows rows[UW];
 };
@@ -1177,6 +1280,22 @@ __device__ __forceinline__ u64 block_total(u64 wave_value) {
   if (threadIdx.x == 0)
     for (int w = 0; w < UW; ++w) t += s_v[w];
   return t;
+}
+
+// Sum over the waves before this one of what the workgroups put in their fourth
+// found word, a barrier ago, and this workgroup's waves in s_waves.
+__device__ __forceinline__ u64 waves_before(const UnionArgs& a, const u64* s_waves, u64& s_base) {
+  if (wave_index() == 0) {
+    u64 before = 0;
+    for (u32 b = lane_id(); b < blockIdx.x; b += WAVE) before += get(a.found + b * 4 + 3);
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
+    if (lane_id() == 0) s_base = before;
+  }
+  __syncthreads();
+  u64 sum = s_base;
+  for (u32 w = 0; w < wave_index(); ++w) sum += s_waves[w];
+  return sum;
 }
 
 __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
@@ -1329,29 +1448,53 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
         cross_input(a, l, UnitWalk(a, wave, waves, units), minima(a, cur), giant);
       } else {
         // a wave's list holds as many edges as its rows have records
-        if (wave_index() == 0) {
-          u64 before = 0;
-          for (u32 b = lane; b < blockIdx.x; b += WAVE) before += get(a.found + b * 4 + 3);
-#pragma unroll
-          for (int o = WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
-          if (lane == 0) s_base = before;
-        }
-        __syncthreads();
-        l.base = s_base;
-        for (u32 w = 0; w < wave_index(); ++w) l.base += s_waves[w];
+        l.base = waves_before(a, s_waves, s_base);
         cross_rows(a, l, wave, waves, minima(a, cur), giant, s_x.rows[wave_index()]);
       }
     }
     a = arguments();
     u64 edges;
     if (!sync_grid(bar, block_total(l.c), edges)) return;
+    // dense ids of the first class's rounds (0: none yet), and whether they are the vertices
+    u32 ids = phase == 0 && n <= DENSE_MAX ? n : 0;
+    const bool identity = ids != 0;
+    bool resolved = false;  // the last relabel resolved them in LDS
+    u64 known = n;  // bound of the roots
     while (edges) {
       if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges | (live << 32);
       const bool first = phase == 0 && round == 0;
-      const u32 lw = hook(a, l, cur, first, first && copies, giant);
-      if (!sync_grid(bar, block_total(lw), live)) return;
+      const bool note = phase == 0 && !ids && known <= 8 * DENSE_MAX;
+      const u32 lw = hook(a, l, cur, first, first && copies, giant,
+                          ids && !identity ? a.dense_parent : a.parent, note);
+      const u64 block_live = block_total(lw);
+      if (note) {
+        if (lane == 0) s_waves[wave_index()] = lw;
+        if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_live);
+      }
+      if (!sync_grid(bar, block_live, live)) return;
+      known = live;
+      const bool enter = note && live <= DENSE_MAX && edges >= DENSE_EDGES_MIN &&
+                         edges >= DENSE_EDGES * live;
+      if (enter) {
+        // the survivors' ids: their order over the waves
+        u64 id = waves_before(a, s_waves, s_base);
+        for (u32 i = lane; i < lw; i += WAVE) {
+          const u32 v = a.s[1][l.base + i], x = static_cast<u32>(id) + i;
+          put(at(a.dense_id, v), x);
+          put(a.dense_vertex + x, v);
+          put(a.dense_parent + x, x);
+          put(minima(a, cur ^ 1) + x, VAL_NONE);
+        }
+        ids = static_cast<u32>(live);
+        u64 none;
+        if (!sync_grid(bar, 0, none)) return;
+      }
       a = arguments();
-      relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
+      if (ids)
+        relabel_dense(a, l, cur ^ 1, ids, enter, identity ? a.parent : a.dense_parent, s_x.dense,
+                      static_cast<u32>(wave));
+      else relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
+      resolved = ids && !enter;
       cur ^= 1;
       ++round;
       if (!sync_grid(bar, block_total(l.c), edges)) return;
@@ -1362,6 +1505,17 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) a.log[UNION_LOG + phase] = round;
+    if (resolved) {
+      for (u64 i = gthread; i < ids; i += threads) {
+        const u32 r = s_x.dense.root[i];
+        if (r != i) {
+          if (identity) put(a.parent + i, r);
+          else put(at(a.parent, get(a.dense_vertex + i)), get(a.dense_vertex + r));
+        }
+      }
+      // (the identity's walks end at the same roots before and after)
+      if (!identity && !sync_grid(bar, 0, sum)) return;
+    }
   }
 
   a = arguments();
@@ -1381,16 +1535,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_count);
   u64 total;
   if (!sync_grid(bar, block_count, total)) return;
-  if (wave_id() == 0) {
-    u64 before = 0;
-    for (u32 b = lane; b < blockIdx.x; b += WAVE) before += get(a.found + b * 4 + 3);
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, WAVE);
-    if (lane == 0) s_base = before;
-  }
-  __syncthreads();
-  u64 at = s_base;
-  for (int w = 0; w < wave_id(); ++w) at += s_waves[w];
+  u64 at = waves_before(a, s_waves, s_base);
   u16* pos = s_x.pos[wave_index()];
   u64 weight = 0;
   for (u64 r = r0; r < r1; ++r) {
@@ -1481,8 +1626,11 @@ u32 union_samples(u64 m) {
 }
 
 u32 union_blocks(u64 m, u32 cus) {
-  // two units per wave at least: fewer workgroups make the barriers cheaper
-  const u64 want = (m + 2 * UW * UNION_UNIT - 1) / (2 * UW * UNION_UNIT);
+  // three units per wave at least: fewer workgroups make the barriers and the
+  // offers of few roots cheaper (2^17 vertices, 2.1 10^6 records: 350 us with 171
+  // workgroups, 359 with 256, 369 with 64; 2^14, 4.9 10^5: 205 with 41, 203 with
+  // 61, 232 with 16)
+  const u64 want = (m + 3 * UW * UNION_UNIT - 1) / (3 * UW * UNION_UNIT);
   return static_cast<u32>(std::max<u64>(1, std::min<u64>({want, cus, UNION_BLOCKS_MAX})));
 }
 

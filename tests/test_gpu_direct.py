@@ -48,6 +48,8 @@ def check(torch, ctx, s, d, w, n, pads=((0, 0, 0),), direct=True, algos=(k.BORUV
 @pytest.mark.parametrize("n,edges", [
     (16, 100), (17, 127), (17, 128), (17, 129), (64, 1000), (256, 4095), (256, 4096), (256, 4097),
     (300, 16 * 256), (1000, 8193), (4097, 65537), (65535, 1 << 17), (65536, (1 << 17) + 1),
+    # dense ids from the start up to 4096 vertices
+    (4095, 30000), (4096, 30000), (4097, 30000), (5000, 300000), (9000, 36001),
     (100003, (1 << 21) - 1), (100003, 1 << 21), (100003, (1 << 21) + 129)])
 def test_sizes_and_alignment(gpu, ctx, n, edges):
     s, d, w = k.gen_gnm_host(n, edges, 254, edges)
