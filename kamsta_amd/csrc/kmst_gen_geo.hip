@@ -45,6 +45,14 @@
 
 namespace kmst {
 
+// OMP_NUM_THREADS when set (the CPU share of the process), else the hardware's
+unsigned host_threads() {
+  const char* e = std::getenv("OMP_NUM_THREADS");
+  long t = e ? std::strtol(e, nullptr, 10) : 0;
+  if (t <= 0) t = static_cast<long>(std::thread::hardware_concurrency());
+  return static_cast<unsigned>(std::min<long>(std::max<long>(t, 1), 64));
+}
+
 // =================================================================== det
 // Elementary functions from the mathematics, deterministic across host and
 // device.  exp: Cody-Waite reduction by ln 2 (W. J. Cody and W. Waite,
@@ -182,15 +190,6 @@ __host__ __device__ inline double unit(u64 h) {  // [0, 1), exact
 __host__ __device__ inline u32 geo_weight(u64 wseed, u32 s, u32 d, u32 max_w) {
   const u32 a = s < d ? s : d, b = s < d ? d : s;
   return 1u + static_cast<u32>(mix64(wseed ^ ((u64(a) << 32) | b)) % max_w);
-}
-
-// host threads for the generators: OMP_NUM_THREADS when set (the CPU share
-// of the process), else the hardware's
-unsigned host_threads() {
-  const char* e = std::getenv("OMP_NUM_THREADS");
-  long t = e ? std::strtol(e, nullptr, 10) : 0;
-  if (t <= 0) t = static_cast<long>(std::thread::hardware_concurrency());
-  return static_cast<unsigned>(std::min<long>(std::max<long>(t, 1), 64));
 }
 
 // f(lo, hi, t) over T contiguous chunks of [0, n), chunk t by thread t

@@ -388,6 +388,8 @@ struct PersistArgs {
 u32 persistent_blocks_max(int device);
 u32 persistent_threads();
 u32 compute_units(int device);
+// Host threads for work on host data (kmst_gen_geo.hip).
+unsigned host_threads();
 void persistent_rounds(hipStream_t st, const PersistArgs& a, u32 blocks);
 
 // The direct solve (kmst_union.hip): a whole solve in one launch of resident

@@ -105,6 +105,19 @@ static_assert(PERSIST_CTL_WORDS + 2 * PERSIST_LOG_TOTAL <= HOST_STAGE_WORDS,
 constexpr u32 HOST_SEQ_WORD = HOST_SAMPLE_WORD + HOST_STAGE_WORDS;
 constexpr size_t HOST_COUNTER_BYTES = (HOST_SEQ_WORD + 64) * 4;
 
+// Pinned memory through which host records travel, in slots of one chunk of
+// records with an event each; at most HOST_THREADS_MAX * 2 slots of
+// STAGE_CHUNK_MAX records (24 MiB), kept for later calls.
+constexpr unsigned HOST_THREADS_MAX = 8;
+constexpr u64 STAGE_CHUNK_MIN = u64{1} << 14, STAGE_CHUNK_MAX = u64{1} << 17;
+struct HostStage {
+  u32* p = nullptr;
+  size_t bytes = 0;
+  std::vector<hipEvent_t> events;
+  void reserve(unsigned slots, u64 chunk);
+  void release();
+};
+
 }  // namespace kmst
 
 struct kmst_context {
@@ -142,6 +155,7 @@ struct kmst_context {
   kmst_tuning tuning{0, 1, kmst::SORT_WIDE_MIN, kmst::PERSIST_MAX_DEFAULT};  // launch shapes of later solves
   // host-API staging
   kmst::DevBuf in_s, in_d, in_w, out_s, out_d, out_w;
+  kmst::HostStage stage;
   // generator scratch
   kmst::DevBuf gen_a, gen_b, gen_c, gen_d;
   // autotuner result fingerprint (and the codec's error word)
