@@ -1365,10 +1365,15 @@ void download_records(kmst_context& C, const kmst_dev_mst& o, uint64_t k, kmst_w
   }
 }
 
+void check_ids(const kmst_wedge& r) {
+  if (r.src >= 0xFFFFFFFFull || r.dst >= 0xFFFFFFFFull)
+    throw kmst::Error(KMST_EINVAL, "vertex id >= 2^32-1");
+}
+
 kmst_status host_solve(const kmst_wedge* in, uint64_t m, const kmst_config* cfg,
                        int32_t algorithm, kmst_wedge* out, uint64_t* out_n,
                        uint64_t* total_weight) {
-  return guarded([&] {
+  auto solve = [&] {
     check_config(cfg);
     if ((!in && m) || !out_n || !total_weight) throw kmst::Error(KMST_EINVAL, "null argument");
     if (m >= (uint64_t{1} << 32) - 1) throw kmst::Error(KMST_EINVAL, "more than 2^32-2 records");
@@ -1401,7 +1406,7 @@ kmst_status host_solve(const kmst_wedge* in, uint64_t m, const kmst_config* cfg,
     }
     if (vmax >= 0xFFFFFFFFull) {
       KMST_HIP(hipStreamSynchronize(ctx->stream));
-      throw kmst::Error(KMST_EINVAL, "vertex id >= 2^32-1");
+      for (uint64_t i = 0; i < m; ++i) check_ids(in[i]);
     }
     const uint64_t n = m ? vmax + 1 : 0;
     const uint64_t cap = n ? n : 1;
@@ -1435,6 +1440,16 @@ kmst_status host_solve(const kmst_wedge* in, uint64_t m, const kmst_config* cfg,
     kmst_dev_edges e{ds, dd, dw, m, n};
     solve_device_impl(ctx, &e, &c, &o, out_n, total_weight);
     if (*out_n) download_records(*ctx, o, *out_n, out);
+  };
+  return guarded([&] {
+    try {
+      solve();
+    } catch (const kmst::Error& e) {
+      // a wide id is refused as one whatever failed before it was met (no GPU)
+      if ((e.status == KMST_EDEVICE || e.status == KMST_ENOMEM) && in)
+        for (uint64_t i = 0; i < m; ++i) check_ids(in[i]);
+      throw;
+    }
   });
 }
 
