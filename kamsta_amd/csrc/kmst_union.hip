@@ -829,8 +829,13 @@ __device__ __forceinline__ void append_crossing(const UnionArgs& a, WaveLists& l
 // A later light class: the wave's own list, from its low end up (the third
 // class's crossing edges go to the same range's front: what is appended never
 // reaches what is still to be read).
+// With `filter`, where most vertices are inside the giant, an edge's ends are
+// first looked up in its bitmap, which stays in the L2s where the parent array
+// does not.  At 2^24 vertices, 2.5 10^7 edges of the third class, 0.88 of the
+// vertices inside: 550 us without, 410 with the lookup; of the second class, half
+// of the vertices inside, 350 either way.
 __device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32 cls, u64* best,
-                                           u32 giant) {
+                                           u32 giant, bool filter) {
   const bool second = cls == 1;
   const u32 *ls = second ? a.s[1] : a.s[0], *ld = second ? a.d[1] : a.d[0];
   const u64* lv = second ? a.v[1] : a.v[0];
@@ -846,11 +851,23 @@ __device__ __forceinline__ void cross_list(const UnionArgs& a, WaveLists& l, u32
       x[4 + e] = ld[q];
       k[e] = lv[q];
     }
+    u32 skip = 0;  // bit e: both ends inside
+    if (filter) {
+      u32 b[8];
+      const u32* bits = reinterpret_cast<const u32*>(a.bits);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = *at(a.parent, x[e]);
+      for (int e = 0; e < 8; ++e) b[e] = *at(bits, x[e] >> 5);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        skip |= ((b[e] >> (x[e] & 31)) & (b[4 + e] >> (x[4 + e] & 31)) & 1u) << e;
+    }
+    if (__all(skip == 15)) continue;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (!((skip >> (e & 3)) & 1)) x[e] = *at(a.parent, x[e]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const bool in = j0 + e * WAVE + lane_id() < listed;
+      const bool in = j0 + e * WAVE + lane_id() < listed && !((skip >> e) & 1);
       s[e] = in ? x[e] : 0u;
       d[e] = in ? x[4 + e] : 0u;
     }
@@ -1394,7 +1411,8 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
         __syncthreads();
         giant = s_giant;
       }
-      u64 outside = 0;                    // the wave's records in rows outside it
+      // last: the wave's records in rows outside it; else its vertices inside
+      u64 count = 0;
       u32 roots = 0;
       for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
         u32 x[4];
@@ -1416,22 +1434,23 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
           }
           roots += static_cast<u32>(__popcll(__ballot(root)));
           if (lane == 0 && v < n) put(a.bits + v / 64, b);
+          if (!last && lane == 0) count += static_cast<u64>(__popcll(b));
           if (last && v < n && !in) {
             const u64 sp = get(a.span + v), len = (sp >> 32) - static_cast<u32>(sp);
-            outside += len > ROW_LONG ? a.m : len;
+            count += len > ROW_LONG ? a.m : len;
           }
         }
       }
 #pragma unroll
-      for (int o = WAVE / 2; o > 0; o >>= 1) outside += __shfl_xor(outside, o, WAVE);
-      if (lane == 0) s_waves[wave_index()] = outside;
-      outside = min(block_total(outside), a.m);
+      for (int o = WAVE / 2; o > 0; o >>= 1) count += __shfl_xor(count, o, WAVE);
+      if (lane == 0) s_waves[wave_index()] = count;
+      count = min(block_total(count), a.m);
       const u64 block_roots = block_total(roots);
       if (threadIdx.x == 0) {
         put(a.found + blockIdx.x * 4 + 2, block_roots);
-        put(a.found + blockIdx.x * 4 + 3, outside);
+        put(a.found + blockIdx.x * 4 + 3, count);
       }
-      if (!sync_grid(bar, outside, sum)) return;
+      if (!sync_grid(bar, count, sum)) return;
       // one wave acquires for the CU: the L1 is its workgroup's alone
       if (wave_index() == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       __syncthreads();
@@ -1443,7 +1462,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       }
       a = arguments();
       if (!last) {
-        cross_list(a, l, phase, minima(a, cur), giant);
+        cross_list(a, l, phase, minima(a, cur), giant, 6 * sum > 5 * u64(n));
       } else if (copies || sum * ROWS_SHARE > a.m) {
         cross_input(a, l, UnitWalk(a, wave, waves, units), minima(a, cur), giant);
       } else {
