@@ -411,6 +411,10 @@ enum : u32 {     // words of UnionArgs::ctl
   UC_RUNS = 5,   // sampled records that begin a run of one source
   UC_WORDS = 8
 };
+struct Publication {
+  u32* host = nullptr;
+  u32 extra_at = 0, seq_at = 0, seq = 0;
+};
 struct UnionArgs {
   const u32 *src = nullptr, *dst = nullptr, *wt = nullptr;  // the input: m records, ids < n
   u64 m = 0;
@@ -450,6 +454,13 @@ struct UnionArgs {
   u32 *out_s = nullptr, *out_d = nullptr, *out_w = nullptr;
   u64 out_cap = 0;
 };
+// Inputs of at most these sizes are solved by one workgroup in registers and LDS.
+constexpr u64 UNION_SMALL_RECORDS = u64{1} << 14;
+constexpr u64 UNION_SMALL_VERTICES = UNION_SMALL_RECORDS / 2;
+// That solve: no word has to be zero before, classes and list buffers are not
+// used, and the publication is complete in every case.
+void union_solve_small(hipStream_t st, const UnionArgs& a, u64* total, u32* groups,
+                       const Publication& p);
 u64 union_mark_words(u64 m);
 u32 union_samples(u64 m);
 u32 union_blocks(u64 m, u32 cus);
@@ -460,10 +471,6 @@ u32 union_chunk(u64 m, u32 blocks);
 // (*joined keeps another value than `blocks`), nothing is done: the caller
 // solves another way.
 // With p.host the 64 counter words at a.ctr and the log are published.
-struct Publication {
-  u32* host = nullptr;
-  u32 extra_at = 0, seq_at = 0, seq = 0;
-};
 void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
                  u32* ended, const Publication& p);
 

@@ -1013,9 +1013,9 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // launches and 7 to 34 read-backs; on a large one it moves each edge of the
 // lightest classes once a round and the others hardly at all, where the round
 // loop scatters, sorts and renumbers both records.  Measured, direct / round
-// loop: 110 / 179 us at 256 vertices, 238 / 549 at 2^14, 361 / 1394 at 2^17, 617
-// / 1736 and 821 / 2599 at 10^6 (16 and 32 records per vertex); 7.5 ms at 2^24
-// (32, random) against 10.4 filtering and 76 not, 5.0 / 8.0 geometric.  Sparse inputs (fewer than
+// loop: 46 / 179 us at 256 vertices, 205 / 540 at 2^14, 328 / 1394 at 2^17, 577
+// / 1736 and 742 / 2599 at 10^6 (16 and 32 records per vertex); 6.8 ms at 2^24
+// (32, random) against 10.4 filtering and 76 not, 4.8 / 8.0 geometric.  Sparse inputs (fewer than
 // two records per vertex: forests) stay with the round loop, and so does a
 // context whose persistent-round limit was set by hand.
 //
@@ -1041,7 +1041,8 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   // light records per vertex: the filter threshold, or more on dense inputs,
   // whose crossing heavy edges fall off exponentially with it
   const double target = std::max(double(std::max<u64>(filter_threshold, 2)), 2.0 + std::log(degree));
-  const bool heavy = target < 0.85 * degree;
+  const bool small = m0 <= UNION_SMALL_RECORDS && n0 <= UNION_SMALL_VERTICES;
+  const bool heavy = !small && target < 0.85 * degree;
   UnionArgs a;
   a.src = in_s;
   a.dst = in_d;
@@ -1100,14 +1101,18 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   a.out_d = out_d;
   a.out_w = out_w;
   a.out_cap = out_cap;
-  fill_u32(st, ctr, 64 + 2 * (UNION_LOG_TOTAL + UNION_BAR_WORDS), 0);
   Publication p;
   if (C.host_mapped) p = Publication{C.host_counters, HOST_SAMPLE_WORD, HOST_SEQ_WORD, ++C.publish_seq};
-  union_solve(st, a, blocks, reinterpret_cast<u64*>(ctr + C_TOTAL64), ctr + C_UGROUPS,
-              ctr + C_UENDED, p);
+  u64* const weight = reinterpret_cast<u64*>(ctr + C_TOTAL64);
+  if (small) {
+    union_solve_small(st, a, weight, ctr + C_UGROUPS, p);
+  } else {
+    fill_u32(st, ctr, 64 + 2 * (UNION_LOG_TOTAL + UNION_BAR_WORDS), 0);
+    union_solve(st, a, blocks, weight, ctr + C_UGROUPS, ctr + C_UENDED, p);
+  }
   if (p.host) await_published(p.seq);
   else fetch(reinterpret_cast<const u32*>(a.log), 2 * UNION_LOG_TOTAL);
-  if (blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
+  if (!small && blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
   check_input_words();
   if (!C.host_counters[C_UNION + UC_DONE]) throw Error(KMST_EDEVICE, "direct solve: not finished");
   const u64 cnt = C.host_counters[C_UCOUNT];

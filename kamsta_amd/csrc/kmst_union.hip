@@ -49,7 +49,7 @@
 // A large one is bound by random accesses, 8 to 16 bytes of 64 to 128 MB tables
 // for every listed edge and round, and by the light pass.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
-// records 85 / 185 us; 2^14, 4.9 10^5 205 / 525 us; 2^17, 2.1 10^6 330 / 1394
+// records 46 / 185 us (union_small_kernel); 2^14, 4.9 10^5 205 / 525 us; 2^17, 2.1 10^6 330 / 1394
 // us; 10^6, 3.2 10^7 740 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
 // 7.2 / 10.4 ms (1.36 ms).
 // Lists are private to a wave, so they need no coherence, counters or
@@ -1637,7 +1637,228 @@ __global__ __launch_bounds__(UT) void union_finish_kernel(UnionArgs a, u32 block
     __hip_atomic_store(p.host + p.seq_at, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// ------------------------------------------------------------ small inputs
+// One workgroup, one launch: the records stay in registers (record k * UT + t
+// with thread t), the parents, minima and marks in LDS, so a round is four
+// workgroup barriers and no memory round trip.  The general solve's phases cost
+// 3 us each for those: 256 vertices, 4.4 10^3 records take 84 us a call with it
+// (three launches) and 46 with this one (one launch, no counters to clear).
+// Every edge takes part from the first round on: a second class would cost more
+// rounds.  The limit is where the records fill the registers.
+constexpr int SMALL_SLOTS = static_cast<int>(UNION_SMALL_RECORDS) / UT;
+constexpr u32 SMALL_WORDS = static_cast<u32>(UNION_SMALL_RECORDS / 32);
+
+__global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total, u32* groups,
+                                                         Publication p) {
+  __shared__ u32 s_parent[UNION_SMALL_VERTICES];
+  __shared__ u64 s_best[UNION_SMALL_VERTICES];
+  __shared__ u32 s_marks[SMALL_WORDS], s_before[SMALL_WORDS];
+  __shared__ u64 s_fwd_hash, s_rev_hash, s_weight;
+  __shared__ u32 s_fwd, s_bad, s_live[3], s_count, s_groups;
+  __shared__ u64 s_log[UNION_LOG];
+  __shared__ u32 s_scan[UW];
+  const u32 t = threadIdx.x, lane = lane_id(), n = a.n, m = static_cast<u32>(a.m);
+  u32 s[SMALL_SLOTS], d[SMALL_SLOTS], w[SMALL_SLOTS];
+#pragma unroll
+  for (int k = 0; k < SMALL_SLOTS; ++k) {
+    s[k] = d[k] = w[k] = 0;
+    if (k * UT + t < m) {
+      s[k] = a.src[k * UT + t];
+      d[k] = a.dst[k * UT + t];
+      w[k] = a.wt[k * UT + t];
+    }
+  }
+  if (t == 0) {
+    s_fwd_hash = s_rev_hash = s_weight = 0;
+    s_fwd = s_bad = s_count = s_groups = 0;
+    s_live[0] = s_live[1] = s_live[2] = 0;
+  }
+  for (u32 v = t; v < n; v += UT) {
+    s_parent[v] = v;
+    s_best[v] = VAL_NONE;
+  }
+  for (u32 i = t; i < SMALL_WORDS; i += UT) s_marks[i] = 0;
+  __syncthreads();
+
+  // validation
+  u64 hf = 0, hr = 0;
+  u32 bad = 0, fwd = 0, alive = 0;  // alive, bit k: record k is a forward one and joins two roots
+#pragma unroll
+  for (int k = 0; k < SMALL_SLOTS; ++k) {
+    if (k * UT >= m) continue;
+    const u32 i = k * UT + t;
+    u32 ps = dpp<DPP_WAVE_SHR1>(0, s[k]), pd = dpp<DPP_WAVE_SHR1>(0, d[k]);
+    if (i < m) {
+      if (lane == 0 && i > 0) {
+        ps = a.src[i - 1];
+        pd = a.dst[i - 1];
+      }
+      const u32 lo = min(s[k], d[k]), hi = max(s[k], d[k]);
+      if (lo == hi || hi >= n) bad |= ERR_INVALID;
+      if (((u64(ps) << 32) | pd) > ((u64(s[k]) << 32) | d[k])) bad |= ERR_UNSORTED;
+      const u64 h = sym_hash(lo, hi, w[k]);
+      if (s[k] < d[k]) {
+        hf += h;
+        ++fwd;
+        alive |= 1u << k;
+      } else {
+        hr += h;
+      }
+    }
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) {
+    hf += __shfl_xor(hf, o, WAVE);
+    hr += __shfl_xor(hr, o, WAVE);
+    fwd += __shfl_xor(fwd, o, WAVE);
+    bad |= __shfl_xor(bad, o, WAVE);
+  }
+  if (lane == 0) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(&s_fwd_hash), static_cast<unsigned long long>(hf));
+    atomicAdd(reinterpret_cast<unsigned long long*>(&s_rev_hash), static_cast<unsigned long long>(hr));
+    atomicAdd(&s_fwd, fwd);
+    atomicOr(&s_bad, bad);
+  }
+  __syncthreads();
+  const bool good = !s_bad && 2 * s_fwd == m && s_fwd_hash == s_rev_hash;
+
+  // rounds: the roots an edge joins, x | y << 16
+  u32 ends[SMALL_SLOTS];
+#pragma unroll
+  for (int k = 0; k < SMALL_SLOTS; ++k) ends[k] = s[k] | (d[k] << 16);
+  u32 round = 0, live = good ? s_fwd : 0, roots = n;
+  while (live && round < UNION_ROUNDS_MAX) {
+    if (t == 0 && round < UNION_LOG) s_log[round] = live | (u64(roots) << 32);
+#pragma unroll
+    for (int k = 0; k < SMALL_SLOTS; ++k) {
+      if (!((alive >> k) & 1)) continue;
+      const u64 key = (u64(w[k]) << 32) | (k * UT + t);
+      const u32 x = ends[k] & 0xFFFF, y = ends[k] >> 16;
+      if (key < s_best[x])
+        atomicMin(reinterpret_cast<unsigned long long*>(&s_best[x]), static_cast<unsigned long long>(key));
+      if (key < s_best[y])
+        atomicMin(reinterpret_cast<unsigned long long*>(&s_best[y]), static_cast<unsigned long long>(key));
+    }
+    if (t == 0) s_live[(round + 1) % 3] = 0;
+    __syncthreads();
+    u32 mine = 0;  // edges that stay | roots that live on << 16
+#pragma unroll
+    for (int k = 0; k < SMALL_SLOTS; ++k) {
+      if (!((alive >> k) & 1)) continue;
+      const u32 i = k * UT + t, x = ends[k] & 0xFFFF, y = ends[k] >> 16;
+      const u64 key = (u64(w[k]) << 32) | i;
+      const bool mx = s_best[x] == key, my = s_best[y] == key;
+      if (!mx && !my) continue;
+      u32 child = mx ? x : y, other = mx ? y : x;
+      if (mx && my) {  // the lower end stays root
+        child = max(x, y);
+        other = min(x, y);
+        mine += 1u << 16;
+      }
+      s_parent[child] = other;
+      atomicOr(&s_marks[i / 32], 1u << (i & 31));
+    }
+    __syncthreads();
+    for (u32 v = t; v < n; v += UT) {
+      // (others shorten the walked paths meanwhile)
+      u32 r = s_parent[v], steps = 0;
+      for (u32 q; (q = s_parent[r]) != r && steps < UNION_SMALL_VERTICES; ++steps) r = q;
+      s_parent[v] = r;
+      s_best[v] = VAL_NONE;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SMALL_SLOTS; ++k) {
+      if (!((alive >> k) & 1)) continue;
+      const u32 x = s_parent[ends[k] & 0xFFFF], y = s_parent[ends[k] >> 16];
+      ends[k] = x | (y << 16);
+      if (x == y) alive &= ~(1u << k);
+      else ++mine;
+    }
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, WAVE);
+    if (lane == 0 && mine) atomicAdd(&s_live[round % 3], mine);
+    ++round;
+    __syncthreads();
+    live = s_live[(round - 1) % 3] & 0xFFFF;
+    roots = s_live[(round - 1) % 3] >> 16;
+  }
+  // output: the marked records in order; s_best counts the edges of a smaller endpoint
+  u32 *count = reinterpret_cast<u32*>(s_best);
+  for (u32 v = t; v < n; v += UT) count[v] = 0;
+  const u32 c = t < SMALL_WORDS ? static_cast<u32>(__popc(s_marks[t])) : 0u;
+  const u32 incl = wave_inclusive_sum(c);
+  if (lane == WAVE - 1) s_scan[wave_index()] = incl;
+  __syncthreads();
+  u32 before = incl - c;
+  for (u32 i = 0; i < wave_index(); ++i) before += s_scan[i];
+  if (t < SMALL_WORDS) s_before[t] = before;
+  if (t == SMALL_WORDS - 1) s_count = before + c;
+  __syncthreads();
+  u64 weight = 0;
+#pragma unroll
+  for (int k = 0; k < SMALL_SLOTS; ++k) {
+    const u32 i = k * UT + t;
+    if (i >= m || !((s_marks[i / 32] >> (i & 31)) & 1)) continue;
+    const u32 o = s_before[i / 32] + static_cast<u32>(__popc(s_marks[i / 32] & ((1u << (i & 31)) - 1)));
+    weight += w[k];
+    if (o < a.out_cap) {  // past the L2: the caller may go on before this launch has ended
+      put(a.out_s + o, s[k]);
+      put(a.out_d + o, d[k]);
+      put(a.out_w + o, w[k]);
+    }
+    if (atomicAdd(&count[s[k]], 1u) == MST_GROUP_SMALL) atomicAdd(&s_groups, 1u);
+  }
+#pragma unroll
+  for (int o = WAVE / 2; o > 0; o >>= 1) weight += __shfl_xor(weight, o, WAVE);
+  if (lane == 0 && weight)
+    atomicAdd(reinterpret_cast<unsigned long long*>(&s_weight), static_cast<unsigned long long>(weight));
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the output
+  __syncthreads();
+
+  // the counter words and the log, to the device's or the host's
+  u32* const ctr = p.host ? p.host : a.ctr;
+  u32* const lg = p.host ? p.host + p.extra_at : reinterpret_cast<u32*>(a.log);
+  auto word = [&](const void* at) { return static_cast<u32>(static_cast<const u32*>(at) - a.ctr); };
+  if (t < 64) {
+    u32 x = 0;
+    // (every round at least halves the components that have edges)
+    if (t == word(a.err)) x = s_bad | (live ? u32(ERR_SPIN) : 0u);
+    if (t == word(a.fwd_count)) x = s_fwd;
+    if (t == word(a.hsum)) x = static_cast<u32>(s_fwd_hash);
+    if (t == word(a.hsum) + 1) x = static_cast<u32>(s_fwd_hash >> 32);
+    if (t == word(a.hsum) + 2) x = static_cast<u32>(s_rev_hash);
+    if (t == word(a.hsum) + 3) x = static_cast<u32>(s_rev_hash >> 32);
+    if (t == word(total)) x = static_cast<u32>(s_weight);
+    if (t == word(total) + 1) x = static_cast<u32>(s_weight >> 32);
+    if (t == word(groups)) x = s_groups;
+    if (t == word(a.count)) x = s_count;
+    if (t == word(a.ctl) + UC_DONE) x = good && !live ? 1u : 0u;
+    if (t - word(a.ctl) - UC_PIVOT < UNION_CLASSES) x = NONE32;
+    ctr[t] = x;
+  }
+  for (u32 i = t; i < 2 * UNION_LOG_TOTAL; i += UT) {
+    const u32 r = i / 2;
+    const u64 x = r < min(round, UNION_LOG) ? s_log[r] : r == UNION_LOG ? u64{round} : 0;
+    lg[i] = static_cast<u32>(i & 1 ? x >> 32 : x);
+  }
+  if (!p.host) return;
+  __threadfence_system();
+  __syncthreads();
+  if (t == 0)
+    __hip_atomic_store(p.host + p.seq_at, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace
+
+void union_solve_small(hipStream_t st, const UnionArgs& a, u64* total, u32* groups,
+                       const Publication& p) {
+  if (a.m > UNION_SMALL_RECORDS || a.n > UNION_SMALL_VERTICES)
+    throw Error(KMST_EINVAL, "small direct solve: size");
+  KTScope t(st, K_PERSIST, 24.0 * a.m + 24.0 * a.n);
+  union_small_kernel<<<1, UT, 0, st>>>(a, total, groups, p);
+  KMST_HIP(hipGetLastError());
+}
 
 u64 union_mark_words(u64 m) { return (m + 31) / 32; }
 u32 union_samples(u64 m) {

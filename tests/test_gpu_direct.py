@@ -46,6 +46,9 @@ def check(torch, ctx, s, d, w, n, pads=((0, 0, 0),), direct=True, algos=(k.BORUV
 # undirected edges of a GNM graph on n vertices: half a unit, one unit, one
 # workgroup's first and last units, two workgroups, a chunk's first record
 @pytest.mark.parametrize("n,edges", [
+    # one workgroup in registers and LDS up to 2^14 records and 2^13 vertices
+    (3, 3), (40, 511), (40, 512), (40, 513), (200, 8191), (200, 8192), (200, 8193),
+    (8191, 8191), (8192, 8192), (8193, 8193),
     (16, 100), (17, 127), (17, 128), (17, 129), (64, 1000), (256, 4095), (256, 4096), (256, 4097),
     (300, 16 * 256), (1000, 8193), (4097, 65537), (65535, 1 << 17), (65536, (1 << 17) + 1),
     # dense ids from the start up to 4096 vertices
