@@ -1014,10 +1014,10 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // lightest classes once a round and the others hardly at all, where the round
 // loop scatters, sorts and renumbers both records.  Measured, direct / round
 // loop: 46 / 179 us at 256 vertices, 205 / 540 at 2^14, 328 / 1394 at 2^17, 577
-// / 1736 and 742 / 2599 at 10^6 (16 and 32 records per vertex); 6.8 ms at 2^24
-// (32, random) against 10.4 filtering and 76 not, 4.8 / 8.0 geometric.  Sparse inputs (fewer than
-// two records per vertex: forests) stay with the round loop, and so does a
-// context whose persistent-round limit was set by hand.
+// / 1736 and 728 / 2599 at 10^6 (16 and 32 records per vertex); 6.65 ms at 2^24
+// (32, random) against 10.4 filtering and 76 not, 4.55 / 8.0 geometric.  Sparse
+// inputs (fewer than two records per vertex: forests) stay with the round loop,
+// and so does a context whose persistent-round limit was set by hand.
 //
 // Light edges beyond what joins vertices stay in the lists round after round,
 // until their components meet: on a random graph 0.25 n of 1.1 n edges at

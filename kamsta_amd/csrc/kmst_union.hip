@@ -50,8 +50,8 @@
 // for every listed edge and round, and by the light pass.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
 // records 46 / 185 us (union_small_kernel); 2^14, 4.9 10^5 205 / 525 us; 2^17, 2.1 10^6 330 / 1394
-// us; 10^6, 3.2 10^7 740 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
-// 7.2 / 10.4 ms (1.36 ms).
+// us; 10^6, 3.2 10^7 728 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
+// 6.65 / 10.4 ms (1.36 ms).
 // Lists are private to a wave, so they need no coherence, counters or
 // workgroup barriers, and their compaction is in place (plain accesses: a wave's
 // range changes hands once, behind a release and an acquire).
@@ -1269,12 +1269,57 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
     if (k[j] < b[j]) lower(best, j * UT + threadIdx.x, k[j]);
 }
 
+// ------------------------------------------------------------ output
+// A wave's 64 mark words: 2048 input positions.
+constexpr u32 WINDOW = WAVE * 32;
+struct Window {
+  u16 pos[WINDOW];             // the marked positions
+  u32 bits[WAVE], before[WAVE];  // the mark words, the marks before each
+};
+// Sources of a window's marked records, from the rows of its vertices: the
+// gather of a third array would fetch nearly every line of it (an MST has one
+// record in 16 or 32).  A solve of 2^24 vertices 6.95 -> 6.65 ms, geometric 4.75
+// -> 4.55, of 10^6 745 -> 728 us.
+// False, with nothing written, where many vertices without records lie between.
+__device__ __forceinline__ bool window_sources(const UnionArgs& a, const Window& win, u64 base,
+                                               u32 v0, u32 v1, u64 at) {
+  if (v1 - v0 > 2 * WINDOW) return false;
+  auto rank = [&](u64 p) {  // marks of the window before position p
+    const u32 x = static_cast<u32>(p - base);
+    return win.before[x / 32] + static_cast<u32>(__popc(win.bits[x / 32] & ((1u << (x & 31)) - 1)));
+  };
+  for (u32 w = v0; w <= v1; w += WAVE) {
+    const u32 v = w + lane_id();
+    u32 first = 0, last = 0;
+    if (v <= v1) {
+      const u64 sp = get(a.span + v);
+      const u64 b = max(u64(static_cast<u32>(sp)), base);
+      const u64 e = min(sp >> 32, base + WINDOW);
+      if (b < e) {
+        first = rank(b);
+        last = rank(e - 1) + ((win.bits[(e - 1 - base) / 32] >> ((e - 1) & 31)) & 1u);
+      }
+    }
+    const bool many = last - first > 16;  // a hub: the wave writes it together
+    if (!many)
+      for (u32 k = first; k < last; ++k)
+        if (at + k < a.out_cap) a.out_s[at + k] = v;
+    for (u64 hubs = __ballot(many); hubs; hubs &= hubs - 1) {
+      const int i = __ffsll(static_cast<unsigned long long>(hubs)) - 1;
+      const u32 f = __shfl(first, i, WAVE), l = __shfl(last, i, WAVE), s = w + i;
+      for (u32 k = f + lane_id(); k < l; k += WAVE)
+        if (at + k < a.out_cap) a.out_s[at + k] = s;
+    }
+  }
+  return true;
+}
+
 // ------------------------------------------------------------ the solve
 union Scratch {
   Stage stage[UW];
   OfferTable table;
   DenseRound dense;
-  u16 pos[UW][UNION_UNIT * 8];  // marked positions of a wave's 64 mark words
+  Window window[UW];
   Rows rows[UW];
 };
 
@@ -1555,23 +1600,27 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   u64 total;
   if (!sync_grid(bar, block_count, total)) return;
   u64 at = waves_before(a, s_waves, s_base);
-  u16* pos = s_x.pos[wave_index()];
+  Window& win = s_x.window[wave_index()];
   u64 weight = 0;
   for (u64 r = r0; r < r1; ++r) {
-    const u64 w = r * WAVE + lane;
+    const u64 w = r * WAVE + lane, base = r * WINDOW;
     const u32 bits = w < words ? get(a.marks + w) : 0u;
+    const u32 v0 = a.src[base], v1 = a.src[min(base + WINDOW, a.m) - 1];
     const u32 c = static_cast<u32>(__popc(bits));
     const u32 incl = wave_inclusive_sum(c);
     const u32 row = __shfl(incl, WAVE - 1, WAVE);
     u32 p = incl - c;
-    for (u32 b = bits; b; b &= b - 1) pos[p++] = static_cast<u16>(lane * 32 + __ffs(b) - 1);
+    win.bits[lane] = bits;
+    win.before[lane] = p;
+    for (u32 b = bits; b; b &= b - 1) win.pos[p++] = static_cast<u16>(lane * 32 + __ffs(b) - 1);
     __builtin_amdgcn_wave_barrier();
+    const bool gather = row && !window_sources(a, win, base, v0, v1, at);
     for (u32 j = lane; j < row; j += WAVE) {
-      const u64 e = r * (WAVE * 32) + pos[j], o = at + j;
+      const u64 e = base + win.pos[j], o = at + j;
       const u32 wt = a.wt[e];
       weight += wt;
       if (o < a.out_cap) {
-        a.out_s[o] = a.src[e];
+        if (gather) a.out_s[o] = a.src[e];
         a.out_d[o] = a.dst[e];
         a.out_w[o] = wt;
       }

@@ -92,6 +92,10 @@ def shape(name):
         u = np.repeat(np.arange(4), n - 4)
         v = np.tile(np.arange(4, n), 4)
         return n, u, v, rng.integers(1, 255, len(u))
+    if name == "gap":  # 40000 ids without records inside a row of 2048 positions
+        u, v = np.triu_indices(300, 1)
+        far = lambda x: np.where(x < 150, x, x + 40000)
+        return 40150 + 150, far(u), far(v), rng.integers(1, 255, len(u))
     if name in ("outer hub", "outer rows"):  # a dense block, and beside it rows of 5000 / 40 records
         u, v = rng.integers(0, 9000, 200000), rng.integers(0, 9000, 200000)
         u, v = np.unique(np.stack([np.minimum(u, v), np.maximum(u, v)])[:, u != v], axis=1)
@@ -106,7 +110,7 @@ def shape(name):
 
 
 @pytest.mark.parametrize("name", ["pair", "triangle", "ring", "ladder", "parallel", "equal", "extremes",
-                                  "islands", "hubs", "outer hub", "outer rows"])
+                                  "islands", "hubs", "gap", "outer hub", "outer rows"])
 def test_shapes(gpu, ctx, name):
     n, u, v, w = shape(name)
     check(gpu, ctx, *symmetric(u, v, w), n)
