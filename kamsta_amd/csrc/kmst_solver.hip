@@ -1013,7 +1013,7 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // launches and 7 to 34 read-backs; on a large one it moves each edge of the
 // lightest classes once a round and the others hardly at all, where the round
 // loop scatters, sorts and renumbers both records.  Measured, direct / round
-// loop: 46 / 179 us at 256 vertices, 205 / 540 at 2^14, 328 / 1394 at 2^17, 577
+// loop: 46 / 179 us at 256 vertices, 205 / 540 at 2^14, 317 / 1394 at 2^17, 577
 // / 1736 and 728 / 2599 at 10^6 (16 and 32 records per vertex); 6.65 ms at 2^24
 // (32, random) against 10.4 filtering and 76 not, 4.55 / 8.0 geometric.  Sparse
 // inputs (fewer than two records per vertex: forests) stay with the round loop,
@@ -1021,12 +1021,14 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 //
 // Light edges beyond what joins vertices stay in the lists round after round,
 // until their components meet: on a random graph 0.25 n of 1.1 n edges at
-// degree 2.2, 0.03 n of 0.7 n at 1.4.  From 2^16 vertices the rounds' work
-// outweighs the barriers of a second light class (at 2^17, 340 us with it, 390
-// without), from DIRECT_FINE_VERTICES that of a third (at 2^24 7.5 ms with three, 9.0
-// with two; at 10^6 random 815 / 835 us, geometric 710 / 650).
+// degree 2.2, 0.03 n of 0.7 n at 1.4.  From DIRECT_MID_VERTICES on the rounds'
+// work outweighs the barriers of a second light class (16 records per vertex,
+// random / geometric, with one class and two: 270 / 257 and 301 / 294 us at 2^16,
+// 317 / 274 and 328 / 385 at 2^17, 413 / 331 and 394 / 373 at 2^18, 614 / 413 and 477
+// / 431 at 2^19), from DIRECT_FINE_VERTICES on that of a third (at 2^24 7.5 ms with
+// three, 9.0 with two; at 10^6 random 815 / 835 us, geometric 710 / 650).
 constexpr double DIRECT_FIRST_DEGREE = 2.2;
-constexpr u64 DIRECT_MID_VERTICES = u64{1} << 16;
+constexpr u64 DIRECT_MID_VERTICES = u64{1} << 18;
 constexpr double DIRECT_FINE_DEGREES[2] = {1.4, 2.4};
 constexpr u64 DIRECT_FINE_VERTICES = u64{1} << 21;
 bool Solver::use_direct() const {

@@ -117,11 +117,11 @@ def test_shapes(gpu, ctx, name):
 
 
 def test_rule(gpu, ctx):
-    """Fewer than two records per vertex: the round loop.  From 2^16 and from 2^21
+    """Fewer than two records per vertex: the round loop.  From 2^18 and from 2^21
     vertices on one and two more light classes."""
     i = np.arange(999)
     check(gpu, ctx, *symmetric(i, i + 1, i % 7 + 1), 1000, direct=False)
-    for n, phases in ((1 << 16) - 1, 2), (1 << 16, 3), ((1 << 21) - 1, 3), (1 << 21, 4):
+    for n, phases in ((1 << 18) - 1, 2), (1 << 18, 3), ((1 << 21) - 1, 3), (1 << 21, 4):
         s, d, w = k.gen_gnm_host(n, 4 * n, 254, n)
         check(gpu, ctx, s, d, w, n, algos=(k.BORUVKA,))
         assert len(ctx.stats()["filter"]) == phases, n
