@@ -397,7 +397,7 @@ void persistent_rounds(hipStream_t st, const PersistArgs& a, u32 blocks);
 constexpr int UNION_THREADS = 1024;
 constexpr u32 UNION_BLOCKS_MAX = 256;  // one per CU
 constexpr u64 UNION_UNIT = 256;        // records a wave takes per step
-constexpr u64 UNION_VERTICES_MAX = u64{1} << 28;
+constexpr u64 UNION_VERTICES_MAX = u64{1} << 28;  // byte offsets of 8-byte words fit 32 bits
 constexpr u32 UNION_CLASSES = 3;       // light weight classes at most
 constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
 constexpr u32 UNION_ROUNDS_MAX = 200;
