@@ -468,8 +468,8 @@ u32 union_chunk(u64 m, u32 blocks);
 // The solve, then the total weight into *total (written when the output is)
 // and the number of smaller endpoints with more than MST_GROUP_SMALL edges
 // into *groups (zero before).  Where the workgroups were not all resident
-// (*joined keeps another value than `blocks`), nothing is done: the caller
-// solves another way.
+// (*joined keeps another value than `blocks`), or hooks lie in a deep chain
+// (UC_DONE stays 0, no error), there is no output: the caller solves another way.
 // With p.host the 64 counter words at a.ctr and the log are published.
 void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
                  u32* ended, const Publication& p);

@@ -1037,7 +1037,7 @@ bool Solver::use_direct() const {
 }
 
 // False when the workgroups were not resident together (the GPU was shared
-// with other work): nothing was done, the round loop solves.
+// with other work) or a round hooked a deep chain: the round loop solves.
 bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n, u64* total) {
   const double degree = double(m0) / double(n0);
   // light records per vertex: the filter threshold, or more on dense inputs,
@@ -1116,7 +1116,7 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   else fetch(reinterpret_cast<const u32*>(a.log), 2 * UNION_LOG_TOTAL);
   if (!small && blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
   check_input_words();
-  if (!C.host_counters[C_UNION + UC_DONE]) throw Error(KMST_EDEVICE, "direct solve: not finished");
+  if (!C.host_counters[C_UNION + UC_DONE]) return false;  // a deep chain
   const u64 cnt = C.host_counters[C_UCOUNT];
   if (cnt > out_cap) throw Error(KMST_EINVAL, "output capacity too small");
   C.stats.packed_keys = false;

@@ -67,6 +67,14 @@ constexpr u64 WALL_TICKS_PER_MS = 100000;              // 100 MHz wall clock
 constexpr u64 BARRIER_TICKS = 10000 * WALL_TICKS_PER_MS;  // bound of a barrier's wait
 constexpr u64 JOIN_TICKS = 5 * WALL_TICKS_PER_MS;      // bound of the first one's
 constexpr u32 WALK_LIMIT = 1u << 26;                   // a longer walk is a corrupted forest
+// Weights in order along a path hook it into one chain, which walks of its
+// hundred thousands of list entries may not shorten for each other (10^6 vertices,
+// descending weights: 394 ms; the round loop 114).  A round that meets a walk this
+// long ends the solve, and the round loop takes over (116 ms in all); a ring of
+// 10^6 ascending weights stays below it (0.49 ms, 1.3 in the round loop), and
+// random weights far below.
+constexpr u32 WALK_DEEP = 1024;
+constexpr int DEEP_SHIFT = 35;  // in a relabel's payload, above the edges of all waves
 
 // wave index, in a scalar register: what follows from it (a wave's units, list
 // and counts) is then wave-uniform to the compiler too
@@ -259,9 +267,11 @@ __device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit,
 // longest of a wave's walks is several times the mean).  A walk stores nothing
 // but every eighth step (a load waits for the stores before it, a round trip to
 // memory per step; the stores that remain let walks over a long chain double),
-// and the root it found where (x's hash ^ salt) & thin is 0.
+// and the root it found where (x's hash ^ salt) & thin is 0.  False where a
+// walk takes more than `limit` steps.
 template <int N>
-__device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u32 salt, u32* err) {
+__device__ __forceinline__ bool find_roots(u32* parent, u32 (&x)[N], u32 thin, u32 salt,
+                                           u32 limit) {
   u32 p[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) p[j] = get(at(parent, x[j]));
@@ -285,10 +295,7 @@ __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u
         if ((step & 7) == 0) put(at(parent, x[j]), y[j]);
       }
     }
-    if (step > WALK_LIMIT) {
-      atomicOr(err, ERR_SPIN);
-      break;
-    }
+    if (step > limit) return false;
   }
 #pragma unroll
   for (int j = 0; j < N; ++j) {
@@ -296,6 +303,7 @@ __device__ __forceinline__ void find_roots(u32* parent, u32 (&x)[N], u32 thin, u
       put(at(parent, x[j]), p[j]);
     x[j] = p[j];
   }
+  return true;
 }
 
 // ------------------------------------------------------------ minima in LDS
@@ -774,7 +782,7 @@ __device__ __forceinline__ u32 most_frequent(u32 x) {
 __device__ __forceinline__ u32 pick_giant(const UnionArgs& a) {
   // (the roots do not change meanwhile: every workgroup picks the same)
   u32 x[1] = {static_cast<u32>((u64(lane_id()) * a.n) / WAVE)};
-  find_roots<1>(a.parent, x, NONE32, 0, a.err);
+  (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
   return most_frequent(x[0]);
 }
 // A graph of unconnected parts has a giant each, one wave per part picks it.
@@ -792,7 +800,7 @@ __device__ __forceinline__ void pick_giants(const UnionArgs& a, u64 wave, u64 wa
     u32 g = NONE32;
     if (len) {
       u32 x[1] = {v0 + static_cast<u32>((u64(lane_id()) * len) / WAVE)};
-      find_roots<1>(a.parent, x, NONE32, 0, a.err);
+      (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
       g = most_frequent(x[0]);
     }
     if (!lead) continue;
@@ -1120,7 +1128,7 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
 constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
 
 __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
-                                        OfferTable& t, u32 giant, u32 wave) {
+                                        OfferTable& t, u32 giant, u32 wave, bool& deep) {
   u64* best = minima(a, out);
   const bool table = live <= TABLE_LIVE;
   // with few roots every wave meets the same ones: some waves' stores do
@@ -1140,7 +1148,10 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
       xy[UR + u] = a.d[0][i];
       k[u] = a.v[0][i];
     }
-    find_roots<2 * UR>(a.parent, xy, thin, wave, a.err);
+    if (!find_roots<2 * UR>(a.parent, xy, thin, wave, WALK_DEEP)) {
+      deep = true;
+      break;
+    }
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
       const u32 x = xy[u], y = xy[UR + u];
@@ -1189,7 +1200,7 @@ struct DenseRound {
 // With `enter` the lists still hold vertices.
 __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, int out, u32 ids,
                                               bool enter, const u32* parent, DenseRound& t,
-                                              u32 wave) {
+                                              u32 wave, bool& deep) {
   u64* best = minima(a, out);
   for (u32 i = threadIdx.x; i < ids; i += UT) t.best[i] = VAL_NONE;
   if (!enter) {
@@ -1223,7 +1234,10 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
       k[u] = a.v[0][i];
     }
     if (enter) {
-      find_roots<2 * UR>(a.parent, xy, 31, wave, a.err);
+      if (!find_roots<2 * UR>(a.parent, xy, 31, wave, WALK_DEEP)) {
+        deep = true;
+        break;
+      }
       u32 id[2 * UR];
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) id[u] = get(at(a.dense_id, xy[u]));
@@ -1464,7 +1478,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           x[j] = static_cast<u32>(v0 + j * threads < n ? v0 + j * threads : v0);
-        find_roots<4>(a.parent, x, 0, 0, a.err);
+        if (!find_roots<4>(a.parent, x, 0, 0, WALK_LIMIT)) atomicOr(a.err, ERR_SPIN);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
@@ -1554,14 +1568,16 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
         if (!sync_grid(bar, 0, none)) return;
       }
       a = arguments();
+      bool deep = false;
       if (ids)
         relabel_dense(a, l, cur ^ 1, ids, enter, identity ? a.parent : a.dense_parent, s_x.dense,
-                      static_cast<u32>(wave));
-      else relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave));
+                      static_cast<u32>(wave), deep);
+      else relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave), deep);
       resolved = ids && !enter;
       cur ^= 1;
       ++round;
-      if (!sync_grid(bar, block_total(l.c), edges)) return;
+      if (!sync_grid(bar, block_total(l.c | (deep ? u64{1} << DEEP_SHIFT : 0)), edges)) return;
+      if (edges >> DEEP_SHIFT) return;
       if (round >= UNION_ROUNDS_MAX) {
         // every round at least halves the components that have edges
         if (gthread == 0) atomicOr(a.err, ERR_SPIN);
