@@ -25,10 +25,10 @@
 #include <memory>
 #include <mutex>
 #include <sstream>
-#include <thread>
 #include <vector>
 
 #include "kmst_kernels.hpp"
+#include "kmst_threads.hpp"
 #include "kmst_solver.hpp"
 
 namespace kmst {
@@ -1280,31 +1280,6 @@ void solve_device_impl(kmst_context* ctx, const kmst_dev_edges* in, const kmst_c
   kmst::g_ktimer = prev;
 }
 
-// f(t) on `threads` host threads, the caller's among them; the first failure
-// is thrown once all have ended.
-template <typename F>
-void on_threads(unsigned threads, F&& f) {
-  std::mutex mu;
-  std::exception_ptr failure;
-  auto run = [&](unsigned t) {
-    try {
-      f(t);
-    } catch (...) {
-      std::lock_guard<std::mutex> lk(mu);
-      if (!failure) failure = std::current_exception();
-    }
-  };
-  std::vector<std::thread> th;
-  try {
-    for (unsigned t = 1; t < threads; ++t) th.emplace_back(run, t);
-  } catch (const std::system_error&) {
-    // no more threads: those that run take all the work
-  }
-  run(0);
-  for (auto& x : th) x.join();
-  if (failure) std::rethrow_exception(failure);
-}
-
 unsigned stage_threads(uint64_t records) {
   return static_cast<unsigned>(std::max<uint64_t>(
       1, std::min<uint64_t>({kmst::host_threads(), kmst::HOST_THREADS_MAX,
@@ -1326,7 +1301,7 @@ uint64_t upload_records(kmst_context& C, const kmst_wedge* in, uint64_t m, uint3
   const uint64_t chunk = stage_chunk(m, threads), chunks = (m + chunk - 1) / chunk;
   C.stage.reserve(2 * threads, chunk);
   std::atomic<uint64_t> next{0}, largest{0};
-  on_threads(threads, [&](unsigned t) {
+  kmst::on_threads(threads, [&](unsigned t) {
     KMST_HIP(hipSetDevice(C.device));
     uint64_t top = 0, c;
     for (unsigned turn = 0; (c = next.fetch_add(1)) < chunks; ++turn) {
@@ -1364,10 +1339,8 @@ void download_records(kmst_context& C, const kmst_dev_mst& o, uint64_t k, kmst_w
     KMST_HIP(hipMemcpyAsync(d, o.dst + at, len * 4, hipMemcpyDeviceToHost, C.stream));
     KMST_HIP(hipMemcpyAsync(w, o.weight + at, len * 4, hipMemcpyDeviceToHost, C.stream));
     KMST_HIP(hipStreamSynchronize(C.stream));
-    const unsigned threads = stage_threads(len);
-    on_threads(threads, [&](unsigned t) {
-      for (uint64_t i = len * t / threads; i < len * (t + 1) / threads; ++i)
-        out[at + i] = kmst_wedge{s[i], d[i], w[i], 0};
+    kmst::for_blocks(stage_threads(len), len, kmst::STAGE_CHUNK_MIN, [&](uint64_t i0, uint64_t i1) {
+      for (uint64_t i = i0; i < i1; ++i) out[at + i] = kmst_wedge{s[i], d[i], w[i], 0};
     });
   }
 }
