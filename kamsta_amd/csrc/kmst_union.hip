@@ -1317,12 +1317,11 @@ __device__ __forceinline__ bool window_sources(const UnionArgs& a, const Window&
     const bool many = last - first > 16;  // a hub: the wave writes it together
     if (!many)
       for (u32 k = first; k < last; ++k)
-        if (at + k < a.out_cap) a.out_s[at + k] = v;
+        a.out_s[at + k] = v;
     for (u64 hubs = __ballot(many); hubs; hubs &= hubs - 1) {
       const int i = __ffsll(static_cast<unsigned long long>(hubs)) - 1;
       const u32 f = __shfl(first, i, WAVE), l = __shfl(last, i, WAVE), s = w + i;
-      for (u32 k = f + lane_id(); k < l; k += WAVE)
-        if (at + k < a.out_cap) a.out_s[at + k] = s;
+      for (u32 k = f + lane_id(); k < l; k += WAVE) a.out_s[at + k] = s;
     }
   }
   return true;
@@ -1615,6 +1614,13 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_count);
   u64 total;
   if (!sync_grid(bar, block_count, total)) return;
+  if (total > a.out_cap) {  // the host refuses the call: the caller's arrays stay as they are
+    if (gthread == 0) {
+      *a.count = static_cast<u32>(total);
+      a.ctl[UC_DONE] = 1;
+    }
+    return;
+  }
   u64 at = waves_before(a, s_waves, s_base);
   Window& win = s_x.window[wave_index()];
   u64 weight = 0;
@@ -1635,11 +1641,9 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       const u64 e = base + win.pos[j], o = at + j;
       const u32 wt = a.wt[e];
       weight += wt;
-      if (o < a.out_cap) {
-        if (gather) a.out_s[o] = a.src[e];
-        a.out_d[o] = a.dst[e];
-        a.out_w[o] = wt;
-      }
+      if (gather) a.out_s[o] = a.src[e];
+      a.out_d[o] = a.dst[e];
+      a.out_w[o] = wt;
     }
     __builtin_amdgcn_wave_barrier();
     at += row;
@@ -1666,7 +1670,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
 __global__ __launch_bounds__(UT) void union_finish_kernel(UnionArgs a, u32 blocks, u64* total,
                                                           u32* groups, u32* ended, Publication p) {
   __shared__ u32 s_last;
-  const u64 count = a.ctl[UC_DONE] ? min<u64>(*a.count, a.out_cap) : 0;
+  const u64 count = a.ctl[UC_DONE] && *a.count <= a.out_cap ? *a.count : 0;
   u32 c = 0;
 #pragma unroll 2
   for (u64 i = u64(blockIdx.x) * UT + threadIdx.x + MST_GROUP_SMALL; i < count;
@@ -1860,6 +1864,7 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
   if (t < SMALL_WORDS) s_before[t] = before;
   if (t == SMALL_WORDS - 1) s_count = before + c;
   __syncthreads();
+  const bool room = s_count <= a.out_cap;  // else the host refuses the call
   u64 weight = 0;
 #pragma unroll
   for (int k = 0; k < SMALL_SLOTS; ++k) {
@@ -1867,7 +1872,7 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
     if (i >= m || !((s_marks[i / 32] >> (i & 31)) & 1)) continue;
     const u32 o = s_before[i / 32] + static_cast<u32>(__popc(s_marks[i / 32] & ((1u << (i & 31)) - 1)));
     weight += w[k];
-    if (o < a.out_cap) {  // past the L2: the caller may go on before this launch has ended
+    if (room) {  // past the L2: the caller may go on before this launch has ended
       put(a.out_s + o, s[k]);
       put(a.out_d + o, d[k]);
       put(a.out_w + o, w[k]);
