@@ -56,6 +56,7 @@
 // workgroup barriers, and their compaction is in place (plain accesses: a wave's
 // range changes hands once, behind a release and an acquire).
 #include "kmst_kernels.hpp"
+#include "kmst_rows.hpp"
 
 namespace kmst {
 
@@ -1026,8 +1027,8 @@ __device__ __forceinline__ void cross_rows(const UnionArgs& a, WaveLists& l, u64
           hi[e] = p[e];
           if (ok[e] && s[e] > d[e]) {
             const u64 sp = a.span[d[e]];
-            lo[e] = static_cast<u32>(sp);
-            hi[e] = static_cast<u32>(sp >> 32) - 1;
+            lo[e] = row_first(sp);
+            hi[e] = row_last(sp);
           }
         }
         do {
@@ -1242,7 +1243,7 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) id[u] = get(at(a.dense_id, xy[u]));
 #pragma unroll
-      for (int u = 0; u < 2 * UR; ++u) xy[u] = id[u];
+      for (int u = 0; u < 2 * UR; ++u) xy[u] = min(id[u], ids - 1);  // (a root without an id: none, if symmetric)
     } else {
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) xy[u] = t.root[xy[u]];
