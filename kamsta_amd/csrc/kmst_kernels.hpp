@@ -402,6 +402,7 @@ constexpr u32 UNION_CLASSES = 3;       // light weight classes at most
 constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
 constexpr u32 UNION_ROUNDS_MAX = 200;
 constexpr u32 UNION_LOG = 60;          // u64 words: rounds (edges, roots << 32), ...
+constexpr u32 UNION_CHAINS = 0x80000000u;  // above the edges (2^31 - 1 at most): shorten_chains ran
 constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 4 phases
 constexpr u32 UNION_BAR_WORDS = 12 * 16;  // u64 words of the grid barrier
 enum : u32 {     // words of UnionArgs::ctl
@@ -468,8 +469,8 @@ u32 union_chunk(u64 m, u32 blocks);
 // The solve, then the total weight into *total (written when the output is)
 // and the number of smaller endpoints with more than MST_GROUP_SMALL edges
 // into *groups (zero before).  Where the workgroups were not all resident
-// (*joined keeps another value than `blocks`), or hooks lie in a deep chain
-// (UC_DONE stays 0, no error), there is no output: the caller solves another way.
+// (*joined keeps another value than `blocks`), there is no output: the caller
+// solves another way.
 // With p.host the 64 counter words at a.ctr and the log are published.
 void union_solve(hipStream_t st, const UnionArgs& a, u32 blocks, u64* total, u32* groups,
                  u32* ended, const Publication& p);

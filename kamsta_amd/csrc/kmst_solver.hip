@@ -1037,7 +1037,7 @@ bool Solver::use_direct() const {
 }
 
 // False when the workgroups were not resident together (the GPU was shared
-// with other work) or a round hooked a deep chain: the round loop solves.
+// with other work): the round loop solves.
 bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n, u64* total) {
   const double degree = double(m0) / double(n0);
   // light records per vertex: the filter threshold, or more on dense inputs,
@@ -1116,7 +1116,7 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   else fetch(reinterpret_cast<const u32*>(a.log), 2 * UNION_LOG_TOTAL);
   if (!small && blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
   check_input_words();
-  if (!C.host_counters[C_UNION + UC_DONE]) return false;  // a deep chain
+  if (!C.host_counters[C_UNION + UC_DONE]) throw Error(KMST_EDEVICE, "direct solve: not finished");
   const u64 cnt = C.host_counters[C_UCOUNT];
   if (cnt > out_cap) throw Error(KMST_EINVAL, "output capacity too small");
   C.stats.packed_keys = false;
@@ -1125,22 +1125,24 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
   std::memcpy(lg, C.host_counters + HOST_SAMPLE_WORD, sizeof(lg));
   const u32* ctl = C.host_counters + C_UNION;
   const u32 logged = static_cast<u32>(std::min<u64>(lg[UNION_LOG + phases - 1], UNION_LOG));
+  auto edges = [&](u64 i) { return lg[i] & (UNION_CHAINS - 1); };
   for (u32 i = 0; i < logged; ++i) {
     RoundStat rs;
     rs.n = lg[i] >> 32;
-    rs.m = 2 * (lg[i] & 0xFFFFFFFFull);
+    rs.m = 2 * edges(i);
     if (i + 1 < logged) {
       rs.n_next = lg[i + 1] >> 32;
-      rs.m_next = 2 * (lg[i + 1] & 0xFFFFFFFFull);
+      rs.m_next = 2 * edges(i + 1);
     }
     if (i == 0) rs.run_starts = ctl[UC_RUNS];
     rs.twins = i == 0 && n0 > TWINS_MIN_N && 2 * ctl[UC_FAR] > a.samples;
-    rs.direct = true;
+    rs.chains = lg[i] & UNION_CHAINS;
+    rs.direct = !rs.chains;
     C.stats.rounds.push_back(rs);
   }
   for (u32 p = 0; p < phases; ++p) {
     const u64 at = p ? lg[UNION_LOG + p - 1] : 0;  // the phase's first round
-    const u64 m = at < UNION_LOG && at < lg[UNION_LOG + p] ? 2 * (lg[at] & 0xFFFFFFFFull) : 0;
+    const u64 m = at < UNION_LOG && at < lg[UNION_LOG + p] ? 2 * edges(at) : 0;
     C.stats.filter.push_back(FilterStat{0, m0, p ? 0 : m, ctl[UC_PIVOT + std::min(p, UNION_CLASSES - 1)],
                                         p == 0, p ? m : 0, false});
   }
@@ -1768,7 +1770,8 @@ size_t kmst_context_stats_json(const kmst_context* ctx, char* buf, size_t cap) {
       << ",\"far_starts\":" << r.far_starts
       << ",\"persistent\":" << (r.persistent ? "true" : "false")
       << ",\"twins\":" << (r.twins ? "true" : "false")
-      << ",\"direct\":" << (r.direct ? "true" : "false");
+      << ",\"direct\":" << (r.direct ? "true" : "false")
+      << ",\"chains\":" << (r.chains ? "true" : "false");
     if (r.persistent)
       o << ",\"phase_us\":[" << r.phase_us[0] << "," << r.phase_us[1] << "," << r.phase_us[2]
         << "," << r.phase_us[3] << "]";

@@ -39,7 +39,9 @@ struct RoundStat {
   // took the src < dst half of records with far-apart ids (round loop:
   // relabelled it and wrote both directions)
   bool twins = false;
-  bool direct = false;      // a round of the direct solve (run_starts: sampled input records)
+  // a round of the direct solve (run_starts: sampled input records) whose roots
+  // were found by walks from the list's entries, or by passes over all vertices
+  bool direct = false, chains = false;
   double phase_us[4] = {0, 0, 0, 0};  // persistent: bind, hook, jump, relabel
 };
 struct FilterStat {

@@ -68,13 +68,18 @@ constexpr u64 WALL_TICKS_PER_MS = 100000;              // 100 MHz wall clock
 constexpr u64 BARRIER_TICKS = 10000 * WALL_TICKS_PER_MS;  // bound of a barrier's wait
 constexpr u64 JOIN_TICKS = 5 * WALL_TICKS_PER_MS;      // bound of the first one's
 constexpr u32 WALK_LIMIT = 1u << 26;                   // a longer walk is a corrupted forest
-// Weights in order along a path hook it into one chain, which walks of its
-// hundred thousands of list entries may not shorten for each other (10^6 vertices,
-// descending weights: 394 ms; the round loop 114).  A round that meets a walk this
-// long ends the solve, and the round loop takes over (116 ms in all); a ring of
-// 10^6 ascending weights stays below it (0.49 ms, 1.3 in the round loop), and
-// random weights far below.
-constexpr u32 WALK_DEEP = 1024;
+// Weights in order along a path hook it into one chain, which walks of the list's
+// entries may not shorten for each other.  A walk longer than this stops, and
+// shorten_chains takes all vertices to their roots before the round goes on.  A
+// step takes some 0.9 us, the passes 15 us up to 10^5 vertices and a time that
+// grows with n past that, hence the limit.  10^6 vertices, descending weights along a path,
+// heavier chords: 0.44 ms, 116 where the round loop took over after 1024 steps
+// (114 alone); 9000 vertices of a band 160 us, 1265 (205); a grid of 300 x 300
+// 166 us, 313 with walks alone (250).  Random weights stay below
+// (of 162 graphs of 8200 to 200000 vertices one met a limit of 8, none one of 10).
+constexpr u32 WALK_DEEP_MIN = 10;
+constexpr int WALK_DEEP_SHIFT = 15;
+__device__ __forceinline__ u32 walk_deep(u32 n) { return WALK_DEEP_MIN + (n >> WALK_DEEP_SHIFT); }
 constexpr int DEEP_SHIFT = 35;  // in a relabel's payload, above the edges of all waves
 
 // wave index, in a scalar register: what follows from it (a wave's units, list
@@ -196,6 +201,18 @@ __device__ __forceinline__ bool sync_grid(Barrier& bar, u64 payload, u64& sum) {
   return s_ok != 0;
 }
 
+// Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
+__device__ __forceinline__ u64 block_total(u64 wave_value) {
+  __shared__ u64 s_v[UW];
+  __syncthreads();  // thread 0 may still be adding the call before
+  if (lane_id() == 0) s_v[wave_index()] = wave_value;
+  __syncthreads();
+  u64 t = 0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < UW; ++w) t += s_v[w];
+  return t;
+}
+
 __device__ __forceinline__ bool join_grid(u32* joined) {
   __shared__ u32 s_join;
   if (threadIdx.x == 0) {
@@ -270,7 +287,7 @@ __device__ __forceinline__ void load_unit(Unit& x, const UnionArgs& a, u64 unit,
 // memory per step; the stores that remain let walks over a long chain double),
 // and the root it found where (x's hash ^ salt) & thin is 0.  False where a
 // walk takes more than `limit` steps.
-template <int N>
+template <int N, int STORE = 8>
 __device__ __forceinline__ bool find_roots(u32* parent, u32 (&x)[N], u32 thin, u32 salt,
                                            u32 limit) {
   u32 p[N];
@@ -293,7 +310,7 @@ __device__ __forceinline__ bool find_roots(u32* parent, u32 (&x)[N], u32 thin, u
       } else {
         moved |= 1u << j;
         p[j] = y[j];
-        if ((step & 7) == 0) put(at(parent, x[j]), y[j]);
+        if (step % STORE == 0) put(at(parent, x[j]), y[j]);
       }
     }
     if (step > limit) return false;
@@ -1128,8 +1145,36 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
 // more, most offers of a workgroup are to distinct roots.
 constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
 
-__device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
-                                        OfferTable& t, u32 giant, u32 wave, bool& deep) {
+// Every vertex onto its root, 24 steps of all walks at a time: where all
+// vertices of a chain walk together and store every third step, a chain's length
+// falls to a quarter in three steps.  More vertices than threads take walk in
+// turn, hence the passes.
+constexpr u32 SHORTEN_STEPS = 24;
+constexpr u32 SHORTEN_PASSES = 32;  // 25^32: more is a corrupted forest
+__device__ __forceinline__ bool shorten_chains(const UnionArgs& a, Barrier& bar, u32 gthread,
+                                               u32 threads) {
+  for (u32 pass = 0; pass < SHORTEN_PASSES; ++pass) {
+    bool open = false;
+    for (u64 v0 = gthread; v0 < a.n; v0 += 4 * threads) {
+      u32 x[4];
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j)
+        x[j] = static_cast<u32>(v0 + j * threads < a.n ? v0 + j * threads : v0);
+      if (!find_roots<4, 3>(a.parent, x, 0, 0, SHORTEN_STEPS)) open = true;
+    }
+    u64 sum;
+    if (!sync_grid(bar, block_total(__any(open) ? 1 : 0), sum)) return false;
+    if (!sum) return true;
+  }
+  if (gthread == 0) atomicOr(a.err, ERR_SPIN);
+  return false;
+}
+
+// True where the wave met a deep chain: its edges from there on are kept as they
+// were.  After shorten_chains the same call finishes the round (what it offered
+// before, it offers again).
+__device__ __forceinline__ bool relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
+                                        OfferTable& t, u32 giant, u32 wave) {
   u64* best = minima(a, out);
   const bool table = live <= TABLE_LIVE;
   // with few roots every wave meets the same ones: some waves' stores do
@@ -1139,6 +1184,7 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
     __syncthreads();
   }
   u32 kept = 0;
+  bool deep = false;
   for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
     u32 xy[2 * UR];
     u64 k[UR];
@@ -1149,10 +1195,7 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
       xy[UR + u] = a.d[0][i];
       k[u] = a.v[0][i];
     }
-    if (!find_roots<2 * UR>(a.parent, xy, thin, wave, WALK_DEEP)) {
-      deep = true;
-      break;
-    }
+    deep = deep || !find_roots<2 * UR>(a.parent, xy, thin, wave, walk_deep(a.n));
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
       const u32 x = xy[u], y = xy[UR + u];
@@ -1164,7 +1207,8 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
         a.s[0][q] = x;
         a.d[0][q] = y;
         a.v[0][q] = k[u];
-        if (table) {
+        if (deep) {
+        } else if (table) {
           if (x != giant) table_offer(t, best, x, k[u]);
           if (y != giant) table_offer(t, best, y, k[u]);
         } else {
@@ -1179,6 +1223,7 @@ __device__ __forceinline__ void relabel(const UnionArgs& a, WaveLists& l, int ou
     __syncthreads();
     table_flush(t, best);
   }
+  return deep;
 }
 
 // Few roots: with at most DENSE_MAX of them left in the first class's rounds,
@@ -1198,10 +1243,13 @@ struct DenseRound {
   u32 root[DENSE_MAX];
   u64 best[DENSE_MAX];
 };
-// With `enter` the lists still hold vertices.
-__device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, int out, u32 ids,
+// With `enter` the lists still hold vertices.  True where the wave met a deep
+// chain: it keeps the edges from there on as vertices, marked by UNRESOLVED.
+constexpr u32 UNRESOLVED = 0x80000000u;
+static_assert(UNION_VERTICES_MAX <= UNRESOLVED, "bit 31 of a vertex is free");
+__device__ __forceinline__ bool relabel_dense(const UnionArgs& a, WaveLists& l, int out, u32 ids,
                                               bool enter, const u32* parent, DenseRound& t,
-                                              u32 wave, bool& deep) {
+                                              u32 wave) {
   u64* best = minima(a, out);
   for (u32 i = threadIdx.x; i < ids; i += UT) t.best[i] = VAL_NONE;
   if (!enter) {
@@ -1224,6 +1272,7 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
     __syncthreads();
   }
   u32 kept = 0;
+  bool deep = false;
   for (u32 j0 = 0; j0 < l.c; j0 += UR * WAVE) {
     u32 xy[2 * UR];
     u64 k[UR];
@@ -1235,15 +1284,13 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
       k[u] = a.v[0][i];
     }
     if (enter) {
-      if (!find_roots<2 * UR>(a.parent, xy, 31, wave, WALK_DEEP)) {
-        deep = true;
-        break;
-      }
+      deep = deep || !find_roots<2 * UR>(a.parent, xy, 31, wave, walk_deep(a.n));
       u32 id[2 * UR];
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) id[u] = get(at(a.dense_id, xy[u]));
 #pragma unroll
-      for (int u = 0; u < 2 * UR; ++u) xy[u] = min(id[u], ids - 1);  // (a root without an id: none, if symmetric)
+      for (int u = 0; u < 2 * UR; ++u)  // (a root without an id: none, if symmetric)
+        xy[u] = deep ? xy[u] | UNRESOLVED : min(id[u], ids - 1);
     } else {
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) xy[u] = t.root[xy[u]];
@@ -1259,10 +1306,10 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
         a.s[0][q] = x;
         a.d[0][q] = y;
         a.v[0][q] = k[u];
-        if (k[u] < t.best[x])
+        if (!deep && k[u] < t.best[x])
           atomicMin(reinterpret_cast<unsigned long long*>(&t.best[x]),
                     static_cast<unsigned long long>(k[u]));
-        if (k[u] < t.best[y])
+        if (!deep && k[u] < t.best[y])
           atomicMin(reinterpret_cast<unsigned long long*>(&t.best[y]),
                     static_cast<unsigned long long>(k[u]));
       }
@@ -1282,6 +1329,15 @@ __device__ __forceinline__ void relabel_dense(const UnionArgs& a, WaveLists& l, 
 #pragma unroll
   for (u32 j = 0; j < DENSE_MAX / UT; ++j)
     if (k[j] < b[j]) lower(best, j * UT + threadIdx.x, k[j]);
+  return deep;
+}
+
+// The edges that a wave kept as vertices, after shorten_chains.
+__device__ __forceinline__ void convert_rest(const UnionArgs& a, const WaveLists& l, u32 ids) {
+  for (u32 j = lane_id(); j < l.c; j += WAVE)
+    for (u32* x : {a.s[0] + l.base + j, a.d[0] + l.base + j})
+      if (*x & UNRESOLVED)
+        *x = min(get(at(a.dense_id, get(at(a.parent, *x & ~UNRESOLVED)))), ids - 1);
 }
 
 // ------------------------------------------------------------ output
@@ -1346,18 +1402,6 @@ __device__ __forceinline__ UnionArgs arguments() {
   return *(const UnionArgs*)p;
 }
 
-// Block-wide sum of a wave-uniform value, in thread 0 (all threads call).
-__device__ __forceinline__ u64 block_total(u64 wave_value) {
-  __shared__ u64 s_v[UW];
-  __syncthreads();  // thread 0 may still be adding the call before
-  if (lane_id() == 0) s_v[wave_index()] = wave_value;
-  __syncthreads();
-  u64 t = 0;
-  if (threadIdx.x == 0)
-    for (int w = 0; w < UW; ++w) t += s_v[w];
-  return t;
-}
-
 // Sum over the waves before this one of what the workgroups put in their fourth
 // found word, a barrier ago, and this workgroup's waves in s_waves.
 __device__ __forceinline__ u64 waves_before(const UnionArgs& a, const u64* s_waves, u64& s_base) {
@@ -1384,8 +1428,8 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   Barrier bar{a.bar, 0, a.err};
   const u32 n = a.n;
   const int lane = lane_id();
-  const u64 G = gridDim.x, gthread = u64(blockIdx.x) * UT + threadIdx.x, threads = G * UT;
-  const u64 wave = u64(blockIdx.x) * UW + wave_index(), waves = G * UW;
+  const u32 G = gridDim.x, gthread = blockIdx.x * UT + threadIdx.x, threads = G * UT;
+  const u32 wave = blockIdx.x * UW + wave_index(), waves = G * UW;
   u64 sum;
 
   // init
@@ -1395,8 +1439,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
     put(a.span + v, u64{0});
     if (a.parts) put(a.giants + v, u8{0});
   }
-  const u64 words = (a.m + 31) / 32;
-  for (u64 i = gthread; i < words; i += threads) put(a.marks + i, 0u);
+  for (u64 i = gthread; i < (a.m + 31) / 32; i += threads) put(a.marks + i, 0u);
   if (blockIdx.x == 0) pick_pivots(a);
   if (!sync_grid(bar, 0, sum)) return;
 
@@ -1476,11 +1519,11 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       for (u64 v0 = gthread; v0 < n; v0 += 4 * threads) {
         u32 x[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (u32 j = 0; j < 4; ++j)
           x[j] = static_cast<u32>(v0 + j * threads < n ? v0 + j * threads : v0);
         if (!find_roots<4>(a.parent, x, 0, 0, WALK_LIMIT)) atomicOr(a.err, ERR_SPIN);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (u32 j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
           const bool in = v < n && (a.parts ? get(at(a.giants, x[j])) != 0 : x[j] == giant);
           const u64 b = __ballot(in);
@@ -1523,7 +1566,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       if (!last) {
         cross_list(a, l, phase, minima(a, cur), giant, 6 * sum > 5 * u64(n));
       } else if (copies || sum * ROWS_SHARE > a.m) {
-        cross_input(a, l, UnitWalk(a, wave, waves, units), minima(a, cur), giant);
+        cross_input(a, l, UnitWalk(a, wave, waves, (a.m + UNION_UNIT - 1) / UNION_UNIT), minima(a, cur), giant);
       } else {
         // a wave's list holds as many edges as its rows have records
         l.base = waves_before(a, s_waves, s_base);
@@ -1538,46 +1581,54 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
     const bool identity = ids != 0;
     bool resolved = false;  // the last relabel resolved them in LDS
     u64 known = n;  // bound of the roots
+    // the round enters the dense ids; its lists hold vertices still
+    bool enter = false, convert = false;
     while (edges) {
-      if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges | (live << 32);
-      const bool first = phase == 0 && round == 0;
-      const bool note = phase == 0 && !ids && known <= 8 * DENSE_MAX;
-      const u32 lw = hook(a, l, cur, first, first && copies, giant,
-                          ids && !identity ? a.dense_parent : a.parent, note);
-      const u64 block_live = block_total(lw);
-      if (note) {
-        if (lane == 0) s_waves[wave_index()] = lw;
-        if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_live);
-      }
-      if (!sync_grid(bar, block_live, live)) return;
-      known = live;
-      const bool enter = note && live <= DENSE_MAX && edges >= DENSE_EDGES_MIN &&
-                         edges >= DENSE_EDGES * live;
-      if (enter) {
-        // the survivors' ids: their order over the waves
-        u64 id = waves_before(a, s_waves, s_base);
-        for (u32 i = lane; i < lw; i += WAVE) {
-          const u32 v = a.s[1][l.base + i], x = static_cast<u32>(id) + i;
-          put(at(a.dense_id, v), x);
-          put(a.dense_vertex + x, v);
-          put(a.dense_parent + x, x);
-          put(minima(a, cur ^ 1) + x, VAL_NONE);
+      if (__builtin_expect(!(edges >> DEEP_SHIFT), 1)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0 && round < UNION_LOG) a.log[round] = edges | (live << 32);
+        const bool first = phase == 0 && round == 0;
+        const bool note = phase == 0 && !ids && known <= 8 * DENSE_MAX;
+        const u32 lw = hook(a, l, cur, first, first && copies, giant,
+                            ids && !identity ? a.dense_parent : a.parent, note);
+        const u64 block_live = block_total(lw);
+        if (note) {
+          if (lane == 0) s_waves[wave_index()] = lw;
+          if (threadIdx.x == 0) put(a.found + blockIdx.x * 4 + 3, block_live);
         }
-        ids = static_cast<u32>(live);
-        u64 none;
-        if (!sync_grid(bar, 0, none)) return;
+        if (!sync_grid(bar, block_live, live)) return;
+        known = live;
+        enter = note && live <= DENSE_MAX && edges >= DENSE_EDGES_MIN && edges >= DENSE_EDGES * live;
+        convert = enter;
+        if (enter) {
+          // the survivors' ids: their order over the waves
+          u64 id = waves_before(a, s_waves, s_base);
+          for (u32 i = lane; i < lw; i += WAVE) {
+            const u32 v = a.s[1][l.base + i], x = static_cast<u32>(id) + i;
+            put(at(a.dense_id, v), x);
+            put(a.dense_vertex + x, v);
+            put(a.dense_parent + x, x);
+            put(minima(a, cur ^ 1) + x, VAL_NONE);
+          }
+          ids = static_cast<u32>(live);
+          u64 none;
+          if (!sync_grid(bar, 0, none)) return;
+        }
+        cur ^= 1;
+        ++round;
+      } else {  // a wave met a deep chain: the same round's relabel again
+        if (!shorten_chains(a, bar, gthread, threads)) return;
+        if (convert) convert_rest(a, l, ids);
+        convert = false;
+        if (blockIdx.x == 0 && threadIdx.x == 0 && round <= UNION_LOG) a.log[round - 1] |= UNION_CHAINS;
       }
       a = arguments();
-      bool deep = false;
+      bool deep;
       if (ids)
-        relabel_dense(a, l, cur ^ 1, ids, enter, identity ? a.parent : a.dense_parent, s_x.dense,
-                      static_cast<u32>(wave), deep);
-      else relabel(a, l, cur ^ 1, live, s_x.table, giant, static_cast<u32>(wave), deep);
+        deep = relabel_dense(a, l, cur, ids, convert, identity ? a.parent : a.dense_parent, s_x.dense,
+                             wave);
+      else deep = relabel(a, l, cur, live, s_x.table, giant, wave);
       resolved = ids && !enter;
-      cur ^= 1;
-      ++round;
       if (!sync_grid(bar, block_total(l.c | (deep ? u64{1} << DEEP_SHIFT : 0)), edges)) return;
-      if (edges >> DEEP_SHIFT) return;
       if (round >= UNION_ROUNDS_MAX) {
         // every round at least halves the components that have edges
         if (gthread == 0) atomicOr(a.err, ERR_SPIN);
@@ -1601,6 +1652,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   a = arguments();
   // output: workgroups own equal contiguous parts of the mark words, their
   // waves equal parts of those
+  const u64 words = (a.m + 31) / 32;
   const u64 rows = (words + WAVE - 1) / WAVE;  // rows of 64 words
   const u64 r0 = (wave * rows) / waves, r1 = ((wave + 1) * rows) / waves;
   u32 cnt = 0;
