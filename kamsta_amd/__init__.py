@@ -23,6 +23,7 @@ import ctypes
 import dataclasses
 import json
 import os
+import threading
 import weakref
 
 import numpy as np
@@ -154,6 +155,15 @@ def _track(obj):
     _order[0] += 1
     obj._order = _order[0]
     _live.add(obj)
+
+
+def _close_handle(obj, destroy):
+    """Destroys obj's handle once, whichever threads close it (ctypes drops the
+    GIL in the call); every close returns after that."""
+    with obj._closing:
+        h, obj._h = obj._h, ctypes.c_void_p()
+        if h:
+            destroy(h)
 
 
 def load():
@@ -344,15 +354,14 @@ class Context:
 
     def __init__(self, device=0):
         self._lib = load()
+        self._closing = threading.RLock()
         self._h = ctypes.c_void_p()
         _check(self._lib.kmst_context_create(device, ctypes.byref(self._h)))
         self.device = device
         _track(self)
 
     def close(self):
-        if self._h:
-            self._lib.kmst_context_destroy(self._h)
-            self._h = ctypes.c_void_p()
+        _close_handle(self, self._lib.kmst_context_destroy)
 
     def __del__(self):
         try:
@@ -485,6 +494,7 @@ class Server:
         if queue_capacity is not None:
             cfg.queue_capacity = queue_capacity
         cfg.buffer_sets = buffer_sets
+        self._closing = threading.RLock()
         self._h = ctypes.c_void_p()
         _check(self._lib.kmst_server_create(ctypes.byref(cfg), ctypes.byref(self._h)))
         self._live = {}
@@ -529,10 +539,8 @@ class Server:
         return b.value, q.value
 
     def close(self):
-        if self._h:
-            self._lib.kmst_server_destroy(self._h)
-            self._h = ctypes.c_void_p()
-            self._live.clear()
+        _close_handle(self, self._lib.kmst_server_destroy)
+        self._live.clear()
 
     def __del__(self):
         try:
