@@ -1361,6 +1361,18 @@ kmst_status host_solve(const kmst_wedge* in, uint64_t m, const kmst_config* cfg,
     if (m >= (uint64_t{1} << 32) - 1) throw kmst::Error(KMST_EINVAL, "more than 2^32-2 records");
     kmst_config c = *cfg;
     c.algorithm = algorithm;
+    uint64_t vmax = 0;
+    std::vector<uint32_t> s, d, w;
+    if (m && c.compression == 1) {  // before the lock: callers convert side by side
+      s.resize(m), d.resize(m), w.resize(m);
+      for (uint64_t i = 0; i < m; ++i) {
+        check_ids(in[i]);
+        s[i] = static_cast<uint32_t>(in[i].src);
+        d[i] = static_cast<uint32_t>(in[i].dst);
+        w[i] = in[i].weight;
+        vmax = std::max<uint64_t>(vmax, std::max(in[i].src, in[i].dst));
+      }
+    }
     std::lock_guard<std::mutex> lk(g_default_mu);
     kmst_context* ctx = default_context(c.device);
     KMST_HIP(hipSetDevice(ctx->device));
@@ -1368,17 +1380,7 @@ kmst_status host_solve(const kmst_wedge* in, uint64_t m, const kmst_config* cfg,
     uint32_t* ds = static_cast<uint32_t*>(ctx->in_s.get(mm * 4));
     uint32_t* dd = static_cast<uint32_t*>(ctx->in_d.get(mm * 4));
     uint32_t* dw = static_cast<uint32_t*>(ctx->in_w.get(mm * 4));
-    uint64_t vmax = 0;
-    std::vector<uint32_t> s, d, w;
-    if (m && c.compression == 1) {
-      s.resize(m), d.resize(m), w.resize(m);
-      for (uint64_t i = 0; i < m; ++i) {
-        s[i] = static_cast<uint32_t>(in[i].src);
-        d[i] = static_cast<uint32_t>(in[i].dst);
-        w[i] = in[i].weight;
-        vmax = std::max<uint64_t>(vmax, std::max(in[i].src, in[i].dst));
-      }
-    } else if (m) {
+    if (m && c.compression == 0) {
       try {
         vmax = upload_records(*ctx, in, m, ds, dd, dw);
       } catch (...) {
