@@ -400,7 +400,6 @@ constexpr u64 UNION_UNIT = 256;        // records a wave takes per step
 constexpr u64 UNION_VERTICES_MAX = u64{1} << 28;  // byte offsets of 8-byte words fit 32 bits
 constexpr u32 UNION_CLASSES = 3;       // light weight classes at most
 constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
-constexpr u32 UNION_ROUNDS_MAX = 200;
 constexpr u32 UNION_LOG = 60;          // u64 words: rounds (edges, roots << 32), ...
 constexpr u32 UNION_CHAINS = 0x80000000u;  // above the edges (2^31 - 1 at most): shorten_chains ran
 constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 4 phases

@@ -57,6 +57,7 @@
 // range changes hands once, behind a release and an acquire).
 #include "kmst_kernels.hpp"
 #include "kmst_rows.hpp"
+#include "kmst_walks.hpp"
 
 namespace kmst {
 
@@ -67,19 +68,6 @@ constexpr int UW = UT / WAVE;
 constexpr u64 WALL_TICKS_PER_MS = 100000;              // 100 MHz wall clock
 constexpr u64 BARRIER_TICKS = 10000 * WALL_TICKS_PER_MS;  // bound of a barrier's wait
 constexpr u64 JOIN_TICKS = 5 * WALL_TICKS_PER_MS;      // bound of the first one's
-constexpr u32 WALK_LIMIT = 1u << 26;                   // a longer walk is a corrupted forest
-// Weights in order along a path hook it into one chain, which walks of the list's
-// entries may not shorten for each other.  A walk longer than this stops, and
-// shorten_chains takes all vertices to their roots before the round goes on.  A
-// step takes some 0.9 us, the passes 15 us up to 10^5 vertices and a time that
-// grows with n past that, hence the limit.  10^6 vertices, descending weights along a path,
-// heavier chords: 0.44 ms, 116 where the round loop took over after 1024 steps
-// (114 alone); 9000 vertices of a band 160 us, 1265 (205); a grid of 300 x 300
-// 166 us, 313 with walks alone (250).  Random weights stay below
-// (of 162 graphs of 8200 to 200000 vertices one met a limit of 8, none one of 10).
-constexpr u32 WALK_DEEP_MIN = 10;
-constexpr int WALK_DEEP_SHIFT = 15;
-__device__ __forceinline__ u32 walk_deep(u32 n) { return WALK_DEEP_MIN + (n >> WALK_DEEP_SHIFT); }
 constexpr int DEEP_SHIFT = 35;  // in a relabel's payload, above the edges of all waves
 
 // wave index, in a scalar register: what follows from it (a wave's units, list
@@ -800,7 +788,7 @@ __device__ __forceinline__ u32 most_frequent(u32 x) {
 __device__ __forceinline__ u32 pick_giant(const UnionArgs& a) {
   // (the roots do not change meanwhile: every workgroup picks the same)
   u32 x[1] = {static_cast<u32>((u64(lane_id()) * a.n) / WAVE)};
-  (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
+  (void)find_roots<1>(a.parent, x, NONE32, 0, walk_limit(a.n));
   return most_frequent(x[0]);
 }
 // A graph of unconnected parts has a giant each, one wave per part picks it.
@@ -818,7 +806,7 @@ __device__ __forceinline__ void pick_giants(const UnionArgs& a, u64 wave, u64 wa
     u32 g = NONE32;
     if (len) {
       u32 x[1] = {v0 + static_cast<u32>((u64(lane_id()) * len) / WAVE)};
-      (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
+      (void)find_roots<1>(a.parent, x, NONE32, 0, walk_limit(a.n));
       g = most_frequent(x[0]);
     }
     if (!lead) continue;
@@ -1521,7 +1509,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
 #pragma unroll
         for (u32 j = 0; j < 4; ++j)
           x[j] = static_cast<u32>(v0 + j * threads < n ? v0 + j * threads : v0);
-        if (!find_roots<4>(a.parent, x, 0, 0, WALK_LIMIT)) atomicOr(a.err, ERR_SPIN);
+        if (!find_roots<4>(a.parent, x, 0, 0, walk_limit(n))) atomicOr(a.err, ERR_SPIN);
 #pragma unroll
         for (u32 j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64
