@@ -302,6 +302,10 @@ kmst_status kmst_k_sort_pairs(kmst_context* ctx, uint32_t* src, uint32_t* dst,
                               uint64_t* val, uint64_t m, uint32_t bits);
 /* K3: parent[v] <- root of v, in place. */
 kmst_status kmst_k_pointer_jump(kmst_context* ctx, uint32_t* parent, uint64_t n);
+/* The next direct solve on ctx that takes several workgroups is called off at
+ * its first barrier, as it is where other work holds the GPU: the round loop
+ * solves. */
+kmst_status kmst_k_call_off(kmst_context* ctx);
 
 #ifdef __cplusplus
 }

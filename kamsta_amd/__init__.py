@@ -50,7 +50,7 @@ EXPORTED_SYMBOLS = [
     "kmst_encode_host",
     "kmst_last_error", "kmst_context_stats_json", "kmst_gen_gnm_device", "kmst_gen_gnm_host",
     "kmst_k_segmented_argmin", "kmst_k_segmented_argmin_packed", "kmst_k_sort_pairs",
-    "kmst_k_pointer_jump",
+    "kmst_k_pointer_jump", "kmst_k_call_off",
     "kmst_server_config_default", "kmst_server_create", "kmst_server_submit", "kmst_server_poll",
     "kmst_server_wait", "kmst_server_counters", "kmst_server_destroy",
 ]
@@ -215,6 +215,7 @@ def load():
         "kmst_k_segmented_argmin_packed": (i32, [vp, vp, vp, vp, u32, u64, u64, vp, vp]),
         "kmst_k_sort_pairs": (i32, [vp, vp, vp, vp, u64, u32]),
         "kmst_k_pointer_jump": (i32, [vp, vp, u64]),
+        "kmst_k_call_off": (i32, [vp]),
         "kmst_server_config_default": (None, [vp]),
         "kmst_server_create": (i32, [vp, ctypes.POINTER(vp)]),
         "kmst_server_submit": (i32, [vp, vp, vp, vp, u64, u64, vp, vp, vp, u64, pu64]),
@@ -467,6 +468,9 @@ class Context:
 
     def pointer_jump(self, parent, n):
         _check(self._lib.kmst_k_pointer_jump(self._h, _ptr(parent), n))
+
+    def call_off(self):
+        _check(self._lib.kmst_k_call_off(self._h))
 
 
 class Server:

@@ -403,6 +403,7 @@ constexpr u64 UNION_CHUNK_MAX = 16;    // units of a chunk at most
 constexpr u32 UNION_LOG = 60;          // u64 words: rounds (edges, roots << 32), ...
 constexpr u32 UNION_CHAINS = 0x80000000u;  // above the edges (2^31 - 1 at most): shorten_chains ran
 constexpr u32 UNION_LOG_TOTAL = 64;    // ... then the rounds at the end of each of 4 phases
+constexpr u32 UNION_CALLED_OFF = 0x80000000u;  // in *joined: every workgroup leaves
 constexpr u32 UNION_BAR_WORDS = 12 * 16;  // u64 words of the grid barrier
 enum : u32 {     // words of UnionArgs::ctl
   UC_PIVOT = 0,  // UNION_CLASSES pivots: the classes' largest weights

@@ -1110,11 +1110,18 @@ bool Solver::direct(u32* out_s, u32* out_d, u32* out_w, u64 out_cap, u64* out_n,
     union_solve_small(st, a, weight, ctr + C_UGROUPS, p);
   } else {
     fill_u32(st, ctr, 64 + 2 * (UNION_LOG_TOTAL + UNION_BAR_WORDS), 0);
+    if (C.call_off && blocks > 1) {
+      fill_u32(st, a.joined, 1, UNION_CALLED_OFF);
+      C.call_off = false;
+    }
     union_solve(st, a, blocks, weight, ctr + C_UGROUPS, ctr + C_UENDED, p);
   }
   if (p.host) await_published(p.seq);
   else fetch(reinterpret_cast<const u32*>(a.log), 2 * UNION_LOG_TOTAL);
-  if (!small && blocks > 1 && C.host_counters[C_UJOINED] != blocks) return false;
+  if (!small && blocks > 1 && C.host_counters[C_UJOINED] != blocks) {
+    C.stats.called_off = true;
+    return false;
+  }
   check_input_words();
   if (!C.host_counters[C_UNION + UC_DONE]) throw Error(KMST_EDEVICE, "direct solve: not finished");
   const u64 cnt = C.host_counters[C_UCOUNT];
@@ -1740,6 +1747,13 @@ kmst_status kmst_k_sort_pairs(kmst_context* ctx, uint32_t* src, uint32_t* dst, u
   });
 }
 
+kmst_status kmst_k_call_off(kmst_context* ctx) {
+  return guarded([&] {
+    if (!ctx) throw kmst::Error(KMST_EINVAL, "null context");
+    ctx->call_off = true;
+  });
+}
+
 kmst_status kmst_k_pointer_jump(kmst_context* ctx, uint32_t* parent, uint64_t n) {
   return guarded([&] {
     if (!ctx) throw kmst::Error(KMST_EINVAL, "null context");
@@ -1761,6 +1775,7 @@ size_t kmst_context_stats_json(const kmst_context* ctx, char* buf, size_t cap) {
   o << "{\"n\":" << s.n << ",\"m\":" << s.m << ",\"algorithm\":" << s.algorithm
     << ",\"packed_keys\":" << (s.packed_keys ? "true" : "false")
     << ",\"lazy_keys\":" << (s.lazy_keys ? "true" : "false")
+    << ",\"called_off\":" << (s.called_off ? "true" : "false")
     << ",\"readback\":\"" << (ctx->host_mapped ? "publish" : "copy") << "\""
     << ",\"mst_edges\":" << s.mst_edges << ",\"total_weight\":" << s.total_weight
     << ",\"mst_long_groups\":" << s.mst_long_groups

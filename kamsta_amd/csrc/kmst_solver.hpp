@@ -57,6 +57,7 @@ struct SolveStats {
   u64 n = 0, m = 0, mst_edges = 0, total_weight = 0;
   int algorithm = 0;
   bool packed_keys = true;
+  bool called_off = false;  // the direct solve's workgroups were not resident together
   bool lazy_keys = false;  // positional keys made by the class scatter, not stored
   u64 max_weight = 0;
   // output order: groups of one smaller endpoint (or position range) longer
@@ -155,6 +156,7 @@ struct kmst_context {
   kmst::SortWork sort_work;  // radix sort state over `hist`
   kmst::LookbackWork lb_work;  // compaction look-back state over `lookback`
   kmst_tuning tuning{0, 1, kmst::SORT_WIDE_MIN, kmst::PERSIST_MAX_DEFAULT};  // launch shapes of later solves
+  bool call_off = false;  // the next direct solve on several workgroups (kmst_k_call_off)
   // host-API staging
   kmst::DevBuf in_s, in_d, in_w, out_s, out_d, out_w;
   kmst::HostStage stage;

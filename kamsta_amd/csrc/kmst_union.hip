@@ -135,7 +135,6 @@ __device__ __forceinline__ u32 dpp(u32 old, u32 x) {
 constexpr u32 GROUPS = 8;
 constexpr u32 LINE = 16;  // u64 words per 128-byte line
 constexpr u64 PAYLOAD_SHIFT = 16;
-constexpr u32 CALLED_OFF = 0x80000000u;
 
 struct Barrier {
   u64* words;  // root words at lines 0..3, group words at lines 4..11
@@ -208,14 +207,14 @@ __device__ __forceinline__ bool join_grid(u32* joined) {
     if (gridDim.x > 1) {
       u32 seen = __hip_atomic_fetch_add(joined, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
       const u64 t0 = wall_clock64();
-      while (seen != gridDim.x && !(seen & CALLED_OFF)) {
+      while (seen != gridDim.x && !(seen & UNION_CALLED_OFF)) {
         if (wall_clock64() - t0 > JOIN_TICKS)
-          (void)atomicCAS(joined, seen, seen | CALLED_OFF);  // fails if someone joined: look again
+          (void)atomicCAS(joined, seen, seen | UNION_CALLED_OFF);  // fails if someone joined: look again
         else
           __builtin_amdgcn_s_sleep(1);
         seen = get(joined);
       }
-      ok = seen & CALLED_OFF ? 0u : 1u;
+      ok = seen & UNION_CALLED_OFF ? 0u : 1u;
     }
     s_join = ok;
   }
