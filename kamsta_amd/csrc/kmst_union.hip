@@ -1213,6 +1213,27 @@ __device__ __forceinline__ bool relabel(const UnionArgs& a, WaveLists& l, int ou
   return deep;
 }
 
+// Every one of `count` parents in LDS onto its root (all threads call, *open is 0
+// before; ends with a barrier).  A walk stops after LDS_WALK steps and all walk again
+// from where they are: a chain falls to a sixteenth.  Walked to the end in one go, with the
+// root at the highest id, a band of 4096 vertices took 435 us a call (60 now), a ring of
+// 8192 1700 (78); a store every step costs random trees, some ten deep, 3 us a round.
+constexpr u32 LDS_WALK = 16;
+constexpr u32 LDS_PASSES = 6;  // 16^6: more is a cycle
+__device__ __forceinline__ void roots_in_lds(u32* parent, u32 count, u32* open) {
+  for (u32 pass = 1; pass <= LDS_PASSES; ++pass) {
+    for (u32 i = threadIdx.x; i < count; i += UT) {
+      // (others shorten the walked paths meanwhile)
+      u32 r = parent[i], steps = 0;
+      for (u32 p; (p = parent[r]) != r && steps < LDS_WALK; ++steps) r = p;
+      parent[i] = r;
+      if (steps == LDS_WALK) *open = pass;
+    }
+    __syncthreads();
+    if (*open < pass) return;
+  }
+}
+
 // Few roots: with at most DENSE_MAX of them left in the first class's rounds,
 // the lists hold dense ids.  A round's hooks then lie over few words, which every
 // workgroup reads into its LDS and resolves there, where a step of a walk takes a
@@ -1229,6 +1250,7 @@ constexpr u64 DENSE_EDGES = 16, DENSE_EDGES_MIN = 4096;  // edges per root, and 
 struct DenseRound {
   u32 root[DENSE_MAX];
   u64 best[DENSE_MAX];
+  u32 open;
 };
 // With `enter` the lists still hold vertices.  True where the wave met a deep
 // chain: it keeps the edges from there on as vertices, marked by UNRESOLVED.
@@ -1238,6 +1260,7 @@ __device__ __forceinline__ bool relabel_dense(const UnionArgs& a, WaveLists& l, 
                                               bool enter, const u32* parent, DenseRound& t,
                                               u32 wave) {
   u64* best = minima(a, out);
+  if (threadIdx.x == 0) t.open = 0;
   for (u32 i = threadIdx.x; i < ids; i += UT) t.best[i] = VAL_NONE;
   if (!enter) {
     u32 p[DENSE_MAX / UT];  // all in flight together
@@ -1250,13 +1273,7 @@ __device__ __forceinline__ bool relabel_dense(const UnionArgs& a, WaveLists& l, 
   }
   __syncthreads();
   if (!enter) {
-    for (u32 i = threadIdx.x; i < ids; i += UT) {
-      // (others shorten the walked paths meanwhile)
-      u32 r = t.root[i], steps = 0;
-      for (u32 p; (p = t.root[r]) != r && steps < DENSE_MAX; ++steps) r = p;
-      t.root[i] = r;
-    }
-    __syncthreads();
+    roots_in_lds(t.root, ids, &t.open);
   }
   u32 kept = 0;
   bool deep = false;
@@ -1763,7 +1780,7 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
   __shared__ u64 s_best[UNION_SMALL_VERTICES];
   __shared__ u32 s_marks[SMALL_WORDS], s_before[SMALL_WORDS];
   __shared__ u64 s_fwd_hash, s_rev_hash, s_weight;
-  __shared__ u32 s_fwd, s_bad, s_live[3], s_count, s_groups;
+  __shared__ u32 s_fwd, s_bad, s_live[3], s_open, s_count, s_groups;
   __shared__ u64 s_log[UNION_LOG];
   __shared__ u32 s_scan[UW];
   const u32 t = threadIdx.x, lane = lane_id(), n = a.n, m = static_cast<u32>(a.m);
@@ -1848,7 +1865,7 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
       if (key < s_best[y])
         atomicMin(reinterpret_cast<unsigned long long*>(&s_best[y]), static_cast<unsigned long long>(key));
     }
-    if (t == 0) s_live[(round + 1) % 3] = 0;
+    if (t == 0) s_live[(round + 1) % 3] = s_open = 0;
     __syncthreads();
     u32 mine = 0;  // edges that stay | roots that live on << 16
 #pragma unroll
@@ -1868,14 +1885,8 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
       atomicOr(&s_marks[i / 32], 1u << (i & 31));
     }
     __syncthreads();
-    for (u32 v = t; v < n; v += UT) {
-      // (others shorten the walked paths meanwhile)
-      u32 r = s_parent[v], steps = 0;
-      for (u32 q; (q = s_parent[r]) != r && steps < UNION_SMALL_VERTICES; ++steps) r = q;
-      s_parent[v] = r;
-      s_best[v] = VAL_NONE;
-    }
-    __syncthreads();
+    for (u32 v = t; v < n; v += UT) s_best[v] = VAL_NONE;
+    roots_in_lds(s_parent, n, &s_open);
 #pragma unroll
     for (int k = 0; k < SMALL_SLOTS; ++k) {
       if (!((alive >> k) & 1)) continue;
