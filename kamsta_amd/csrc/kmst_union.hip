@@ -1110,8 +1110,17 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
           other = x[u];
         }
         bool hooked = true;
-        if (copies) hooked = atomicCAS(at(parent, child), child, other) == child;
-        else put(at(parent, child), other);
+        if (copies) {
+          // a wave's lanes hold the copies of one edge together: the first of them
+          // claims its child, if no other wave has (claims of one address take 12 ns each:
+          // 10^6 copies between two vertices 12 ms, without the look and the choice)
+          const u32 lead = __builtin_amdgcn_readfirstlane(child);
+          const u64 same = __ballot(child == lead);
+          hooked = (child != lead || mbcnt(same) == 0) && get(at(parent, child)) == child &&
+                   atomicCAS(at(parent, child), child, other) == child;
+        } else {
+          put(at(parent, child), other);
+        }
         if (hooked) {
           lives = mx && my;
           if (lives) put(at(next, other), VAL_NONE);  // the root that lives on
