@@ -787,7 +787,7 @@ __device__ __forceinline__ u32 most_frequent(u32 x) {
 __device__ __forceinline__ u32 pick_giant(const UnionArgs& a) {
   // (the roots do not change meanwhile: every workgroup picks the same)
   u32 x[1] = {static_cast<u32>((u64(lane_id()) * a.n) / WAVE)};
-  (void)find_roots<1>(a.parent, x, NONE32, 0, walk_limit(a.n));
+  (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
   return most_frequent(x[0]);
 }
 // A graph of unconnected parts has a giant each, one wave per part picks it.
@@ -805,7 +805,7 @@ __device__ __forceinline__ void pick_giants(const UnionArgs& a, u64 wave, u64 wa
     u32 g = NONE32;
     if (len) {
       u32 x[1] = {v0 + static_cast<u32>((u64(lane_id()) * len) / WAVE)};
-      (void)find_roots<1>(a.parent, x, NONE32, 0, walk_limit(a.n));
+      (void)find_roots<1>(a.parent, x, NONE32, 0, WALK_LIMIT);
       g = most_frequent(x[0]);
     }
     if (!lead) continue;
@@ -1191,7 +1191,7 @@ __device__ __forceinline__ bool relabel(const UnionArgs& a, WaveLists& l, int ou
       xy[UR + u] = a.d[0][i];
       k[u] = a.v[0][i];
     }
-    deep = deep || !find_roots<2 * UR>(a.parent, xy, thin, wave, walk_deep(a.n));
+    deep = deep || !find_roots<2 * UR>(a.parent, xy, thin, wave, WALK_DEEP);
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
       const u32 x = xy[u], y = xy[UR + u];
@@ -1297,7 +1297,7 @@ __device__ __forceinline__ bool relabel_dense(const UnionArgs& a, WaveLists& l, 
       k[u] = a.v[0][i];
     }
     if (enter) {
-      deep = deep || !find_roots<2 * UR>(a.parent, xy, 31, wave, walk_deep(a.n));
+      deep = deep || !find_roots<2 * UR>(a.parent, xy, 31, wave, WALK_DEEP);
       u32 id[2 * UR];
 #pragma unroll
       for (int u = 0; u < 2 * UR; ++u) id[u] = get(at(a.dense_id, xy[u]));
@@ -1534,7 +1534,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
 #pragma unroll
         for (u32 j = 0; j < 4; ++j)
           x[j] = static_cast<u32>(v0 + j * threads < n ? v0 + j * threads : v0);
-        if (!find_roots<4>(a.parent, x, 0, 0, walk_limit(n))) atomicOr(a.err, ERR_SPIN);
+        if (!find_roots<4>(a.parent, x, 0, 0, WALK_LIMIT)) atomicOr(a.err, ERR_SPIN);
 #pragma unroll
         for (u32 j = 0; j < 4; ++j) {
           const u64 v = v0 + j * threads;  // consecutive over a wave, from a multiple of 64

@@ -11,26 +11,19 @@ constexpr std::uint32_t UNION_ROUNDS_MAX = 200;
 
 // Weights in order along a path hook it into one chain, which walks of the list's
 // entries may not shorten for each other.  A walk longer than this stops, and
-// shorten_chains takes all vertices to their roots before the round goes on.  A
-// step takes some 0.9 us, the passes 15 us up to 10^5 vertices and a time that
-// grows with n past that, hence the limit.  10^6 vertices, descending weights along a path,
-// heavier chords: 0.44 ms, 116 where the round loop took over after 1024 steps
-// (114 alone); 9000 vertices of a band 160 us, 1265 (205); a grid of 300 x 300
-// 166 us, 313 with walks alone (250).  Random weights stay below
-// (of 162 graphs of 8200 to 200000 vertices one met a limit of 8, none one of 10).
-constexpr std::uint32_t WALK_DEEP_MIN = 10;
-constexpr int WALK_DEEP_SHIFT = 15;
-constexpr std::uint32_t walk_deep(std::uint32_t n) {
-  return WALK_DEEP_MIN + (n >> WALK_DEEP_SHIFT);
-}
+// shorten_chains takes all vertices to their roots before the round goes on.  Both cost
+// with n: at 10^6 vertices a step of all walks takes 4 to 11 us, the passes 15 to 30; hence
+// one limit for all sizes.  Bands 8 wide, the vertices in random order, with limits of
+// 10, 12, 16 and 42: 1301, 1328, 1415 and 1778 us at 2^20 vertices; at 2^22 2705, 2756,
+// 2900 and (with 138) 4191.  Random weights stay below: of 76 random, geometric and
+// hyperbolic graphs of 2^17 to 2^24 vertices two met a limit of 10 (1 % slower), none one of 14.
+constexpr std::uint32_t WALK_DEEP = 12;
 
 // Steps of a walk in a whole forest: after a round every vertex that hooked in it is
-// within walk_deep of a root, and a later round adds as much.  The symmetry sums
+// within WALK_DEEP of a root, and a later round adds as much.  The symmetry sums
 // can collide, and hooks of records that are not symmetric may close a cycle, which
 // rounds on dense ids do not meet: a walk past this is one, and the solve ends with an error.
 // With a bound of 2^26 steps each such walk took a minute.
-constexpr std::uint32_t walk_limit(std::uint32_t n) {
-  return UNION_ROUNDS_MAX * (walk_deep(n) + 2);
-}
+constexpr std::uint32_t WALK_LIMIT = UNION_ROUNDS_MAX * (WALK_DEEP + 2);
 
 }  // namespace kmst
