@@ -1223,23 +1223,27 @@ __device__ __forceinline__ bool relabel(const UnionArgs& a, WaveLists& l, int ou
 }
 
 // Every one of `count` parents in LDS onto its root (all threads call, *open is 0
-// before; ends with a barrier).  A walk stops after LDS_WALK steps and all walk again
-// from where they are: a chain falls to a sixteenth.  Walked to the end in one go, with the
-// root at the highest id, a band of 4096 vertices took 435 us a call (60 now), a ring of
-// 8192 1700 (78); a store every step costs random trees, some ten deep, 3 us a round.
+// before; ends with a barrier), and beside(i) for each.  A walk stops after LDS_WALK
+// steps and all walk again from where they are: a chain falls to a sixteenth.  Walked to
+// the end in one go, with the root at the highest id, a band of 4096 vertices took 435 us a
+// call (60 now), a ring of 8192 1700 (78); random trees, some ten deep, take one pass and 0.2
+// us a round for the look at *open (2^8 vertices 47.9 -> 48.9 us).  A store every step
+// costs those 3 us a round.
 constexpr u32 LDS_WALK = 16;
 constexpr u32 LDS_PASSES = 6;  // 16^6: more is a cycle
-__device__ __forceinline__ void roots_in_lds(u32* parent, u32 count, u32* open) {
-  for (u32 pass = 1; pass <= LDS_PASSES; ++pass) {
+template <typename F>
+__device__ __forceinline__ void roots_in_lds(u32* parent, u32 count, u32* open, F&& beside) {
+  for (u32 pass = 1;; ++pass) {
     for (u32 i = threadIdx.x; i < count; i += UT) {
       // (others shorten the walked paths meanwhile)
       u32 r = parent[i], steps = 0;
       for (u32 p; (p = parent[r]) != r && steps < LDS_WALK; ++steps) r = p;
       parent[i] = r;
+      beside(i);
       if (steps == LDS_WALK) *open = pass;
     }
     __syncthreads();
-    if (*open < pass) return;
+    if (*open < pass || pass == LDS_PASSES) return;
   }
 }
 
@@ -1282,7 +1286,7 @@ __device__ __forceinline__ bool relabel_dense(const UnionArgs& a, WaveLists& l, 
   }
   __syncthreads();
   if (!enter) {
-    roots_in_lds(t.root, ids, &t.open);
+    roots_in_lds(t.root, ids, &t.open, [](u32) {});
   }
   u32 kept = 0;
   bool deep = false;
@@ -1894,8 +1898,7 @@ __global__ __launch_bounds__(UT) void union_small_kernel(UnionArgs a, u64* total
       atomicOr(&s_marks[i / 32], 1u << (i & 31));
     }
     __syncthreads();
-    for (u32 v = t; v < n; v += UT) s_best[v] = VAL_NONE;
-    roots_in_lds(s_parent, n, &s_open);
+    roots_in_lds(s_parent, n, &s_open, [&](u32 v) { s_best[v] = VAL_NONE; });
 #pragma unroll
     for (int k = 0; k < SMALL_SLOTS; ++k) {
       if (!((alive >> k) & 1)) continue;
