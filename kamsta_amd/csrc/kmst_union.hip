@@ -283,6 +283,8 @@ __device__ __forceinline__ bool find_roots(u32* parent, u32 (&x)[N], u32 thin, u
   u32 open = 0, moved = 0;  // bit j: walk j has not ended / has left its first parent
 #pragma unroll
   for (int j = 0; j < N; ++j) open |= p[j] != x[j] ? 1u << j : 0u;
+  // (unrolled as far as a constant limit the loop costs 10^6 spokes of a wheel 475 us, not 405)
+#pragma unroll 1
   for (u32 step = 1; __any(open != 0); ++step) {
     u32 y[N];
 #pragma unroll
