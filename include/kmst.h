@@ -160,7 +160,11 @@ typedef struct kmst_tuning {
   uint64_t persistent_max;   /* rounds on at most this many live records (with at most
                                 twice as many vertex ids, plus 1024, and at most 32 records
                                 per vertex id or at most 2^14 records) run to the end in
-                                one persistent cooperative launch; 0 = never */
+                                one persistent cooperative launch; 0 = never.  Any value
+                                but the default also keeps every solve on the round loop:
+                                with the default, inputs of at least two records per
+                                vertex take the direct solve (1.5 to 11 times faster),
+                                which none of these fields changes */
 } kmst_tuning;
 
 /* The defaults (0, 1, 2^20, 2^18). */

@@ -102,6 +102,7 @@ class Tuning:
     balanced_digits: int = 1       # digit widths balanced over the passes
     sort_wide_min: int = 1 << 20   # with sort_threads 0: 512-thread tiles from here on
     persistent_max: int = 1 << 18  # rounds on at most this many records: one persistent launch
+                                   # (any other value also turns the direct solve off)
 
     def _c(self):
         return _Tuning(self.sort_threads, self.balanced_digits, self.sort_wide_min,

@@ -1012,21 +1012,33 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // graph is one launch and one read-back, where the round loop needs 60 to 250
 // launches and 7 to 34 read-backs; on a large one it moves each edge of the
 // lightest classes once a round and the others hardly at all, where the round
-// loop scatters, sorts and renumbers both records.  Measured, direct / round
-// loop: 46 / 179 us at 256 vertices, 205 / 540 at 2^14, 317 / 1394 at 2^17, 577
-// / 1736 and 728 / 2599 at 10^6 (16 and 32 records per vertex); 6.65 ms at 2^24
-// (32, random) against 10.4 filtering and 76 not, 4.55 / 8.0 geometric.  Sparse
-// inputs (fewer than two records per vertex: forests) stay with the round loop,
-// and so does a context whose persistent-round limit was set by hand.
+// loop scatters, sorts and renumbers both records (figures: kmst_union.hip).
+// Sparse inputs (fewer than two records per vertex: forests) stay with the round
+// loop, and so does a context whose persistent-round limit was set by hand.  The
+// first line is on the safe side: random graphs, direct / plain round loop, take
+// at 1, 2 and 3 records per vertex 208 / 247, 260 / 285 and 281 / 283 us at 2^14
+// vertices, 281 / 343, 323 / 445 and 354 / 484 at 2^17, 335 / 597, 454 / 919 and 564 /
+// 1150 at 2^20, 0.91 / 1.57, 2.06 / 2.77 and 2.16 / 4.06 ms at 2^23.
+// Known to be slower than the round loop (plain): weights in order along a band 8
+// to 16 wide, 2^12 to 2^16 vertices, by 7 to 22 %; the same of 2^20 vertices in random
+// order, 1.32 against 0.82 ms; a wheel of 10^6 vertices whose hub's edges are the
+// heaviest, 2.3 against 1.65 ms (every wave's minimum goes to the hub).
 //
 // Light edges beyond what joins vertices stay in the lists round after round,
 // until their components meet: on a random graph 0.25 n of 1.1 n edges at
 // degree 2.2, 0.03 n of 0.7 n at 1.4.  From DIRECT_MID_VERTICES on the rounds'
-// work outweighs the barriers of a second light class (16 records per vertex,
-// random / geometric, with one class and two: 270 / 257 and 301 / 294 us at 2^16,
-// 317 / 274 and 328 / 385 at 2^17, 413 / 331 and 394 / 373 at 2^18, 614 / 413 and 477
-// / 431 at 2^19), from DIRECT_FINE_VERTICES on that of a third (at 2^24 7.5 ms with
-// three, 9.0 with two; at 10^6 random 815 / 835 us, geometric 710 / 650).
+// work outweighs the barriers of a second light class, from
+// DIRECT_FINE_VERTICES on those of a third.  One / two / three classes, 16 and 32
+// records per vertex random and 16 geometric, us:
+//   2^17   311 / 326 / 371     336 / 334 / 377     273 / 314 / 388
+//   2^18   407 / 389 / 418     433 / 384 / 412     329 / 393 / 439
+//   2^19   607 / 474 / 482     694 / 520 / 516     400 / 414 / 487
+//   2^20   883 / 641 / 639    1006 / 706 / 716     580 / 559 / 636
+//   2^21  1536 / 1025 / 946   1781 / 1207 / 1105   874 / 800 / 904
+//   2^22  3209 / 1922 / 1618  3566 / 2102 / 1944  1569 / 1337 / 1419
+// The lines lie where random graphs turn; geometric ones lose 64 and 14 us at
+// 2^18 and 2^19 to the second class, 104 and 82 at 2^21 and 2^22 to the third (at 2^24 three
+// classes gain: random 7.5 ms, 9.0 with two).
 constexpr double DIRECT_FIRST_DEGREE = 2.2;
 constexpr u64 DIRECT_MID_VERTICES = u64{1} << 18;
 constexpr double DIRECT_FINE_DEGREES[2] = {1.4, 2.4};

@@ -36,8 +36,9 @@ struct RoundStat {
   u32 run_starts = 0;       // of RUN_SAMPLES sampled next-round records (0: not sampled)
   u32 far_starts = 0;       // ... whose source is 16 or more ids from the record before
   bool persistent = false;  // ran inside the persistent launch
-  // took the src < dst half of records with far-apart ids (round loop:
-  // relabelled it and wrote both directions)
+  // round loop: relabelled the src < dst half of records with far-apart ids and wrote
+  // both directions.  The direct solve always takes that half: there it says that
+  // the ids are far apart
   bool twins = false;
   // a round of the direct solve (run_starts: sampled input records) whose roots
   // were found by walks from the list's entries, or by passes over all vertices

@@ -1,6 +1,7 @@
 // kmst_union.hip -- the direct solve: a whole minimum spanning forest in one
-// launch of resident workgroups, on undirected edge lists over a union-find
-// parent array.
+// launch of resident workgroups (and two short ones: a fill of the counters
+// before it, their publication after it), on undirected edge lists over a
+// union-find parent array.
 //
 // Phases (every size is read on the device; a grid barrier between phases):
 //
@@ -49,9 +50,9 @@
 // A large one is bound by random accesses, 8 to 16 bytes of 64 to 128 MB tables
 // for every listed edge and round, and by the light pass.
 // Measured a whole solve, this against the round loop: 256 vertices, 4.4 10^3
-// records 46 / 185 us (union_small_kernel); 2^14, 4.9 10^5 205 / 525 us; 2^17, 2.1 10^6 330 / 1394
-// us; 10^6, 3.2 10^7 728 / 2599 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
-// 6.65 / 10.4 ms (1.36 ms).
+// records 50 / 185 us (union_small_kernel); 2^14, 5.2 10^5 208 / 534 us; 2^17, 2.1 10^6 317 / 1394
+// us; 10^6, 3.2 10^7 729 / 2628 us (a copy of its bytes: 81 us); 2^24, 5.4 10^8
+// 6.75 / 10.5 ms (1.36 ms).
 // Lists are private to a wave, so they need no coherence, counters or
 // workgroup barriers, and their compaction is in place (plain accesses: a wave's
 // range changes hands once, behind a release and an acquire).
@@ -1259,7 +1260,7 @@ __device__ __forceinline__ void roots_in_lds(u32* parent, u32 count, u32* open, 
 // to 7 us, 40 to 9 as walks with a hashed table of minima; at 2^14, 3 10^4 edges, in 8
 // to 5 us, 18 to 7.  Entering takes two barriers more: not worth it with few
 // edges (geometric graphs, 13 us of 570 at 10^6 vertices), nor with more ids for every workgroup to
-// read (with 8192 a solve of 2^17 vertices takes 345 us, with 4096 330).
+// read (with 8192 a solve of 2^17 vertices takes 15 us more than with 4096).
 constexpr u32 DENSE_MAX = 4096;
 constexpr u64 DENSE_EDGES = 16, DENSE_EDGES_MIN = 4096;  // edges per root, and in all, at least
 struct DenseRound {
