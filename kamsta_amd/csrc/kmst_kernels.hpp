@@ -410,6 +410,7 @@ enum : u32 {     // words of UnionArgs::ctl
   UC_DONE = 3,   // the output is written
   UC_FAR = 4,    // sampled records whose ids are FAR_SPAN or more apart
   UC_RUNS = 5,   // sampled records that begin a run of one source
+  UC_HUB = 6,    // one vertex has a fifth of the records, or a few have
   UC_WORDS = 8
 };
 struct Publication {

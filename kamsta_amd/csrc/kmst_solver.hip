@@ -1021,8 +1021,8 @@ void Solver::filter_rec(RecView P, RecView Q, bool stop, int depth) {
 // 1150 at 2^20, 0.91 / 1.57, 2.06 / 2.77 and 2.16 / 4.06 ms at 2^23.
 // Known to be slower than the round loop (plain): weights in order along a band 8
 // to 16 wide, 2^12 to 2^16 vertices, by 7 to 22 %; the same of 2^20 vertices in random
-// order, 1.32 against 0.82 ms; a wheel of 10^6 vertices whose hub's edges are the
-// heaviest, 2.3 against 1.65 ms (every wave's minimum goes to the hub).
+// order, 1.32 against 0.82 ms; a wheel of 10^6 vertices whose hub has the highest id
+// and the heaviest edges, 1.77 against 1.22 ms (hub at the lowest id: 1.06, 1.6).
 //
 // Light edges beyond what joins vertices stay in the lists round after round,
 // until their components meet: on a random graph 0.25 n of 1.1 n edges at

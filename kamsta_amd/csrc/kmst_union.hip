@@ -366,10 +366,10 @@ constexpr u32 SAMPLE_RUN = 16;
 __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
   __shared__ u32 h[256];
   __shared__ u32 s_scan[UW];
-  __shared__ u32 s_digit, s_below, s_max, s_far, s_runs;
+  __shared__ u32 s_digit, s_below, s_max, s_far, s_runs, s_hub;
   const u32 t = threadIdx.x, samples = a.samples;
   const u32 runs_of = (samples + SAMPLE_RUN - 1) / SAMPLE_RUN;
-  if (t == 0) s_max = s_far = s_runs = 0;
+  if (t == 0) s_max = s_far = s_runs = s_hub = 0;
   __syncthreads();
   u32 x[PIVOT_PER_THREAD], mx = 0, far = 0, runs = 0;
 #pragma unroll
@@ -385,6 +385,8 @@ __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
       const u32 s = a.src[i], d = a.dst[i];
       far += max(s, d) - min(s, d) >= FAR_SPAN ? 1u : 0u;
       runs += i == 0 || a.src[i - 1] != s ? 1u : 0u;
+      if (q % SAMPLE_RUN == 0 && q && a.src[(u64(q / SAMPLE_RUN - 1) * a.m) / runs_of] == s)
+        atomicAdd(&s_hub, 1u);  // the row reaches back to the run before
     }
   }
 #pragma unroll
@@ -402,6 +404,7 @@ __device__ __forceinline__ void pick_pivots(const UnionArgs& a) {
   if (t == 0) {
     put(a.ctl + UC_FAR, s_far);
     put(a.ctl + UC_RUNS, s_runs);
+    put(a.ctl + UC_HUB, 5 * s_hub > runs_of ? 1u : 0u);
   }
   const int top = s_max >> 24 ? 24 : s_max >> 16 ? 16 : s_max >> 8 ? 8 : 0;
   u32 pivot = NONE32;
@@ -1142,6 +1145,11 @@ __device__ __forceinline__ u32 hook(const UnionArgs& a, const WaveLists& l, int 
 
 // Rounds with at most this many live roots fold their offers in LDS; with
 // more, most offers of a workgroup are to distinct roots.
+// So do inputs where one vertex has a fifth of the records, whatever the roots: every
+// wave's minimum goes to it, 80 ns each.  Wheels of 10^6 vertices, hub edges the heaviest, at the
+// lowest and the highest id: 1950 and 2054 us, with the fold 1063 and 1768 (round loop
+// 1595 and 1224); of 2^17 457 and 427, 396 and 275 (690 and 674).  With an eighth of the
+// records, beside a band of 2^17 vertices, the fold makes no difference (505 us; 800).
 constexpr u64 TABLE_LIVE = u64{1} << TABLE_BITS;
 
 // Every vertex onto its root, 24 steps of all walks at a time: where all
@@ -1173,11 +1181,10 @@ __device__ __forceinline__ bool shorten_chains(const UnionArgs& a, Barrier& bar,
 // were.  After shorten_chains the same call finishes the round (what it offered
 // before, it offers again).
 __device__ __forceinline__ bool relabel(const UnionArgs& a, WaveLists& l, int out, u64 live,
-                                        OfferTable& t, u32 giant, u32 wave) {
+                                        bool table, OfferTable& t, u32 giant, u32 wave) {
   u64* best = minima(a, out);
-  const bool table = live <= TABLE_LIVE;
   // with few roots every wave meets the same ones: some waves' stores do
-  const u32 thin = !table ? 0u : live > 1024 ? 3u : live > 128 ? 31u : 255u;
+  const u32 thin = live > TABLE_LIVE ? 0u : live > 1024 ? 3u : live > 128 ? 31u : 255u;
   if (table) {
     table_clear(t);
     __syncthreads();
@@ -1442,7 +1449,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   __shared__ Scratch s_x;
   __shared__ Found s_all;
   __shared__ u64 s_waves[UW], s_base;  // prefix sums over the waves
-  __shared__ u32 s_giant;
+  __shared__ u32 s_giant, s_hub;
   UnionArgs a = arguments();
   if (!join_grid(a.joined)) return;
   Barrier bar{a.bar, 0, a.err};
@@ -1485,6 +1492,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
   if (!sync_grid(bar, mine.fwd, sum)) return;
   if (wave_id() == 0) {
     u64 hf = 0, hr = 0, bd = 0;
+    const u32 hub = get(a.ctl + UC_HUB);
     for (u32 b = lane; b < G; b += WAVE) {
       hf += get(a.found + b * 4);
       hr += get(a.found + b * 4 + 1);
@@ -1496,6 +1504,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       hr += __shfl_xor(hr, o, WAVE);
       bd |= __shfl_xor(bd, o, WAVE);
     }
+    if (lane == 0) s_hub = hub;
     if (lane == 0)
       s_all = Found{hf, hr, static_cast<u32>(sum), static_cast<u32>(bd >> 32), static_cast<u32>(bd)};
   }
@@ -1646,7 +1655,7 @@ __global__ __launch_bounds__(UT) void union_solve_kernel(UnionArgs) {
       if (ids)
         deep = relabel_dense(a, l, cur, ids, convert, identity ? a.parent : a.dense_parent, s_x.dense,
                              wave);
-      else deep = relabel(a, l, cur, live, s_x.table, giant, wave);
+      else deep = relabel(a, l, cur, live, live <= TABLE_LIVE || s_hub, s_x.table, giant, wave);
       resolved = ids && !enter;
       if (!sync_grid(bar, block_total(l.c | (deep ? u64{1} << DEEP_SHIFT : 0)), edges)) return;
       if (round >= UNION_ROUNDS_MAX) {
